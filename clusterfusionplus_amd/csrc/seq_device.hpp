@@ -153,6 +153,11 @@ template <typename T> __device__ __forceinline__ void store4(void* p, f32x4 v) {
         *reinterpret_cast<u32x2*>(p) = u32x2{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
     }
 }
+// two values to T, 8 or 4 bytes
+template <typename T> __device__ __forceinline__ void store2(void* p, float a, float b) {
+    if constexpr (sizeof(T) == 4) *reinterpret_cast<float2*>(p) = make_float2(a, b);
+    else *reinterpret_cast<uint32_t*>(p) = pack_bf16(a, b);
+}
 // N = 4: one access of 16 (T: 8) bytes; N = 1: one element
 template <int N> __device__ __forceinline__ void add_n(float (&s)[N], const float* __restrict__ p) {
     if constexpr (N == 4) {
@@ -166,6 +171,24 @@ template <int N> __device__ __forceinline__ void add_n(float (&s)[N], const floa
 template <typename T, int N> __device__ __forceinline__ void put_n(T* p, const float (&v)[N]) {
     if constexpr (N == 4) store4<T>(p, f32x4{v[0], v[1], v[2], v[3]});
     else *p = from_f32<T>(v[0]);
+}
+
+// Partial results of a product whose k was split: `parts` rows of n floats, `stride` apart; the first becomes their sum, in order.
+// The whole workgroup, which then reads the row.
+__device__ __forceinline__ void merge_parts(float* row, int n, int parts, size_t stride) {
+    if (parts <= 1) return;
+    const int n4 = ((uintptr_t)row & 15) == 0 && (stride & 3) == 0 ? n / 4 : 0;
+    for (int i = threadIdx.x; i < n4; i += kSeqThreads) {
+        f32x4 v = *reinterpret_cast<const f32x4*>(row + i * 4);
+        for (int k = 1; k < parts; ++k) v += *reinterpret_cast<const f32x4*>(row + k * stride + i * 4);
+        *reinterpret_cast<f32x4*>(row + i * 4) = v;
+    }
+    for (int i = n4 * 4 + threadIdx.x; i < n; i += kSeqThreads) {
+        float v = row[i];
+        for (int k = 1; k < parts; ++k) v += row[k * stride + i];
+        row[i] = v;
+    }
+    __syncthreads();
 }
 
 // Element d of head h of a run of heads (D elements each) after the norm over the whole projection and the rotation: the

@@ -22,6 +22,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <iterator>
 #include <map>
 #include <new>
 #include <tuple>
@@ -31,6 +32,7 @@
 
 #include "cfpp_seq.h"
 #include "seq_device.hpp"
+#include "seq_gemm.hpp"
 #include "seq_latent.hpp"
 
 using namespace cfpp;
@@ -76,7 +78,9 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_embed(const int* __restrict
 struct SeqPostNorm {
     const float* x;
     float* x_out;            // may be x
-    const float* y;          // nullable
+    const float* y;          // nullable: the sum of `parts` rows, part_stride floats apart
+    int parts;
+    size_t part_stride;
     const float* ys;         // nullable: [T][top][width], outputs of the chosen experts
     int top;
     float slot_weight;
@@ -108,7 +112,8 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_postnorm(SeqPostNorm a) {
 #pragma unroll
             for (int j = 0; j < N; ++j) s[j] *= a.slot_weight;
         }
-        if (a.y != nullptr) add_n<N>(s, a.y + (size_t)t * a.width + i);
+        if (a.y != nullptr)
+            for (int k = 0; k < a.parts; ++k) add_n<N>(s, a.y + k * a.part_stride + (size_t)t * a.width + i);
         float v[N];
 #pragma unroll
         for (int j = 0; j < N; ++j) v[j] = 0.0f;
@@ -145,8 +150,9 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_postnorm(SeqPostNorm a) {
 // One workgroup per token: raw q | k | v rows (fp32, biases included) -> norm over all of q and all of k, rotation, value
 // mixing -> q [T][H][Dp], portion k [G][cap][Dp] and v [G][cap][Vp].
 struct SeqQkv {
-    const float* qkv;
-    int ld;
+    float* qkv;              // partial results of `parts` splits, part_stride floats apart; the first becomes their sum
+    int ld, parts;
+    size_t part_stride;
     const float *qn, *kn;
     const float2* cs;        // [positions][rot / 2]
     float eps, lambda;
@@ -159,6 +165,7 @@ template <typename T>
 __global__ __launch_bounds__(kSeqThreads) void k_seq_qkv_finish(SeqQkv a) {
     __shared__ float2 red[kSeqWaves];
     const int t = blockIdx.x, nq = a.H * a.D, nk = a.G * a.D, nv = a.G * a.V;
+    merge_parts(a.qkv + (size_t)t * a.ld, nq + nk + nv, a.parts, a.part_stride);
     const float* q = a.qkv + (size_t)t * a.ld;
     const float *k = q + nq, *v = k + nk;
     const float2 sums = block_sum2(share_sq(q, nq, threadIdx.x), share_sq(k, nk, threadIdx.x), red);
@@ -227,202 +234,6 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_append(SeqAppend a) {
             *reinterpret_cast<u32x4*>(a.kc + ((size_t)g * a.rows + r) * a.krow + u * 16) = ld16(a.k + ((size_t)g * a.cap + t) * a.krow + u * 16);
         else
             *reinterpret_cast<u32x4*>(a.vc + ((size_t)g * a.rows + r) * a.vrow + (u - ku) * 16) = ld16(a.v + ((size_t)g * a.cap + t) * a.vrow + (u - ku) * 16);
-    }
-}
-
-// ------------------------------------------------------------------------------------------------
-// matrix products of a portion: out[token][row] = W[row] . a[token]
-// ------------------------------------------------------------------------------------------------
-// kEpiHeads: rows of keys of all heads, then rows of values of all heads, each head's rows [position] in a buffer of its own.
-// kEpiStreams (one token): the output row goes into the residual streams.
-enum : int { kEpiF32 = 0, kEpiRelu2 = 1, kEpiGated = 2, kEpiHead = 3, kEpiHeads = 4, kEpiStreams = 5 };
-struct SeqGemm {
-    const char* w;           // [n rows][kbytes]
-    const char* a;           // [tokens][lda bytes]
-    int n, m, kbytes, lda;
-    const float* bias;       // nullable (kEpiF32, kEpiGated)
-    float* yf;               // kEpiF32 / kEpiHead: [tokens][ldy]
-    int ldy;
-    char* yt;                // kEpiRelu2 / kEpiGated: T, [tokens][ldyt bytes]; kEpiHeads: keys
-    int ldyt;
-    float mul, cap;          // kEpiHead
-    char* yv;                // kEpiHeads: values; key rows of kd elements, kp bytes apart, heads kh bytes apart; values alike
-    int nk, kd, kp, vd, vp;  // ... nk: rows of keys
-    size_t kh, vh;
-    // tiles of tokens sorted by expert (tile_off null: a plain product)
-    const int* tile_off;     // [experts + 1] prefix sums of tiles
-    const int* row_off;      // [experts + 1] prefix sums of sorted slots
-    const int* slots;        // sorted slots: token * top + j
-    int experts, slot_div;   // input row of slot s: s / slot_div
-    size_t w_stride;
-};
-
-// rows of 128 bytes: units of row r are stored at unit ^ swz(r), which spreads 16 consecutive rows over all banks
-__device__ __forceinline__ int swz128(int row) { return (row >> 1) & 7; }
-
-template <typename T, int BW, int BT, int EPI>
-__global__ __launch_bounds__(kSeqThreads, 2) void k_seq_gemm(SeqGemm p) {
-    constexpr int MI = BW / 32, NI = BT / 32;            // 16 x 16 tiles of a wave; waves are 2 (rows) x 2 (tokens)
-    constexpr int WI = BW / 32, AI = BT / 32;            // 1 KB copies per wave and k step
-    __shared__ __align__(1024) char lds[2][(BW + BT) * kRowBytes];
-    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-    const int wr = wave >> 1, wc = wave & 1;
-
-    const int tiles_w = (p.n + BW - 1) / BW;
-    int tw, tt, m = p.m, row0 = 0;
-    const char* w = p.w;
-    {
-        // every XCD works on a contiguous range of tiles; inside it tiles go through groups of up to 8 token tiles
-        const int total = gridDim.x, per = total / 8, rem = total % 8, xcd = blockIdx.x % 8, i = blockIdx.x / 8;
-        const int id = xcd * per + min(xcd, rem) + i;
-        if (p.tile_off != nullptr) {
-            tt = id / tiles_w;
-            tw = id - tt * tiles_w;
-            if (tt >= p.tile_off[p.experts]) return;
-            int lo = 0, hi = p.experts;                  // last expert whose first tile is <= tt
-            while (hi - lo > 1) {
-                const int mid = (lo + hi) >> 1;
-                if (p.tile_off[mid] <= tt) lo = mid; else hi = mid;
-            }
-            // (experts without tokens have no tiles: skip to the one that owns the tile)
-            while (p.tile_off[lo + 1] <= tt) ++lo;
-            w += (size_t)lo * p.w_stride;
-            row0 = p.row_off[lo] + (tt - p.tile_off[lo]) * BT;
-            m = p.row_off[lo + 1] - row0;
-            tt = 0;
-        } else {
-            const int tiles_t = (p.m + BT - 1) / BT, group = 8 * tiles_w, gi = id / group, first = gi * 8;
-            const int gs = min(8, tiles_t - first), r = id - gi * group;
-            tt = first + r % gs;
-            tw = r / gs;
-        }
-    }
-    const char* src_w[WI];
-    const char* src_a[AI];
-#pragma unroll
-    for (int i = 0; i < WI; ++i) {
-        const int r = wave * (BW / 4) + i * 8 + (lane >> 3);
-        src_w[i] = w + (size_t)min(tw * BW + r, p.n - 1) * p.kbytes + ((lane & 7) ^ swz128(r)) * 16;
-    }
-#pragma unroll
-    for (int i = 0; i < AI; ++i) {
-        const int r = wave * (BT / 4) + i * 8 + (lane >> 3);
-        int tok = min(tt * BT + r, m - 1);
-        if (p.tile_off != nullptr) tok = p.slots[row0 + tok] / p.slot_div;
-        src_a[i] = p.a + (size_t)tok * p.lda + ((lane & 7) ^ swz128(r)) * 16;
-    }
-    auto stage = [&](int buf, int k) {
-        char* base = lds[buf];
-#pragma unroll
-        for (int i = 0; i < WI; ++i) copy_to_lds16(src_w[i] + k, base + (wave * (BW / 4) + i * 8) * kRowBytes);
-#pragma unroll
-        for (int i = 0; i < AI; ++i) copy_to_lds16(src_a[i] + k, base + BW * kRowBytes + (wave * (BT / 4) + i * 8) * kRowBytes);
-    };
-    f32x4 acc[MI][NI];
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < NI; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    const int col = lane & 15, g = lane >> 4, nk = p.kbytes / kRowBytes;
-    stage(0, 0);
-    for (int k = 0; k < nk; ++k) {
-        __syncthreads();                                 // this step's tile has arrived; the other buffer is free
-        if (k + 1 < nk) stage((k + 1) & 1, (k + 1) * kRowBytes);
-        const char* lw = lds[k & 1];
-        const char* la = lw + BW * kRowBytes;
-#pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            u32x4 fw[MI], fa[NI];
-#pragma unroll
-            for (int i = 0; i < MI; ++i) {
-                const int r = wr * (BW / 2) + i * 16 + col;
-                fw[i] = *reinterpret_cast<const u32x4*>(lw + r * kRowBytes + ((s * 4 + g) ^ swz128(r)) * 16);
-            }
-#pragma unroll
-            for (int j = 0; j < NI; ++j) {
-                const int r = wc * (BT / 2) + j * 16 + col;
-                fa[j] = *reinterpret_cast<const u32x4*>(la + r * kRowBytes + ((s * 4 + g) ^ swz128(r)) * 16);
-            }
-#pragma unroll
-            for (int i = 0; i < MI; ++i)
-#pragma unroll
-                for (int j = 0; j < NI; ++j) acc[i][j] = mma16<T>(fw[i], fa[j], acc[i][j]);
-        }
-    }
-    // kEpiHeads: where row n goes at position 0, and the bytes from one position to the next; `whole`: rows n0 .. n0 + 3 lie together
-    auto head_row = [&](int n, int& rp) {
-        const bool k = n < p.nk;
-        const int d = k ? p.kd : p.vd, m = k ? n : n - p.nk, h = m / d;
-        rp = k ? p.kp : p.vp;
-        return (k ? p.yt + h * p.kh : p.yv + h * p.vh) + (m - h * d) * (int)sizeof(T);
-    };
-    char* dst[MI];
-    int pitch[MI];
-    bool whole[MI];
-    if constexpr (EPI == kEpiHeads) {
-#pragma unroll
-        for (int i = 0; i < MI; ++i) {
-            const int n0 = min(tw * BW + wr * (BW / 2) + i * 16 + g * 4, p.n - 1);
-            dst[i] = head_row(n0, pitch[i]);
-            whole[i] = ((p.kd | p.vd) & 3) == 0 && n0 + 3 < p.n;       // (n0, the keys' rows and the heads' rows are multiples of four)
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < NI; ++j) {
-        const int tl = tt * BT + wc * (BT / 2) + j * 16 + col;
-        if (tl >= m) continue;
-        const int row = p.tile_off != nullptr ? p.slots[row0 + tl] : tl;
-#pragma unroll
-        for (int i = 0; i < MI; ++i) {
-            const int n0 = tw * BW + wr * (BW / 2) + i * 16 + g * 4;
-            const f32x4 v = acc[i][j];
-            if constexpr (EPI == kEpiF32 || EPI == kEpiHead) {
-                float* y = p.yf + (size_t)row * p.ldy + n0;
-                f32x4 o = v;
-                if (EPI == kEpiF32 && p.bias != nullptr) {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        if (n0 + r < p.n) o[r] += p.bias[n0 + r];
-                }
-                if (EPI == kEpiHead) {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) o[r] = soft_cap(o[r] * p.mul, p.cap);
-                }
-                if (n0 + 3 < p.n && (p.ldy & 3) == 0) {
-                    *reinterpret_cast<f32x4*>(y) = o;
-                } else {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        if (n0 + r < p.n) y[r] = o[r];
-                }
-            } else if constexpr (EPI == kEpiRelu2) {
-                T* y = reinterpret_cast<T*>(p.yt + (size_t)row * p.ldyt) + n0;
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    if (n0 + r < p.n) y[r] = from_f32<T>(relu2(v[r]));
-            } else if constexpr (EPI == kEpiHeads) {
-                if (whole[i]) {
-                    store4<T>(dst[i] + (size_t)row * pitch[i], v);
-                } else {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        if (n0 + r < p.n) {
-                            int rp;
-                            char* b = head_row(n0 + r, rp);
-                            *reinterpret_cast<T*>(b + (size_t)row * rp) = from_f32<T>(v[r]);
-                        }
-                }
-            } else {
-                T* y = reinterpret_cast<T*>(p.yt + (size_t)row * p.ldyt) + n0 / 2;
-#pragma unroll
-                for (int r = 0; r < 4; r += 2)
-                    if (n0 + r < p.n) {
-                        const float bg = p.bias != nullptr ? p.bias[n0 + r] : 0.0f, bu = p.bias != nullptr ? p.bias[n0 + r + 1] : 0.0f;
-                        y[r / 2] = from_f32<T>(silu(v[r] + bg) * (v[r + 1] + bu));
-                    }
-            }
-        }
     }
 }
 
@@ -1267,6 +1078,7 @@ struct cfpp_seq {
     float *x, *qkv, *y, *ys, *v_first;
     char *xb, *q, *k, *v, *o, *h, *hs, *wb;
     int ld_qkv;
+    size_t y_room, qkv_room; // floats of y and qkv: products that are split leave their partial results there
     SeqRoute* routes;
     std::vector<SeqRoute> host_routes;
     int max_experts = 0;
@@ -1308,33 +1120,127 @@ void allow_lds(K kernel, size_t bytes) {
 }
 
 // ---- portions ----------------------------------------------------------------------------------
-// max_tiles: upper bound of the expert products' token tiles (their number is known on the device only)
-template <typename T, int EPI>
-void launch_gemm(const SeqGemm& g, int max_tiles, bool big, hipStream_t st) {
-    const int tile = big ? 128 : 64, tw = ceil_div(g.n, tile), tt = g.tile_off != nullptr ? max_tiles : ceil_div(g.m, tile);
-    if (big) hipLaunchKernelGGL((k_seq_gemm<T, 128, 128, EPI>), dim3(tw * tt), dim3(kSeqThreads), 0, st, g);
-    else hipLaunchKernelGGL((k_seq_gemm<T, 64, 64, EPI>), dim3(tw * tt), dim3(kSeqThreads), 0, st, g);
+// The tiles of the matrix products and what they cost, in us, as measured on an MI355X over 2 to 4000 tokens, 1500 to 50432
+// rows and k of 1408 to 14336 (bf16; fp32: 2 to 2000 tokens): a step of 128 bytes of k when a compute unit has one workgroup, the
+// share of a step when it has `resident` of them (the more of them, the more bytes in flight; past that they take turns), and
+// what a workgroup costs beside its steps.  The estimate below is within 10 % (root mean square) of the times measured, and what
+// it chooses is 2 % slower than the best choice on average, 20 % at worst.  (Two more tiles, 128 x 96 and 128 x 160, were within
+// 0.2 % of the others on average and are left out.)
+struct GemmShape { int rows, tokens, resident; float step, share, fixed; };
+constexpr GemmShape kShapes16[] = {{64, 16, 2, 0.190f, 0.177f, 1.5f}, {64, 32, 2, 0.179f, 0.201f, 1.8f}, {64, 64, 2, 0.256f, 0.239f, 2.2f},
+                                   {64, 96, 2, 0.297f, 0.280f, 2.8f}, {128, 128, 2, 0.705f, 0.549f, 5.0f}, {256, 128, 1, 0.862f, 0.862f, 6.9f},
+                                   {256, 256, 1, 1.104f, 1.104f, 12.9f}};
+constexpr GemmShape kShapes32[] = {{64, 16, 2, 0.270f, 0.212f, 1.7f}, {64, 32, 2, 0.357f, 0.312f, 2.0f}, {64, 64, 3, 0.586f, 0.515f, 2.7f},
+                                   {128, 128, 2, 1.619f, 1.959f, 5.8f}};
+struct GemmPlan { int shape, splits; };
+
+// `tiles` tiles of `steps` steps on `cus` compute units; a stream of weights of `bytes` bytes takes what 5.8 TB/s take.
+float gemm_cost(const GemmShape& c, double tiles, float steps, int cus, double bytes) {
+    const int load = (int)ceil(tiles / cus), full = load / c.resident, rest = load % c.resident;
+    float t = full * (steps * std::max(c.step, c.resident * c.share) + c.fixed);
+    if (rest > 0) t += steps * std::max(c.step, rest * c.share) + c.fixed;
+    return std::max(t, (float)(bytes / 5.8e6));
 }
 
-// large tiles where they still give every compute unit one
-template <typename T, int EPI>
-void gemm(const cfpp_seq* s, const SeqGemm& g, hipStream_t st) {
-    launch_gemm<T, EPI>(g, 0, ceil_div(g.n, 128) * ceil_div(g.m, 128) >= s->cus, st);
+// The cheapest tile, and with `room` floats for partial results the cheapest number of splits of k as well.  Reading a partial
+// result costs its bytes at 5 TB/s, and 0.3 us.  No split has fewer than three steps.
+template <typename T>
+GemmPlan plan_gemm(const cfpp_seq* s, const SeqGemm& g, size_t room) {
+    const GemmShape* shapes = sizeof(T) == 2 ? kShapes16 : kShapes32;
+    const int count = sizeof(T) == 2 ? (int)std::size(kShapes16) : (int)std::size(kShapes32);
+    static const int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16};
+    const int nk = g.kbytes / kRowBytes;
+    GemmPlan best{0, 1};
+    float least = INFINITY;
+    for (int i = 0; i < count; ++i)
+        for (int sp : kSplits) {
+            if (sp > 1 && (room == 0 || nk / sp < 3 || (size_t)sp * g.m * g.ldy > room)) break;
+            const double tiles = (double)ceil_div(g.n, shapes[i].rows) * ceil_div(g.m, shapes[i].tokens) * sp;
+            float t = gemm_cost(shapes[i], tiles, (float)nk / sp, s->cus, (double)g.n * g.kbytes);
+            if (sp > 1) t += 0.3f + 4e-6f * sp * g.m * g.n / 5.0f;
+            if (t < least) {
+                least = t;
+                best = {i, sp};
+            }
+        }
+    return best;
 }
 
+template <typename T, int BW, int BT, int WR, int WC, int NB, int EPI>
+void launch_gemm(const SeqGemm& g, int tiles_t, hipStream_t st) {
+    const size_t lds = (size_t)NB * (BW + BT) * kRowBytes;
+    allow_lds(k_seq_gemm<T, BW, BT, WR, WC, NB, EPI>, lds);
+    hipLaunchKernelGGL((k_seq_gemm<T, BW, BT, WR, WC, NB, EPI>), dim3(ceil_div(g.n, BW) * tiles_t * g.splits), dim3(kWave * WR * WC), lds, st, g);
+}
+// tiles_t: tiles of tokens (experts: an upper bound, their number is known on the device only)
+template <typename T, int EPI>
+void launch_shape(const SeqGemm& g, int shape, int tiles_t, hipStream_t st) {
+    // (the buffers hold what keeps a weight stream going, and let two workgroups share a compute unit)
+    if constexpr (sizeof(T) == 2) {
+        switch (shape) {
+            case 0: return launch_gemm<T, 64, 16, 4, 1, 6, EPI>(g, tiles_t, st);
+            case 1: return launch_gemm<T, 64, 32, 4, 1, 5, EPI>(g, tiles_t, st);
+            case 2: return launch_gemm<T, 64, 64, 2, 2, 4, EPI>(g, tiles_t, st);
+            case 3: return launch_gemm<T, 64, 96, 2, 2, 4, EPI>(g, tiles_t, st);
+            case 4: return launch_gemm<T, 128, 128, 2, 2, 2, EPI>(g, tiles_t, st);
+            case 5: return launch_gemm<T, 256, 128, 4, 2, 3, EPI>(g, tiles_t, st);
+        }
+        constexpr size_t lds = 2 * 512 * kRowBytes;
+        allow_lds(k_seq_gemm8<EPI>, lds);
+        hipLaunchKernelGGL(k_seq_gemm8<EPI>, dim3(ceil_div(g.n, 256) * tiles_t * g.splits), dim3(512), lds, st, g);
+    } else {
+        switch (shape) {
+            case 0: return launch_gemm<T, 64, 16, 4, 1, 6, EPI>(g, tiles_t, st);
+            case 1: return launch_gemm<T, 64, 32, 4, 1, 5, EPI>(g, tiles_t, st);
+            case 2: return launch_gemm<T, 64, 64, 2, 2, 3, EPI>(g, tiles_t, st);
+        }
+        launch_gemm<T, 128, 128, 2, 2, 2, EPI>(g, tiles_t, st);
+    }
+}
+
+// `room`: floats behind g.yf for partial results; the number of those that the product leaves there
+template <typename T, int EPI>
+int gemm(const cfpp_seq* s, SeqGemm g, hipStream_t st, size_t room = 0) {
+    const GemmPlan plan = plan_gemm<T>(s, g, EPI == kEpiF32 ? room : 0);
+    g.splits = plan.splits;
+    g.split_stride = (size_t)g.m * g.ldy;
+    launch_shape<T, EPI>(g, plan.shape, ceil_div(g.m, (sizeof(T) == 2 ? kShapes16 : kShapes32)[plan.shape].tokens), st);
+    return plan.splits;
+}
+
+// Tile of the expert products of a portion of n tokens (both use it).  An expert has avg +- sqrt(avg) of them; where that fits a
+// tile, it has one, and the product is a stream of weights.
+int expert_shape(const cfpp_seq* s, const LayerPlan& L, int n) {
+    const GemmShape* shapes = s->esize == 2 ? kShapes16 : kShapes32;
+    const int count = s->esize == 2 ? (int)std::size(kShapes16) : (int)std::size(kShapes32);
+    const double avg = (double)n * L.d.top / L.d.experts, live = L.d.experts * std::min(1.0, avg);
+    int best = 0;
+    float least = INFINITY;
+    for (int i = 0; i < count; ++i) {
+        const GemmShape& c = shapes[i];
+        const double per = avg + 1.5 * sqrt(avg) <= c.tokens ? 1.0 : std::max(1.0, avg / c.tokens + 0.5);
+        const float t = gemm_cost(c, live * per * ceil_div(2 * L.d.ff, c.rows), (float)s->xpitch / kRowBytes, s->cus, live * 2.0 * L.d.ff * s->xpitch);
+        if (t < least) {
+            least = t;
+            best = i;
+        }
+    }
+    return best;
+}
 // tokens per tile of the expert products
-int expert_tile(const LayerPlan& L, int n) { return (long long)n * L.d.top >= 96LL * L.d.experts ? 128 : 64; }
+int expert_tile(const cfpp_seq* s, const LayerPlan& L, int n) { return (s->esize == 2 ? kShapes16 : kShapes32)[expert_shape(s, L, n)].tokens; }
 
 template <typename T, int EPI>
 void expert_gemm(const cfpp_seq* s, const LayerPlan& L, SeqGemm g, int n, hipStream_t st) {
     const SeqRoute& r = s->host_routes[L.route];
-    const int bt = expert_tile(L, n), slots = n * L.d.top;
+    const int shape = expert_shape(s, L, n), slots = n * L.d.top;
     g.m = slots;
     g.tile_off = r.tile_off;
     g.row_off = r.row_off;
     g.slots = r.slots;
     g.experts = L.d.experts;
-    launch_gemm<T, EPI>(g, slots / bt + std::min(L.d.experts, slots), bt == 128, st);
+    g.splits = 1;
+    launch_shape<T, EPI>(g, shape, slots / expert_tile(s, L, n) + std::min(L.d.experts, slots), st);
 }
 
 template <typename T, int NK, int NT>
@@ -1393,12 +1299,12 @@ NextInput next_input(const cfpp_seq* s, size_t li, int q) {
     return {nullptr, nullptr};
 }
 
-// The mixer of a portion, from s->xb to s->y.
+// The mixer of a portion between its projection (`parts` partial results in s->qkv) and its output rows (s->o).
 template <typename T>
-void portion_grouped(cfpp_seq* s, const LayerPlan& L, int slot, int n, int pos, hipStream_t st) {
+void portion_grouped(cfpp_seq* s, const LayerPlan& L, int slot, int n, int pos, int parts, hipStream_t st) {
     const cfpp_seq_layer& d = L.d;
     const int cap = s->portion;
-    SeqQkv f{s->qkv, s->ld_qkv, d.q_norm, d.k_norm, L.cs, s->d.eps, d.v_lambda, d.heads, d.kv_heads, d.dim, L.Dp, d.vdim, L.Vp,
+    SeqQkv f{s->qkv, s->ld_qkv, parts, (size_t)n * s->ld_qkv, d.q_norm, d.k_norm, L.cs, s->d.eps, d.v_lambda, d.heads, d.kv_heads, d.dim, L.Dp, d.vdim, L.Vp,
              d.rot_dims, pos, cap, L.v_role, s->v_first, s->q, s->k, s->v};
     hipLaunchKernelGGL(k_seq_qkv_finish<T>, dim3(n), dim3(kSeqThreads), 0, st, f);
 
@@ -1439,10 +1345,10 @@ LatentRow latent_row_of(const cfpp_seq* s, const LayerPlan& L) {
 }
 
 template <typename T>
-void portion_latent(cfpp_seq* s, const LayerPlan& L, int slot, int n, int pos, hipStream_t st) {
+void portion_latent(cfpp_seq* s, const LayerPlan& L, int slot, int n, int pos, int parts, hipStream_t st) {
     const cfpp_seq_layer& d = L.d;
     char* kc = L.kc + (size_t)slot * s->d.capacity * L.crow;
-    SeqLatentFinish f{s->qkv, s->ld_qkv, L.own, latent_row_of<T>(s, L), L.cs, d.heads, d.dim, d.rot_dims, pos, L.plain, L.qrow, s->q, kc};
+    SeqLatentFinish f{s->qkv, s->ld_qkv, L.n_qkv, parts, (size_t)n * s->ld_qkv, L.own, latent_row_of<T>(s, L), L.cs, d.heads, d.dim, d.rot_dims, pos, L.plain, L.qrow, s->q, kc};
     hipLaunchKernelGGL(k_seq_latent_finish<T>, dim3(n), dim3(kSeqThreads), 0, st, f);
 
     const int ctx = pos + n, cap = s->d.capacity;
@@ -1519,12 +1425,12 @@ int run_portion(cfpp_seq* s, int slot, int n, int pos, int n_want, float* logits
             for (; j < s->layers.size(); ++j) {
                 const LayerPlan& M = s->layers[j];
                 if (M.route < 0) continue;
-                if (expert_tile(M, n) != expert_tile(L, n)) break;
+                if (expert_tile(s, M, n) != expert_tile(s, L, n)) break;
                 ++count;
             }
             const size_t lds = (size_t)s->max_experts * 8;
             allow_lds(k_seq_route, lds);
-            hipLaunchKernelGGL(k_seq_route, dim3((unsigned)count), dim3(1024), lds, st, s->routes + L.route, s->tokens, n, expert_tile(L, n));
+            hipLaunchKernelGGL(k_seq_route, dim3((unsigned)count), dim3(1024), lds, st, s->routes + L.route, s->tokens, n, expert_tile(s, L, n));
             i = j - 1;
         }
     }
@@ -1541,10 +1447,10 @@ int run_portion(cfpp_seq* s, int slot, int n, int pos, int n_want, float* logits
         g.bias = d.b_qkv;
         g.yf = s->qkv;
         g.ldy = s->ld_qkv;
-        gemm<T, kEpiF32>(s, g, st);
+        const int parts = gemm<T, kEpiF32>(s, g, st, s->qkv_room);
 
-        if (L.latent) portion_latent<T>(s, L, slot, n, pos, st);
-        else portion_grouped<T>(s, L, slot, n, pos, st);
+        if (L.latent) portion_latent<T>(s, L, slot, n, pos, parts, st);
+        else portion_grouped<T>(s, L, slot, n, pos, parts, st);
 
         g = SeqGemm{};
         g.w = (const char*)d.w_o;
@@ -1554,9 +1460,11 @@ int run_portion(cfpp_seq* s, int slot, int n, int pos, int n_want, float* logits
         g.kbytes = g.lda = (int)pitch_of(d.heads * d.vdim, s->esize);
         g.yf = s->y;
         g.ldy = width;
-        gemm<T, kEpiF32>(s, g, st);
-        // the residual sum of a sublayer: y (nullable) and the chosen experts' outputs (`top` 0: none)
-        auto close = [&](int q, const float* y, int top) {
+        const int o_parts = gemm<T, kEpiF32>(s, g, st, s->y_room);
+        // the residual sum of a sublayer: y (`parts` partial results, 0: none) and the chosen experts' outputs (`top` 0: none)
+        auto close = [&](int q, int parts, int top) {
+            const float* y = parts > 0 ? s->y : nullptr;
+            const size_t stride = (size_t)n * width;
             float* c = q == 1 || d.ff_kind == CFPP_SEQ_FF_NONE ? copy : nullptr;
             const float* ys = top > 0 ? s->ys : nullptr;
             const float share = top > 0 ? 1.0f / (float)top : 0.0f;
@@ -1566,6 +1474,8 @@ int run_portion(cfpp_seq* s, int slot, int n, int pos, int n_want, float* logits
                 SeqStreams a{};
                 a.x = s->x;
                 a.y = y;
+                a.parts = parts;
+                a.part_stride = stride;
                 a.ys = ys;
                 a.top = top;
                 a.slot_weight = share;
@@ -1580,6 +1490,8 @@ int run_portion(cfpp_seq* s, int slot, int n, int pos, int n_want, float* logits
                 SeqPostNorm pn{};
                 pn.x = pn.x_out = s->x;
                 pn.y = y;
+                pn.parts = parts;
+                pn.part_stride = stride;
                 pn.ys = ys;
                 pn.top = top;
                 pn.slot_weight = share;
@@ -1594,7 +1506,7 @@ int run_portion(cfpp_seq* s, int slot, int n, int pos, int n_want, float* logits
                 postnorm<T>(s, pn, n, st);
             }
         };
-        close(0, s->y, 0);
+        close(0, o_parts, 0);
         if (d.ff_kind == CFPP_SEQ_FF_NONE) continue;
 
         if (d.ff_kind != CFPP_SEQ_FF_TABLE_EXPERTS) {
@@ -1623,8 +1535,7 @@ int run_portion(cfpp_seq* s, int slot, int n, int pos, int n_want, float* logits
             g.bias = d.b_down;
             g.yf = s->y;
             g.ldy = width;
-            gemm<T, kEpiF32>(s, g, st);
-            close(1, s->y, 0);
+            close(1, gemm<T, kEpiF32>(s, g, st, s->y_room), 0);
         } else {
             const int hp = (int)pitch_of(d.ff, s->esize);
             g = SeqGemm{};
@@ -1647,6 +1558,7 @@ int run_portion(cfpp_seq* s, int slot, int n, int pos, int n_want, float* logits
             g.ldy = width;
             g.slot_div = 1;
             expert_gemm<T, kEpiF32>(s, L, g, n, st);
+            int parts = 0;
             if (d.shared_ff > 0) {
                 const int sp = (int)pitch_of(d.shared_ff, s->esize);
                 g = SeqGemm{};
@@ -1666,9 +1578,9 @@ int run_portion(cfpp_seq* s, int slot, int n, int pos, int n_want, float* logits
                 g.kbytes = g.lda = sp;
                 g.yf = s->y;
                 g.ldy = width;
-                gemm<T, kEpiF32>(s, g, st);
+                parts = gemm<T, kEpiF32>(s, g, st, s->y_room);
             }
-            close(1, d.shared_ff > 0 ? s->y : nullptr, d.top);
+            close(1, parts, d.top);
         }
     }
     if (n_want > 0) {
@@ -2048,6 +1960,9 @@ int cfpp_seq_create(const cfpp_seq_desc* desc, cfpp_seq** out) {
     s->portion = std::min(D.max_portion, D.capacity);
     (void)hipGetDevice(&s->device);
     if (hipDeviceGetAttribute(&s->cus, hipDeviceAttributeMultiprocessorCount, s->device) != hipSuccess || s->cus < 1) s->cus = 256;
+    for (int i = 0; i < D.n_layers; ++i)                 // inputs that are gathered slot by slot lie in less than 4 GiB
+        if (D.layers[i].ff_kind == CFPP_SEQ_FF_TABLE_EXPERTS)
+            s->portion = (int)std::min<size_t>(s->portion, 0xffffffffu / std::max((size_t)s->xpitch, D.layers[i].top * pitch_of(D.layers[i].ff, esize)));
     const size_t P = (size_t)s->portion, C = (size_t)D.capacity;
     size_t n_qkv = 0, o_bytes = 0, h_bytes = 0, hs_bytes = 0, q_bytes = 0, k_bytes = 0, v_bytes = 0, vf = 0, ys = 0, part = 0, items = 0, dec_h = 0;
     std::map<std::tuple<double, int, double, double, double, double>, float2*> tables;
@@ -2140,9 +2055,13 @@ int cfpp_seq_create(const cfpp_seq_desc* desc, cfpp_seq** out) {
     s->want = s->tokens != nullptr ? s->tokens + P : nullptr;
     const size_t rows_of_x = std::max(1, D.streams);
     s->x = s->alloc<float>(P * rows_of_x * D.width);
-    s->y = s->alloc<float>(P * D.width);
+    // eight partial results, or 64 MB of them: a portion of a few tokens is split the most
+    const auto room = [](size_t floats) { return std::max(floats, std::min(8 * floats, (size_t)16 << 20)); };
+    s->y_room = room(P * D.width);
+    s->qkv_room = room(P * s->ld_qkv);
+    s->y = s->alloc<float>(s->y_room);
     s->ys = s->alloc<float>(P * ys);
-    s->qkv = s->alloc<float>(P * s->ld_qkv);
+    s->qkv = s->alloc<float>(s->qkv_room);
     s->v_first = s->alloc<float>(P * vf);
     s->xb = s->alloc<char>(P * s->xpitch);
     s->wb = s->alloc<char>(P * s->xpitch);

@@ -47,8 +47,10 @@ __device__ __forceinline__ void latent_row(const LatentRow& a, const float* __re
 // ---- portions ----------------------------------------------------------------------------------
 // One workgroup per token: raw projection (fp32) -> queries [token][head][plain | rotated | zeros] and the cache row.
 struct SeqLatentFinish {
-    const float* z;
-    int ld, own;             // own: the layer makes cache rows
+    float* z;                // partial results of `parts` splits, part_stride floats apart; the first becomes their sum
+    int ld, n, parts;        // n: values of a row
+    size_t part_stride;
+    int own;                 // the layer makes cache rows
     LatentRow kv;
     const float2* cs;        // [positions][R / 2]
     int H, D, R, pos0, rot_at, qrow;      // rot_at: bytes in front of the rotated part of a query
@@ -58,6 +60,7 @@ template <typename T>
 __global__ __launch_bounds__(kSeqThreads) void k_seq_latent_finish(SeqLatentFinish a) {
     __shared__ float red[kSeqWaves];
     const int t = blockIdx.x, n = a.D + a.R;
+    merge_parts(a.z + (size_t)t * a.ld, a.n, a.parts, a.part_stride);
     const float* z = a.z + (size_t)t * a.ld;
     const float2* cs = a.cs + (size_t)(a.pos0 + t) * (a.R / 2);
     char* q = a.q + (size_t)t * a.H * a.qrow;
@@ -445,7 +448,9 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_latent_out(SeqLatentOut a) 
 // are), and the next sublayer's input norm(sum_t in[t] x_t).
 struct SeqStreams {
     float* x;                // [tokens][streams][width]
-    const float* y;          // the sublayer's output, nullable
+    const float* y;          // the sublayer's output, nullable: the sum of `parts` rows, part_stride floats apart
+    int parts;
+    size_t part_stride;
     const float* ys;         // nullable: [tokens][top][width], outputs of the chosen experts
     int top;
     float slot_weight;
@@ -512,7 +517,8 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_streams(SeqStreams a) {
 #pragma unroll
                 for (int j = 0; j < N; ++j) y[j] *= a.slot_weight;
             }
-            if (a.y != nullptr) add_n<N>(y, a.y + (size_t)t * a.width + i);
+            if (a.y != nullptr)
+                for (int k = 0; k < a.parts; ++k) add_n<N>(y, a.y + k * a.part_stride + (size_t)t * a.width + i);
 #pragma unroll
             for (int s = 0; s < S; ++s)
 #pragma unroll
