@@ -90,6 +90,26 @@ __device__ __forceinline__ void copy_to_lds16(const void* g, void* lds) {
 // waits until at most N of the wave's vector memory operations are still on their way
 template <int N> __device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
+// an address that is the same in all lanes, in scalar registers
+__device__ __forceinline__ const char* uniform(const char* p) {
+    const uint64_t v = (uint64_t)(uintptr_t)p;
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((int)(uint32_t)v), hi = __builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+    return (const char*)(uintptr_t)((uint64_t)hi << 32 | lo);
+}
+
+// 64 units of 16 bytes from `base` (wave-uniform) + the lanes' offsets, or from the lanes' addresses, to LDS from byte `lds`
+// (wave-uniform) on.  Written out: the compiler does not know of the copy, so that it puts no waits of its own for it; who reads the
+// tile waits with wait_vm or pipe_barrier.
+__device__ __forceinline__ void copy_to_lds16_at(uint32_t off, const void* base, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory");
+}
+__device__ __forceinline__ void copy_to_lds16_from(const void* p, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(p), "s"(lds) : "memory");
+}
+__device__ __forceinline__ uint32_t lds_address(const void* p) { return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)p; }
+// waits for all but the wave's N newest copies and for its reads of LDS, then for the other waves
+template <int N> __device__ __forceinline__ void pipe_barrier() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory"); }
+
 // A barrier of the workgroup behind its LDS accesses only.  Written out: __syncthreads(), and a fence over LDS as well, would
 // also wait for the loads in flight, those that go straight to LDS among them.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
@@ -312,6 +332,21 @@ __device__ __forceinline__ void attn_softmax(AttnState<NT>& st, f32x4 (&s)[NKT],
 #pragma unroll
     for (int i = 0; i < NT / 16; ++i)
         if (i < vtiles) st.acc[i] *= c;
+}
+
+// Eight weights of a lane (keys 4 g .. of one group of 16 keys, then of the next) as high and low bf16 parts, in the order of a
+// product's k.
+__device__ __forceinline__ void split_weights(f32x4 a, f32x4 b, u32x4& hi, u32x4& lo) {
+    hi = u32x4{pack_bf16(a[0], a[1]), pack_bf16(a[2], a[3]), pack_bf16(b[0], b[1]), pack_bf16(b[2], b[3])};
+    const float v[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) lo[j] = pack_bf16(v[2 * j] - __uint_as_float(hi[j] << 16), v[2 * j + 1] - __uint_as_float(hi[j] & 0xffff0000u));
+}
+// A transposing read of LDS: lane i of a group of 16 gives the address of four bf16 of a row (rows of the group's lanes i / 4, columns
+// 4 (i % 4) ..) and receives the group's four rows of column i.
+__device__ __forceinline__ u32x2 read_transposed(const void* p) {
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(uintptr_t)p));
 }
 
 // acc += V^T p for the keys of one tile and CT column tiles, which share the reads of V^T

@@ -43,15 +43,6 @@ struct SeqGemm {
 // rows of 128 bytes: units of row r are stored at unit ^ swz(r), which spreads 16 consecutive rows over all banks
 __device__ __forceinline__ int swz128(int row) { return (row >> 1) & 7; }
 
-// 64 units of 16 bytes from `base` (wave-uniform) + the lanes' offsets to LDS from byte `lds` (wave-uniform) on.  Written out: the
-// compiler does not know of the copy, so that it puts no waits of its own for it; who reads the tile waits with wait_vm or pipe_barrier.
-__device__ __forceinline__ void copy_to_lds16_at(uint32_t off, const void* base, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory");
-}
-__device__ __forceinline__ uint32_t lds_address(const void* p) { return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)p; }
-// waits for all but the wave's N newest copies and for its reads of LDS, then for the other waves
-template <int N> __device__ __forceinline__ void pipe_barrier() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory"); }
-
 // Which tile a workgroup works on.
 struct GemmTile {
     const char* w;           // the matrix (of the expert)

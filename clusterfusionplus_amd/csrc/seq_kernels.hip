@@ -31,6 +31,7 @@
 #include <vector>
 
 #include "cfpp_seq.h"
+#include "seq_attn.hpp"
 #include "seq_device.hpp"
 #include "seq_gemm.hpp"
 #include "seq_latent.hpp"
@@ -268,163 +269,6 @@ __global__ __launch_bounds__(1024) void k_seq_route(const SeqRoute* layers, cons
     for (int s = threadIdx.x; s < n; s += blockDim.x) {
         const int t = s / a.top;
         a.slots[atomicAdd(&next[a.table[(size_t)tokens[t] * a.top + (s - t * a.top)]], 1)] = s;
-    }
-}
-
-// ------------------------------------------------------------------------------------------------
-// attention of a portion
-// ------------------------------------------------------------------------------------------------
-// The query columns of one key / value head are (token, head of the group), head fastest; a workgroup takes 64 CT of them
-// and walks the keys its tokens can see, first the cached ones (positions before k_split), then those in the buffer.  Behind a
-// key's own row comes the part that all heads share, if there is one.  The softmax is online, the sink is added to the
-// denominator at the end.
-struct SeqAttn {
-    const char *q, *k, *v, *kc, *vc;
-    const char* kr;          // rows of the shared part, of position 0 on
-    char* out;
-    const float* sink;       // nullable
-    const float* gate;       // nullable: [T][ldg], the outputs are multiplied by its sigmoid
-    int T, H, R, dsteps, qrow, krow, vrow, V, vtiles, pos0, chunk, cap, rows, ldo, k_split, runits, rrow, ldg;
-    float scale_log2;
-};
-template <int UN> __device__ __forceinline__ int swz_key(int row) { return UN % 16 ? (row >> 1) & 7 : row & 15; }
-
-// (the next tile's keys go straight to the other LDS buffer and its values into registers while this one is worked on)
-// (NK: elements of a key row in LDS, NT: value columns.  The products run over all of them, without branches between the reads
-// of LDS: past the end of the query there are zeros, and of the columns past the end of a value nothing is stored)
-template <typename T, int NK, int NT, int CT>
-__global__ __launch_bounds__(kSeqThreads, (NT <= 128 ? 2 : 1)) void k_seq_attn(SeqAttn a) {
-    constexpr int KT = sizeof(T) == 2 ? 64 : 32;
-    constexpr int NB = NK * (int)sizeof(T), UN = NB / 16;                    // bytes and units of a key row in LDS
-    constexpr int VS = VtSteps<T, KT, NT, kSeqThreads>::n;
-    __shared__ __align__(1024) char ks[2][KT * NB];
-    __shared__ __align__(16) char vt[NT * VtTile<T, KT>::pitch];
-    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 15, g = lane >> 4;
-    // the longest walks first; every second group of eight runs backwards, so that each XCD (workgroups go round them) gets as
-    // many long ones as the others
-    const int gq = blockIdx.y, ncols = a.T * a.R, gx = gridDim.x;
-    int bx = blockIdx.x;
-    if (((bx >> 3) & 1) && (bx | 7) < gx) bx ^= 7;
-    const int c0 = (gx - 1 - bx) * 64 * CT;
-
-    int pq[CT], first[CT], tok[CT], head[CT];
-    u32x4 qf[CT][NB / 64];
-    AttnState<NT> st[CT];
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct) {
-        const int cc = min(c0 + (wave * CT + ct) * 16 + col, ncols - 1);
-        tok[ct] = cc / a.R;
-        head[ct] = gq * a.R + (cc - tok[ct] * a.R);
-        pq[ct] = a.pos0 + tok[ct];
-        first[ct] = chunk_start(pq[ct], a.chunk);
-        const char* qr = a.q + ((size_t)tok[ct] * a.H + head[ct]) * a.qrow + g * 16;
-#pragma unroll
-        for (int s = 0; s < NB / 64; ++s) {
-            qf[ct][s] = ld16(qr + min(s, a.dsteps - 1) * 64);
-            if (s >= a.dsteps) qf[ct][s] = u32x4{0, 0, 0, 0};
-        }
-        attn_reset(st[ct]);
-    }
-    // keys the workgroup needs, and those every column of this wave sees / any column sees
-    const int t_first = c0 / a.R, t_last = min(a.T - 1, (c0 + 64 * CT - 1) / a.R);
-    const int k_first = chunk_start(a.pos0 + t_first, a.chunk), k_end = a.pos0 + t_last + 1;
-    const int w_first = min(c0 + wave * CT * 16, ncols - 1) / a.R, w_last = min(c0 + (wave + 1) * CT * 16 - 1, ncols - 1) / a.R;
-    const int all_lo = chunk_start(a.pos0 + w_last, a.chunk), all_hi = a.pos0 + w_first;
-    const int any_lo = chunk_start(a.pos0 + w_first, a.chunk), any_hi = a.pos0 + w_last;
-    const int dunits = a.krow / 16, vunits = a.vrow / 16;
-
-    // tiles: [k_first, k_split) in the cache, then [k_split, k_end) in the buffer
-    struct Tile { int k0, hi; const char *k, *v; };      // first key, end of its part, row of position 0
-    auto tile_at = [&](int k0) {
-        const bool cached = k0 < a.k_split;
-        const size_t row0 = (size_t)gq * (cached ? a.rows : a.cap) - (cached ? chunk_start(a.pos0, a.chunk) : a.k_split);
-        return Tile{k0, cached ? min(k_end, a.k_split) : k_end, (cached ? a.kc : a.k) + (ptrdiff_t)row0 * a.krow, (cached ? a.vc : a.v) + (ptrdiff_t)row0 * a.vrow};
-    };
-    u32x4 vr[VS][4];
-    auto fetch = [&](const Tile& t, int buf) {
-        for (int i = wave; i < KT * NB / 1024; i += kSeqWaves) {
-            const int r = (i * 64 + lane) / UN, u = ((i * 64 + lane) % UN) ^ swz_key<UN>(r), key = min(t.k0 + r, t.hi - 1);
-            const char* src = t.k + (ptrdiff_t)key * a.krow + (u < dunits ? u : 0) * 16;
-            if (u >= dunits && u < dunits + a.runits) src = a.kr + (ptrdiff_t)key * a.rrow + (u - dunits) * 16;
-            copy_to_lds16(src, ks[buf] + i * 1024);
-        }
-        vt_request<T, KT, kSeqThreads, 0, VS>(vr, vunits, tid, [&](int key) { return t.v + (ptrdiff_t)min(t.k0 + key, t.hi - 1) * a.vrow; });
-    };
-    Tile t = tile_at(k_first);
-    fetch(t, 0);
-    for (int buf = 0;; buf ^= 1) {
-        __syncthreads();                                 // the tile's keys are there; nobody reads the last tile's values any more
-        vt_store<T, KT, kSeqThreads, 0, VS>(vr, vt, vunits, tid);
-        const int next = min(t.k0 + KT, t.hi);
-        Tile tn = t;
-        if (next < k_end) {
-            tn = tile_at(next);
-            fetch(tn, buf ^ 1);
-        }
-        lds_barrier();                                   // (waits for the stores to LDS, not for the next tile)
-        if (t.k0 <= any_hi && next > any_lo) {
-            // the fragments of the next 16 keys are read while these are multiplied
-            f32x4 s[CT][KT / 16];
-            u32x4 kf[2][NB / 64];
-            auto read = [&](int kt) __attribute__((always_inline)) {
-                const int r = kt * 16 + col;
-#pragma unroll
-                for (int d = 0; d < NB / 64; ++d)
-                    kf[kt & 1][d] = *reinterpret_cast<const u32x4*>(ks[buf] + r * NB + ((d * 4 + g) ^ swz_key<UN>(r)) * 16);
-            };
-            read(0);
-#pragma unroll
-            for (int kt = 0; kt < KT / 16; ++kt) {
-                if (kt + 1 < KT / 16) read(kt + 1);
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int ct = 0; ct < CT; ++ct) {
-                    s[ct][kt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                    for (int d = 0; d < NB / 64; ++d) s[ct][kt] = mma16<T>(kf[kt & 1][d], qf[ct][d], s[ct][kt]);
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            const bool full = t.k0 + KT <= t.hi && t.k0 >= all_lo && t.k0 + KT - 1 <= all_hi;
-#pragma unroll
-            for (int ct = 0; ct < CT; ++ct) {
-#pragma unroll
-                for (int kt = 0; kt < KT / 16; ++kt)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) s[ct][kt][r] *= a.scale_log2;
-                if (!full) {
-#pragma unroll
-                    for (int kt = 0; kt < KT / 16; ++kt)
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const int key = t.k0 + kt * 16 + g * 4 + r;
-                            if (key >= t.hi || key > pq[ct] || key < first[ct]) s[ct][kt][r] = kMasked;
-                        }
-                }
-                attn_softmax<NT, KT / 16>(st[ct], s[ct], NT / 16);
-            }
-            __builtin_amdgcn_sched_barrier(0);           // (values read ahead of the softmax would take its registers)
-            attn_pv<T, NT, KT, CT>(st, s, vt, NT / 16, lane);
-        }
-        if (next >= k_end) break;
-        t = tn;
-    }
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct) {
-        if (c0 + (wave * CT + ct) * 16 + col >= ncols) continue;
-        const float snk = a.sink != nullptr ? a.sink[head[ct]] * kLog2e : kNegBig, m = fmaxf(st[ct].m, snk), c = fast_exp2(st[ct].m - m);
-        const float f = c / (st[ct].l * c + fast_exp2(snk - m));       // (no sink: the last term is zero)
-        T* o = reinterpret_cast<T*>(a.out + (size_t)tok[ct] * a.ldo) + head[ct] * a.V;
-        const float* gate = a.gate + (size_t)tok[ct] * a.ldg + head[ct] * a.V;
-#pragma unroll
-        for (int i = 0; i < NT / 16; ++i)
-            if (i < a.vtiles) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int v = i * 16 + g * 4 + r;
-                    if (v < a.V) o[v] = from_f32<T>(a.gate != nullptr ? st[ct].acc[i][r] * f * sigmoid(gate[v]) : st[ct].acc[i][r] * f);
-                }
-            }
     }
 }
 
@@ -1243,25 +1087,45 @@ void expert_gemm(const cfpp_seq* s, const LayerPlan& L, SeqGemm g, int n, hipStr
     launch_shape<T, EPI>(g, shape, slots / expert_tile(s, L, n) + std::min(L.d.experts, slots), st);
 }
 
+// Columns of a workgroup and splits of the keys.  bf16: two column tiles per wave share the reads of keys and values; one, where that
+// leaves fewer columns empty or where two workgroups per compute unit are not reached.  Splits fill the chip: two workgroups per
+// compute unit, each with two tiles at least.
 template <typename T, int NK, int NT>
-void launch_attn(const SeqAttn& a, int G, int cus, hipStream_t st) {
-    const int cols = a.T * a.R;
-    if constexpr (sizeof(T) == 2) {                      // (fp32: two column tiles do not fit the registers)
-        if (ceil_div(cols, 128) * G >= 2 * cus) {
-            hipLaunchKernelGGL((k_seq_attn<T, NK, NT, 2>), dim3(ceil_div(cols, 128), G), dim3(kSeqThreads), 0, st, a);
-            return;
+void launch_attn(SeqAttn a, int G, int cus, size_t room, float* part, hipStream_t st) {
+    using L = AttnTile<T, NK, NT>;
+    const int cols = a.T * a.R, tiles = ceil_div(std::min(a.pos0 + a.T, a.chunk > 0 ? a.chunk : a.pos0 + a.T), L::keys);
+    const bool two = sizeof(T) == 2 && ceil_div(cols, 128) * G >= 2 * cus;       // (fp32: two column tiles do not fit the registers)
+    const int wgs = ceil_div(cols, two ? 128 : 64) * G, per_cu = NT <= 128 ? 2 : 1;
+    const size_t floats = (size_t)a.T * a.H * (a.vtiles * 16 + 2);
+    a.splits = std::max(1, (int)std::min<size_t>({(size_t)16, (size_t)(per_cu * cus / wgs), (size_t)(tiles / 2), room / floats}));
+    a.part = part;
+    a.ml = part + (size_t)a.splits * a.T * a.H * a.vtiles * 16;
+    const size_t lds = 2 * L::size;
+    auto go = [&](auto n, auto sh) {
+        constexpr int CT = decltype(n)::value;
+        constexpr bool SH = decltype(sh)::value;
+        allow_lds(k_seq_attn<T, NK, NT, CT, SH>, lds);
+        hipLaunchKernelGGL((k_seq_attn<T, NK, NT, CT, SH>), dim3(ceil_div(cols, 64 * CT), G, a.splits), dim3(kSeqThreads), lds, st, a);
+    };
+    auto pick = [&](auto sh) {
+        if constexpr (sizeof(T) == 2) {
+            if (two) return go(std::integral_constant<int, 2>{}, sh);
         }
-    }
-    hipLaunchKernelGGL((k_seq_attn<T, NK, NT, 1>), dim3(ceil_div(cols, 64), G), dim3(kSeqThreads), 0, st, a);
+        go(std::integral_constant<int, 1>{}, sh);
+    };
+    if (a.runits > 0) pick(std::true_type{});
+    else pick(std::false_type{});
+    if (a.splits > 1)
+        hipLaunchKernelGGL(k_seq_attn_merge<T>, dim3(a.T, ceil_div(a.H * a.vtiles * 4, kSeqThreads)), dim3(kSeqThreads), 0, st, a);
 }
 
 template <typename T>
 void attn(const cfpp_seq* s, const SeqAttn& a, int G, hipStream_t st) {
     const int nk = a.qrow / (int)sizeof(T), nv = a.vtiles * 16;
-    if (nk <= 64 && nv <= 64) launch_attn<T, 64, 64>(a, G, s->cus, st);
-    else if (nk <= 128 && nv <= 128) launch_attn<T, 128, 128>(a, G, s->cus, st);
-    else if (nk <= 192 && nv <= 128) launch_attn<T, 192, 128>(a, G, s->cus, st);
-    else launch_attn<T, 256, 256>(a, G, s->cus, st);
+    if (nk <= 64 && nv <= 64) launch_attn<T, 64, 64>(a, G, s->cus, s->y_room, s->y, st);
+    else if (nk <= 128 && nv <= 128) launch_attn<T, 128, 128>(a, G, s->cus, s->y_room, s->y, st);
+    else if (nk <= 192 && nv <= 128) launch_attn<T, 192, 128>(a, G, s->cus, s->y_room, s->y, st);
+    else launch_attn<T, 256, 256>(a, G, s->cus, s->y_room, s->y, st);
 }
 
 template <typename T>

@@ -1,0 +1,41 @@
+"""Attention of a portion: keys shared among workgroups, tiles of keys that begin and end anywhere, scores of either sign."""
+import pytest
+import torch
+
+from tests import kagapel_models as K
+from tests import nibotar_models as N
+from tests.test_gpu_nibotar import DTYPES, IDS, LIMIT
+
+pytestmark = pytest.mark.gpu
+
+
+def grouped(scale=None, chunk=None, dims=(40, 56)):
+    return N, N.model(64, 51, [(N.attn(6, 2, *dims, scale=scale, chunk=chunk, rot=8), None)])
+
+
+def latent(scale=None, dims=(40, 16, 56, 48)):
+    return K, K.model(64, 51, [K.gated(3, *dims, scale=scale), K.sunk(3, *dims, scale=scale, kv_from=0)], positions=1400)
+
+
+MODELS = {"grouped": grouped(), "grouped_chunks": grouped(chunk=400), "grouped_small": grouped(dims=(16, 32)), "grouped_large": grouped(dims=(200, 250)),
+          "latent": latent(), "latent_wide": latent(dims=(128, 64, 128, 96)), "latent_large": latent(dims=(160, 64, 200, 96)),
+          "negative": grouped(scale=-0.2), "zero": grouped(scale=0.0), "latent_negative": latent(scale=-0.2)}
+
+
+# (context, tokens): one and two tiles (64 keys in bf16, 32 in fp32) per workgroup and fewer than that, first and last keys of a
+# tile, several column tiles, the edge of a chunk inside the portion
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("name", list(MODELS))
+def test_portions_far_into_a_sequence(name, dtype):
+    from clusterfusionplus_amd import kagapel, nibotar
+    M, cfg = MODELS[name]
+    w, toks, res = M.weights(cfg, 5), M.prompt(cfg, 1300, 6), []
+    want = M.oracle(cfg, w, toks, res)
+    m = (nibotar if M is N else kagapel).from_tensors(cfg, w, dtype, capacity=1300)
+    pos = 0
+    for n in (64, 63, 2, 127, 129, 3, 37, 70, 300, 5, 200, 2, 290, 8):
+        logits, layers = m.forward(0, toks[pos:pos + n], pos, range(n), residuals=True)
+        assert N.error(layers[-1], res[-1][pos:pos + n]) < LIMIT[dtype], (pos, n)
+        assert N.error(logits, want[pos:pos + n]) < LIMIT[dtype], (pos, n)
+        pos += n
+    assert pos == 1300
