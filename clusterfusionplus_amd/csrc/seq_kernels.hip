@@ -1,8 +1,9 @@
 // Kernels and host side of the sequence models (include/cfpp_seq.h).
 //
 // Prefill (a portion of T tokens): per layer
-//   k_seq_gemm (q, k, v rows + bias) -> k_seq_qkv_finish (norms over the projections, rotation, value mixing) -> k_seq_attn ->
-//   k_seq_append (what later portions can see goes into the cache) -> k_seq_gemm (output rows) -> k_seq_postnorm ->
+//   k_seq_gemm (q, k, v rows + bias) -> k_seq_qkv_finish (norms over the projections, rotation, value mixing; keys and values into
+//   the cache) -> k_seq_attn -> k_seq_append (portions that cross chunks: what later portions can see goes into the cache only now) ->
+//   k_seq_gemm (output rows) -> k_seq_postnorm ->
 //   k_seq_gemm (up rows with the activation) -> k_seq_gemm (down rows) -> k_seq_postnorm;
 //   table experts: the same two products over tiles of tokens sorted by expert (k_seq_route), plus the shared expert's.
 // Decode (one token): five launches per layer, each with its neighbours' work fused in:
@@ -149,7 +150,7 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_postnorm(SeqPostNorm a) {
 }
 
 // One workgroup per token: raw q | k | v rows (fp32, biases included) -> norm over all of q and all of k, rotation, value
-// mixing -> q [T][H][Dp], portion k [G][cap][Dp] and v [G][cap][Vp].
+// mixing -> q [T][H][Dp], k [G][..][Dp] and v [G][..][Vp]: rows of the portion's buffers, or of the cache itself.
 struct SeqQkv {
     float* qkv;              // partial results of `parts` splits, part_stride floats apart; the first becomes their sum
     int ld, parts;
@@ -157,7 +158,8 @@ struct SeqQkv {
     const float *qn, *kn;
     const float2* cs;        // [positions][rot / 2]
     float eps, lambda;
-    int H, G, D, Dp, V, Vp, rot, pos0, cap;
+    int H, G, D, Dp, V, Vp, rot, pos0;
+    size_t khead, vhead;     // bytes from one head's rows to the next one's
     int v_role;              // 0: plain, 1: this layer's values are the ones later layers mix in, 2: mix
     float* v_first;          // [T][G * V]
     char *q, *k, *v;
@@ -175,7 +177,7 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_qkv_finish(SeqQkv a) {
     char* qo = a.q + (size_t)t * a.H * a.Dp * sizeof(T);
     char* ko = a.k + (size_t)t * a.Dp * sizeof(T);
     char* vo = a.v + (size_t)t * a.Vp * sizeof(T);
-    const size_t khead = (size_t)a.cap * a.Dp * sizeof(T), vhead = (size_t)a.cap * a.Vp * sizeof(T);
+    const size_t khead = a.khead, vhead = a.vhead;
     // four elements at a time: head `h`, elements d .. d + 3 of its padded row (zeros past the end: the padding is written
     // too, since layers of other sizes share these buffers)
     auto rotated = [&](const float* row, const float* w, float inv, int d) {
@@ -222,6 +224,85 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_qkv_finish(SeqQkv a) {
         }
         store4<T>(vo + g * vhead + d * sizeof(T), x);
     }
+}
+
+// The same where heads are whole groups of four elements and the row fits U groups per thread: everything is read once, in one round
+// trip (partial results of a split product included), and stays in registers.  Bound by its bytes: 2048 tokens of 3 x 4096 values take
+// 50 us in k_seq_qkv_finish and 42 us here, 37 tokens of 6144 in four parts 13 and 8.6 us.
+template <typename T, int U>
+__global__ __launch_bounds__(kSeqThreads) void k_seq_qkv_finish4(SeqQkv a) {
+    __shared__ float2 red[kSeqWaves];
+    const int t = blockIdx.x, tid = threadIdx.x, nq = a.H * a.D, nk = a.G * a.D, nv = a.G * a.V, n4 = (nq + nk + nv) / 4;
+    const f32x4* row = reinterpret_cast<const f32x4*>(a.qkv + (size_t)t * a.ld);
+    f32x4 x[U];
+#pragma unroll
+    for (int j = 0; j < U; ++j) x[j] = row[min(tid + j * kSeqThreads, n4 - 1)];
+    for (int p = 1; p < a.parts; ++p) {
+        const f32x4* r = reinterpret_cast<const f32x4*>(a.qkv + (size_t)t * a.ld + p * a.part_stride);
+#pragma unroll
+        for (int j = 0; j < U; ++j) x[j] += r[min(tid + j * kSeqThreads, n4 - 1)];
+    }
+    float sq = 0.0f, sk = 0.0f;
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+        const int i = (tid + j * kSeqThreads) * 4;
+        float s = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s = fmadd(x[j][r], x[j][r], s);
+        sq += i < nq ? s : 0.0f;
+        sk += i >= nq && i < nq + nk ? s : 0.0f;
+    }
+    const float2 sums = block_sum2(sq, sk, red);
+    const float iq = inv_rms(sums.x, nq, a.eps), ik = inv_rms(sums.y, nk, a.eps);
+    const float2* cs = a.cs + (size_t)(a.pos0 + t) * (a.rot / 2);
+    char* qo = a.q + (size_t)t * a.H * a.Dp * sizeof(T);
+    char* ko = a.k + (size_t)t * a.Dp * sizeof(T);
+    char* vo = a.v + (size_t)t * a.Vp * sizeof(T);
+    const float rd = 1.0f / (float)a.D, rv = 1.0f / (float)a.V;
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+        const int i = (tid + j * kSeqThreads) * 4;
+        if (i >= nq + nk + nv) continue;
+        if (i < nq + nk) {
+            const bool q = i < nq;
+            const int e = q ? i : i - nq, h = (int)(((float)e + 0.5f) * rd), d = e - h * a.D;      // (e < 2^16: exact)
+            const f32x4 w = *reinterpret_cast<const f32x4*>((q ? a.qn : a.kn) + e);
+            const float inv = q ? iq : ik;
+            f32x4 y;
+#pragma unroll
+            for (int r = 0; r < 4; r += 2) {
+                const float2 cc = d + r < a.rot ? cs[(d + r) / 2] : make_float2(1.0f, 0.0f);
+                const float u = x[j][r] * w[r], v = x[j][r + 1] * w[r + 1];
+                y[r] = rotate_finish(RotIn{u, v, cc.x, -cc.y}, inv);
+                y[r + 1] = rotate_finish(RotIn{v, u, cc.x, cc.y}, inv);
+            }
+            store4<T>((q ? qo + (size_t)h * a.Dp * sizeof(T) : ko + h * a.khead) + d * sizeof(T), y);
+        } else {
+            const int e = i - nq - nk, g = (int)(((float)e + 0.5f) * rv), d = e - g * a.V;
+            f32x4 y = x[j];
+            f32x4* first = reinterpret_cast<f32x4*>(a.v_first + (size_t)t * nv + e);
+            if (a.v_role == 1) *first = y;
+            if (a.v_role == 2) {
+                const f32x4 f = *first;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) y[r] = (1.0f - a.lambda) * y[r] + a.lambda * f[r];
+            }
+            store4<T>(vo + g * a.vhead + d * sizeof(T), y);
+        }
+    }
+    // zeros behind the heads: layers of other sizes share these buffers
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    const int dz = (a.Dp - a.D) / 4, vz = (a.Vp - a.V) / 4;
+    if (dz > 0)
+        for (int i = tid; i < (a.H + a.G) * dz; i += kSeqThreads) {
+            const int h = i / dz, d = a.D + (i - h * dz) * 4;
+            store4<T>((h < a.H ? qo + (size_t)h * a.Dp * sizeof(T) : ko + (h - a.H) * a.khead) + d * sizeof(T), zero);
+        }
+    if (vz > 0)
+        for (int i = tid; i < a.G * vz; i += kSeqThreads) {
+            const int g = i / vz, d = a.V + (i - g * vz) * 4;
+            store4<T>(vo + g * a.vhead + d * sizeof(T), zero);
+        }
 }
 
 // Portion rows -> cache rows: one workgroup per kept position.
@@ -1168,12 +1249,20 @@ template <typename T>
 void portion_grouped(cfpp_seq* s, const LayerPlan& L, int slot, int n, int pos, int parts, hipStream_t st) {
     const cfpp_seq_layer& d = L.d;
     const int cap = s->portion;
-    SeqQkv f{s->qkv, s->ld_qkv, parts, (size_t)n * s->ld_qkv, d.q_norm, d.k_norm, L.cs, s->d.eps, d.v_lambda, d.heads, d.kv_heads, d.dim, L.Dp, d.vdim, L.Vp,
-             d.rot_dims, pos, cap, L.v_role, s->v_first, s->q, s->k, s->v};
-    hipLaunchKernelGGL(k_seq_qkv_finish<T>, dim3(n), dim3(kSeqThreads), 0, st, f);
-
     char* kc = L.kc + (size_t)slot * d.kv_heads * L.rows * L.krow;
     char* vc = L.vc + (size_t)slot * d.kv_heads * L.rows * L.vrow;
+    // The portion's keys and values go straight into the cache, unless it crosses the edge of a chunk: then it would overwrite rows
+    // that its first tokens still see, and only what the last chunk needs is kept afterwards.
+    const int last = pos + n - 1, cs0 = d.chunk > 0 ? last / d.chunk * d.chunk : 0, first = std::max(pos, cs0) - pos;
+    const bool direct = cs0 <= pos;
+    SeqQkv f{s->qkv, s->ld_qkv, parts, (size_t)n * s->ld_qkv, d.q_norm, d.k_norm, L.cs, s->d.eps, d.v_lambda, d.heads, d.kv_heads, d.dim, L.Dp, d.vdim, L.Vp,
+             d.rot_dims, pos, (size_t)(direct ? L.rows : cap) * L.krow, (size_t)(direct ? L.rows : cap) * L.vrow, L.v_role, s->v_first, s->q,
+             direct ? kc + (size_t)(pos - cs0) * L.krow : s->k, direct ? vc + (size_t)(pos - cs0) * L.vrow : s->v};
+    auto finish = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(n), dim3(kSeqThreads), 0, st, f); };
+    if (d.dim % 4 == 0 && d.vdim % 4 == 0 && L.n_qkv <= 8 * 4 * kSeqThreads) finish(k_seq_qkv_finish4<T, 8>);
+    else if (d.dim % 4 == 0 && d.vdim % 4 == 0 && L.n_qkv <= 16 * 4 * kSeqThreads) finish(k_seq_qkv_finish4<T, 16>);
+    else finish(k_seq_qkv_finish<T>);
+
     SeqAttn a{};
     a.q = s->q;
     a.k = s->k;
@@ -1190,7 +1279,8 @@ void portion_grouped(cfpp_seq* s, const LayerPlan& L, int slot, int n, int pos, 
     a.vrow = L.vrow;
     a.V = d.vdim;
     a.vtiles = L.Vp / 16;
-    a.pos0 = a.k_split = pos;
+    a.pos0 = pos;
+    a.k_split = direct ? pos + n : pos;
     a.chunk = d.chunk;
     a.cap = cap;
     a.rows = L.rows;
@@ -1198,7 +1288,7 @@ void portion_grouped(cfpp_seq* s, const LayerPlan& L, int slot, int n, int pos, 
     a.scale_log2 = d.scale * kLog2e;
     attn<T>(s, a, d.kv_heads, st);
 
-    const int last = pos + n - 1, cs0 = d.chunk > 0 ? last / d.chunk * d.chunk : 0, first = std::max(pos, cs0) - pos;
+    if (direct) return;
     SeqAppend ap{s->k, s->v, kc, vc, d.kv_heads, L.krow, L.vrow, cap, L.rows, first, pos + first - cs0};
     hipLaunchKernelGGL(k_seq_append, dim3(n - first), dim3(kSeqThreads), 0, st, ap);
 }

@@ -39,3 +39,20 @@ def test_portions_far_into_a_sequence(name, dtype):
         assert N.error(logits, want[pos:pos + n]) < LIMIT[dtype], (pos, n)
         pos += n
     assert pos == 1300
+
+
+# projections of up to 8192 and 16384 values, and of more; heads that are no whole groups of four; values mixed; padded heads
+PROJECTIONS = {"12k": [N.attn(64, 16, 128, 128)], "17k": [N.attn(128, 4, 128, 128)], "mixed_12k": [N.attn(48, 12, 100, 132, v_mix=True, chunk=31), N.attn(48, 12, 100, 132, v_mix=True)],
+               "no_fours": [N.attn(6, 2, 42, 30, v_mix=True), N.attn(6, 2, 40, 30, v_mix=True), N.attn(10, 5, 42, 12, v_mix=True)]}
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("name", list(PROJECTIONS))
+def test_projection_sizes(name, dtype):
+    from clusterfusionplus_amd import nibotar
+    cfg = N.model(64, 51, [(m, None) for m in PROJECTIONS[name]])
+    w, toks = N.weights(cfg, 5), N.prompt(cfg, 90, 6)
+    want = N.oracle(cfg, w, toks)
+    m = nibotar.from_tensors(cfg, w, dtype, capacity=100)
+    logits = torch.cat([m.forward(0, toks[:33], 0, range(33)), m.forward(0, toks[33:62], 33, range(29)), m.forward(0, toks[62:], 62, range(28))])
+    assert N.error(logits, want) < LIMIT[dtype]
