@@ -318,32 +318,47 @@ __global__ __launch_bounds__(kSeqThreads, (NT <= 128 ? 2 : 1)) void k_seq_attn(S
     }
 }
 
-// Workgroup (token, 256 groups of four output columns): the splits' sums, relative to the largest maximum, with the sink and the gate.
-template <typename T>
+// Workgroup (token, 256 groups of four output columns): the splits' sums, relative to the largest maximum, with the sink and the
+// gate.  At most S splits, all of them requested before the first is used.
+template <typename T, int S>
 __global__ __launch_bounds__(kSeqThreads) void k_seq_attn_merge(SeqAttn a) {
     const int t = blockIdx.x, per = a.vtiles * 4, i = blockIdx.y * kSeqThreads + threadIdx.x, h = i / per, v0 = (i - h * per) * 4;
     if (h >= a.H) return;
-    const float snk = a.sink != nullptr ? a.sink[h] * kLog2e : kNegBig;
     const size_t row0 = (size_t)t * a.H + h, step = (size_t)a.T * a.H;
+    float2 ml[S];
+    f32x4 p[S];
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+        if (s < a.splits) {
+            ml[s] = *reinterpret_cast<const float2*>(a.ml + (row0 + s * step) * 2);
+            p[s] = *reinterpret_cast<const f32x4*>(a.part + (row0 + s * step) * (a.vtiles * 16) + v0);
+        }
+    const float snk = a.sink != nullptr ? a.sink[h] * kLog2e : kNegBig;
     float m = snk;
-    for (int s = 0; s < a.splits; ++s) m = fmaxf(m, a.ml[(row0 + s * step) * 2]);
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+        if (s < a.splits) m = fmaxf(m, ml[s].x);
     float l = fast_exp2(snk - m);
     f32x4 y = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-    for (int s = 0; s < a.splits; ++s) {
-        const size_t row = row0 + s * step;
-        const float2 ml = *reinterpret_cast<const float2*>(a.ml + row * 2);
-        const f32x4 p = *reinterpret_cast<const f32x4*>(a.part + row * (a.vtiles * 16) + v0);
-        const float c = fast_exp2(ml.x - m);
-        l = fmadd(ml.y, c, l);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) y[r] = fmadd(p[r], c, y[r]);
-    }
+    for (int s = 0; s < S; ++s)
+        if (s < a.splits) {
+            const float c = fast_exp2(ml[s].x - m);
+            l = fmadd(ml[s].y, c, l);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) y[r] = fmadd(p[s][r], c, y[r]);
+        }
     T* o = reinterpret_cast<T*>(a.out + (size_t)t * a.ldo) + h * a.V;
     const float* gate = a.gate + (size_t)t * a.ldg + h * a.V;
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-        if (v0 + r < a.V) o[v0 + r] = from_f32<T>(a.gate != nullptr ? y[r] / l * sigmoid(gate[v0 + r]) : y[r] / l);
+    for (int r = 0; r < 4; ++r) y[r] = a.gate != nullptr && v0 + r < a.V ? y[r] / l * sigmoid(gate[v0 + r]) : y[r] / l;
+    if ((a.V & 3) == 0) {
+        if (v0 < a.V) store4<T>(o + v0, y);
+    } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (v0 + r < a.V) o[v0 + r] = from_f32<T>(y[r]);
+    }
 }
 
 }  // namespace cfpp

@@ -211,6 +211,26 @@ __device__ __forceinline__ void merge_parts(float* row, int n, int parts, size_t
     __syncthreads();
 }
 
+// A row of n4 groups of four values in the registers of a workgroup: group tid + j kSeqThreads is x[j] (past the end: the last one).
+// Adds `parts` rows, `stride` floats apart, in order; the loads of C of them are in flight together.
+template <int U, int C> __device__ __forceinline__ void add_rows4(f32x4 (&x)[U], const float* __restrict__ rows, int parts, size_t stride, int n4) {
+    for (int p = 0; p < parts; p += C) {
+        f32x4 r[C][U];
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+            if (p + c < parts) {
+#pragma unroll
+                for (int j = 0; j < U; ++j) r[c][j] = reinterpret_cast<const f32x4*>(rows + (p + c) * stride)[min((int)threadIdx.x + j * kSeqThreads, n4 - 1)];
+            }
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+            if (p + c < parts) {
+#pragma unroll
+                for (int j = 0; j < U; ++j) x[j] += r[c][j];
+            }
+    }
+}
+
 // Element d of head h of a run of heads (D elements each) after the norm over the whole projection and the rotation: the
 // element and its partner with their norm weights, and (cos, sin) of the pair.  `row` is the run in the projection, `w` in
 // the norm weight, `cs` the pairs of the position.

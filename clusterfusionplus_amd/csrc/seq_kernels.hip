@@ -149,6 +149,55 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_postnorm(SeqPostNorm a) {
     for (int i = w4 + threadIdx.x; i < a.width; i += kSeqThreads) out(std::integral_constant<int, 1>{}, i, inv);
 }
 
+// The same for rows of whole groups of four elements, up to 1024 U of them: the row stays in registers, and everything is requested
+// before anything is used.  Bound by its bytes where there are many tokens (2048 of 4096 values: 25 us for 150 MB), by one round trip
+// and two barriers where there are few (37 tokens, four parts: 8.8 us in k_seq_postnorm and 4.6 us here).
+template <typename T, int U>
+__global__ __launch_bounds__(kSeqThreads) void k_seq_postnorm4(SeqPostNorm a) {
+    __shared__ float red[kSeqWaves];
+    const int t = a.rows != nullptr ? a.rows[blockIdx.x] : (int)blockIdx.x, tid = threadIdx.x, n4 = a.width / 4;
+    f32x4 v[U], w[U], s[U];
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+        const int i = min(tid + j * kSeqThreads, n4 - 1);
+        v[j] = reinterpret_cast<const f32x4*>(a.x + (size_t)t * a.width)[i];
+        w[j] = reinterpret_cast<const f32x4*>(a.w)[i];
+        s[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    if (a.ys != nullptr) {
+        add_rows4<U, (U <= 4 ? 4 : 2)>(s, a.ys + (size_t)t * a.top * a.width, a.top, a.width, n4);
+#pragma unroll
+        for (int j = 0; j < U; ++j) s[j] *= a.slot_weight;
+    }
+    if (a.y != nullptr) add_rows4<U, (U <= 4 ? 4 : 2)>(s, a.y + (size_t)t * a.width, a.parts, a.part_stride, n4);
+    float ss = 0.0f;
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+        if (a.rows == nullptr) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[j][r] = fmadd(a.alpha, v[j][r], s[j][r]);
+        }
+        if (tid + j * kSeqThreads < n4) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) ss = fmadd(v[j][r], v[j][r], ss);
+        }
+    }
+    const float inv = inv_rms(block_sum(ss, red), a.width, a.eps);
+    T* xb = reinterpret_cast<T*>(a.xb + (size_t)blockIdx.x * a.pitch);
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+        const int i = tid + j * kSeqThreads;
+        if (i >= n4) continue;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[j][r] = v[j][r] * inv * (a.noff + w[j][r]);
+        if (a.rows == nullptr) {
+            reinterpret_cast<f32x4*>(a.x_out + (size_t)t * a.width)[i] = v[j];
+            if (a.copy != nullptr) reinterpret_cast<f32x4*>(a.copy + (size_t)t * a.width)[i] = v[j];
+        }
+        store4<T>(xb + i * 4, v[j]);
+    }
+}
+
 // One workgroup per token: raw q | k | v rows (fp32, biases included) -> norm over all of q and all of k, rotation, value
 // mixing -> q [T][H][Dp], k [G][..][Dp] and v [G][..][Vp]: rows of the portion's buffers, or of the cache itself.
 struct SeqQkv {
@@ -233,15 +282,10 @@ template <typename T, int U>
 __global__ __launch_bounds__(kSeqThreads) void k_seq_qkv_finish4(SeqQkv a) {
     __shared__ float2 red[kSeqWaves];
     const int t = blockIdx.x, tid = threadIdx.x, nq = a.H * a.D, nk = a.G * a.D, nv = a.G * a.V, n4 = (nq + nk + nv) / 4;
-    const f32x4* row = reinterpret_cast<const f32x4*>(a.qkv + (size_t)t * a.ld);
     f32x4 x[U];
 #pragma unroll
-    for (int j = 0; j < U; ++j) x[j] = row[min(tid + j * kSeqThreads, n4 - 1)];
-    for (int p = 1; p < a.parts; ++p) {
-        const f32x4* r = reinterpret_cast<const f32x4*>(a.qkv + (size_t)t * a.ld + p * a.part_stride);
-#pragma unroll
-        for (int j = 0; j < U; ++j) x[j] += r[min(tid + j * kSeqThreads, n4 - 1)];
-    }
+    for (int j = 0; j < U; ++j) x[j] = reinterpret_cast<const f32x4*>(a.qkv + (size_t)t * a.ld)[min(tid + j * kSeqThreads, n4 - 1)];
+    add_rows4<U, (U <= 8 ? 3 : 1)>(x, a.qkv + (size_t)t * a.ld + a.part_stride, a.parts - 1, a.part_stride, n4);
     float sq = 0.0f, sk = 0.0f;
 #pragma unroll
     for (int j = 0; j < U; ++j) {
@@ -1196,8 +1240,10 @@ void launch_attn(SeqAttn a, int G, int cus, size_t room, float* part, hipStream_
     };
     if (a.runits > 0) pick(std::true_type{});
     else pick(std::false_type{});
-    if (a.splits > 1)
-        hipLaunchKernelGGL(k_seq_attn_merge<T>, dim3(a.T, ceil_div(a.H * a.vtiles * 4, kSeqThreads)), dim3(kSeqThreads), 0, st, a);
+    auto merge = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(a.T, ceil_div(a.H * a.vtiles * 4, kSeqThreads)), dim3(kSeqThreads), 0, st, a); };
+    if (a.splits > 8) merge(k_seq_attn_merge<T, 16>);
+    else if (a.splits > 4) merge(k_seq_attn_merge<T, 8>);
+    else if (a.splits > 1) merge(k_seq_attn_merge<T, 4>);
 }
 
 template <typename T>
@@ -1211,6 +1257,10 @@ void attn(const cfpp_seq* s, const SeqAttn& a, int G, hipStream_t st) {
 
 template <typename T>
 void postnorm(const cfpp_seq* s, const SeqPostNorm& n, int rows, hipStream_t st) {
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(rows), dim3(kSeqThreads), 0, st, n); };
+    if (s->d.width % 4 == 0 && s->d.width <= 2048) return go(k_seq_postnorm4<T, 2>);
+    if (s->d.width % 4 == 0 && s->d.width <= 4096) return go(k_seq_postnorm4<T, 4>);
+    if (s->d.width % 4 == 0 && s->d.width <= 8192) return go(k_seq_postnorm4<T, 8>);
     const size_t lds = (size_t)s->d.width * 4;
     allow_lds(k_seq_postnorm<T>, lds);
     hipLaunchKernelGGL(k_seq_postnorm<T>, dim3(rows), dim3(kSeqThreads), lds, st, n);
@@ -1226,6 +1276,11 @@ void streams(const cfpp_seq* s, SeqStreams a, int rows, hipStream_t st) {
     a.noff = s->d.norm_offset;
     auto go = [&](auto n) {
         constexpr int S = decltype(n)::value;
+        auto in_registers = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(rows), dim3(kSeqThreads), 0, st, a); };
+        if constexpr (S <= 4) {
+            if (a.width % 4 == 0 && a.width <= 2048) return in_registers(k_seq_streams4<T, S, 2>);
+            if (a.width % 4 == 0 && a.width <= 4096) return in_registers(k_seq_streams4<T, S, 4>);
+        }
         allow_lds(k_seq_streams<T, S>, lds);
         hipLaunchKernelGGL((k_seq_streams<T, S>), dim3(rows), dim3(kSeqThreads), lds, st, a);
     };

@@ -571,4 +571,89 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_streams(SeqStreams a) {
     for (int i = w4 + threadIdx.x; i < a.width; i += kSeqThreads) put(std::integral_constant<int, 1>{}, i);
 }
 
+// The same for rows of whole groups of four elements, up to 1024 U of them: the streams stay in registers, and everything is requested
+// before anything is used.
+template <typename T, int S, int U>
+__global__ __launch_bounds__(kSeqThreads) void k_seq_streams4(SeqStreams a) {
+    __shared__ float red[kSeqWaves];
+    const int t = a.rows != nullptr ? a.rows[blockIdx.x] : (int)blockIdx.x, tid = threadIdx.x, n4 = a.width / 4;
+    float* x = a.x + (size_t)t * a.streams * a.width;
+    f32x4 o[S][U], w[U], y[U];
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+        const int i = min(tid + j * kSeqThreads, n4 - 1);
+        if (a.tokens == nullptr) {
+#pragma unroll
+            for (int s = 0; s < S; ++s) o[s][j] = reinterpret_cast<const f32x4*>(x + (size_t)min(s, a.streams - 1) * a.width)[i];
+        } else {
+            const T* e = reinterpret_cast<const T*>(a.embed + (size_t)a.tokens[t] * a.embed_pitch) + i * 4;
+            const T* p = a.pos != nullptr ? reinterpret_cast<const T*>(a.pos + (size_t)(a.state != nullptr ? a.state[1] : a.pos0 + t) * a.embed_pitch) + i * 4 : nullptr;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[0][j][r] = to_f32(e[r]) + (p != nullptr ? to_f32(p[r]) : 0.0f);
+#pragma unroll
+            for (int s = 1; s < S; ++s) o[s][j] = o[0][j];
+        }
+        w[j] = a.w != nullptr ? reinterpret_cast<const f32x4*>(a.w)[i] : f32x4{0.f, 0.f, 0.f, 0.f};
+        y[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    if (a.ys != nullptr) {
+        add_rows4<U, 2>(y, a.ys + (size_t)t * a.top * a.width, a.top, a.width, n4);
+#pragma unroll
+        for (int j = 0; j < U; ++j) y[j] *= a.slot_weight;
+    }
+    if (a.y != nullptr) add_rows4<U, (U <= 2 ? 4 : 2)>(y, a.y + (size_t)t * a.width, a.parts, a.part_stride, n4);
+    float ss = 0.0f;
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+        const int i = tid + j * kSeqThreads;
+        if (a.tokens == nullptr && a.mix != nullptr) {
+            f32x4 v[S];
+#pragma unroll
+            for (int s = 0; s < S; ++s) {
+                const bool live = s < a.streams;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[s][r] = (live ? a.out[s] : 0.0f) * y[j][r];
+#pragma unroll
+                for (int k = 0; k < S; ++k) {
+                    const float m = live && k < a.streams ? a.mix[k * a.streams + s] : 0.0f;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[s][r] = fmadd(m, o[k][j][r], v[s][r]);
+                }
+            }
+#pragma unroll
+            for (int s = 0; s < S; ++s) o[s][j] = v[s];
+        }
+        f32x4 u = {0.f, 0.f, 0.f, 0.f}, all = u;
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+            if (s < a.streams) {
+                const float in = a.in != nullptr ? a.in[s] : 1.0f;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) u[r] = fmadd(in, o[s][j][r], u[r]);
+                all += o[s][j];
+            }
+        if (i < n4) {
+            if (a.rows == nullptr) {
+#pragma unroll
+                for (int s = 0; s < S; ++s)
+                    if (s < a.streams) reinterpret_cast<f32x4*>(x + (size_t)s * a.width)[i] = o[s][j];
+            }
+            if (a.copy != nullptr) reinterpret_cast<f32x4*>(a.copy + (size_t)t * a.width)[i] = all;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) ss = fmadd(u[r], u[r], ss);
+        }
+        y[j] = u;
+    }
+    if (a.w == nullptr) return;
+    const float inv = inv_rms(block_sum(ss, red), a.width, a.eps);
+    T* xb = reinterpret_cast<T*>(a.xb + (size_t)blockIdx.x * a.pitch);
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+        const int i = tid + j * kSeqThreads;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) y[j][r] = y[j][r] * inv * (a.noff + w[j][r]);
+        if (i < n4) store4<T>(xb + i * 4, y[j]);
+    }
+}
+
 }  // namespace cfpp
