@@ -103,6 +103,10 @@ __device__ __forceinline__ const char* uniform(const char* p) {
 __device__ __forceinline__ void copy_to_lds16_at(uint32_t off, const void* base, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory");
 }
+// ... of bytes that nobody reads again: they leave the caches to the others'
+__device__ __forceinline__ void copy_to_lds16_once(uint32_t off, const void* base, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(off), "s"(base), "s"(lds) : "memory");
+}
 __device__ __forceinline__ void copy_to_lds16_from(const void* p, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(p), "s"(lds) : "memory");
 }

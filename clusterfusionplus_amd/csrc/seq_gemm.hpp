@@ -36,6 +36,9 @@ struct SeqGemm {
     const int* slots;        // sorted slots: token * top + j
     int experts, slot_div;   // input row of slot s: s / slot_div
     size_t w_stride;
+    // (k_seq_gemm) The weights are read by one tile of tokens only, as a stream past the caches, in which the inputs stay: 37 tokens x 14336 x 4096
+    // 27.1 -> 24.8 us, 64 experts of 2816 x 2048 with 66 tokens each 171 -> 159 us; with two token tiles it costs (36 -> 42 us).
+    int once;
     int splits;              // of k (kEpiF32); the s-th partial result lies s * split_stride floats behind yf
     size_t split_stride;
 };
@@ -216,7 +219,10 @@ __global__ __launch_bounds__(kWave* WR* WC) void k_seq_gemm(SeqGemm p) {
     auto request = [&]() __attribute__((always_inline)) {
         const uint32_t b = l0 + fill * kStep;
 #pragma unroll
-        for (int i = 0; i < WI; ++i) copy_to_lds16_at(vw[i], bw, b + (wave + i * NW) * 1024);
+        for (int i = 0; i < WI; ++i) {
+            if (p.once) copy_to_lds16_once(vw[i], bw, b + (wave + i * NW) * 1024);
+            else copy_to_lds16_at(vw[i], bw, b + (wave + i * NW) * 1024);
+        }
 #pragma unroll
         for (int i = 0; i < AI; ++i) copy_to_lds16_at(va[i], ba, b + BW * kRowBytes + min(wave + i * NW, AC - 1) * 1024);
         bw += kRowBytes;

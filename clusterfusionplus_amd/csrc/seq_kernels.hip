@@ -1096,20 +1096,22 @@ void allow_lds(K kernel, size_t bytes) {
 // it chooses is 2 % slower than the best choice on average, 20 % at worst.  (Two more tiles, 128 x 96 and 128 x 160, were within
 // 0.2 % of the others on average and are left out.)
 struct GemmShape { int rows, tokens, resident; float step, share, fixed; };
-constexpr GemmShape kShapes16[] = {{64, 16, 2, 0.190f, 0.177f, 1.5f}, {64, 32, 2, 0.179f, 0.201f, 1.8f}, {64, 64, 2, 0.256f, 0.239f, 2.2f},
-                                   {64, 96, 2, 0.297f, 0.280f, 2.8f}, {128, 128, 2, 0.705f, 0.549f, 5.0f}, {256, 128, 1, 0.862f, 0.862f, 6.9f},
-                                   {256, 256, 1, 1.104f, 1.104f, 12.9f}};
-constexpr GemmShape kShapes32[] = {{64, 16, 2, 0.270f, 0.212f, 1.7f}, {64, 32, 2, 0.357f, 0.312f, 2.0f}, {64, 64, 3, 0.586f, 0.515f, 2.7f},
-                                   {128, 128, 2, 1.619f, 1.959f, 5.8f}};
+constexpr GemmShape kShapes16[] = {{64, 16, 2, 0.213f, 0.180f, 1.7f}, {64, 32, 2, 0.228f, 0.204f, 1.9f}, {64, 64, 2, 0.269f, 0.241f, 2.4f},
+                                   {64, 96, 2, 0.304f, 0.282f, 2.9f}, {256, 96, 1, 0.804f, 0.804f, 5.5f}, {128, 128, 2, 0.618f, 0.618f, 5.3f},
+                                   {256, 128, 1, 0.919f, 0.919f, 6.9f}, {256, 256, 1, 1.098f, 1.098f, 13.9f}};
+constexpr GemmShape kShapes32[] = {{64, 16, 2, 0.285f, 0.215f, 1.7f}, {64, 32, 2, 0.393f, 0.320f, 2.0f}, {64, 64, 3, 0.614f, 0.520f, 2.7f},
+                                   {128, 128, 2, 1.865f, 1.957f, 5.9f}};
 struct GemmPlan { int shape, splits; };
 
-// `tiles` tiles of `steps` steps on `cus` compute units; a stream of weights of `bytes` bytes takes what 5.8 TB/s take.
-float gemm_cost(const GemmShape& c, double tiles, float steps, int cus, double bytes) {
+// `tiles` tiles of `steps` steps on `cus` compute units
+float gemm_tiles_cost(const GemmShape& c, double tiles, float steps, int cus) {
     const int load = (int)ceil(tiles / cus), full = load / c.resident, rest = load % c.resident;
     float t = full * (steps * std::max(c.step, c.resident * c.share) + c.fixed);
     if (rest > 0) t += steps * std::max(c.step, rest * c.share) + c.fixed;
-    return std::max(t, (float)(bytes / 5.8e6));
+    return t;
 }
+// what a stream of so many bytes takes at 5.8 TB/s
+float stream_cost(double bytes) { return (float)(bytes / 5.8e6); }
 
 // The cheapest tile, and with `room` floats for partial results the cheapest number of splits of k as well.  Reading a partial
 // result costs its bytes at 5 TB/s, and 0.3 us.  No split has fewer than three steps.
@@ -1125,7 +1127,7 @@ GemmPlan plan_gemm(const cfpp_seq* s, const SeqGemm& g, size_t room) {
         for (int sp : kSplits) {
             if (sp > 1 && (room == 0 || nk / sp < 3 || (size_t)sp * g.m * g.ldy > room)) break;
             const double tiles = (double)ceil_div(g.n, shapes[i].rows) * ceil_div(g.m, shapes[i].tokens) * sp;
-            float t = gemm_cost(shapes[i], tiles, (float)nk / sp, s->cus, (double)g.n * g.kbytes);
+            float t = std::max(gemm_tiles_cost(shapes[i], tiles, (float)nk / sp, s->cus), stream_cost((double)g.n * g.kbytes));
             if (sp > 1) t += 0.3f + 4e-6f * sp * g.m * g.n / 5.0f;
             if (t < least) {
                 least = t;
@@ -1151,8 +1153,9 @@ void launch_shape(const SeqGemm& g, int shape, int tiles_t, hipStream_t st) {
             case 1: return launch_gemm<T, 64, 32, 4, 1, 5, EPI>(g, tiles_t, st);
             case 2: return launch_gemm<T, 64, 64, 2, 2, 4, EPI>(g, tiles_t, st);
             case 3: return launch_gemm<T, 64, 96, 2, 2, 4, EPI>(g, tiles_t, st);
-            case 4: return launch_gemm<T, 128, 128, 2, 2, 2, EPI>(g, tiles_t, st);
-            case 5: return launch_gemm<T, 256, 128, 4, 2, 3, EPI>(g, tiles_t, st);
+            case 4: return launch_gemm<T, 256, 96, 8, 1, 3, EPI>(g, tiles_t, st);
+            case 5: return launch_gemm<T, 128, 128, 2, 2, 2, EPI>(g, tiles_t, st);
+            case 6: return launch_gemm<T, 256, 128, 4, 2, 3, EPI>(g, tiles_t, st);
         }
         constexpr size_t lds = 2 * 512 * kRowBytes;
         allow_lds(k_seq_gemm8<EPI>, lds);
@@ -1173,43 +1176,50 @@ int gemm(const cfpp_seq* s, SeqGemm g, hipStream_t st, size_t room = 0) {
     const GemmPlan plan = plan_gemm<T>(s, g, EPI == kEpiF32 ? room : 0);
     g.splits = plan.splits;
     g.split_stride = (size_t)g.m * g.ldy;
-    launch_shape<T, EPI>(g, plan.shape, ceil_div(g.m, (sizeof(T) == 2 ? kShapes16 : kShapes32)[plan.shape].tokens), st);
+    const int tiles_t = ceil_div(g.m, (sizeof(T) == 2 ? kShapes16 : kShapes32)[plan.shape].tokens);
+    g.once = tiles_t == 1;
+    launch_shape<T, EPI>(g, plan.shape, tiles_t, st);
     return plan.splits;
 }
 
 // Tile of the expert products of a portion of n tokens (both use it).  An expert has avg +- sqrt(avg) of them; where that fits a
-// tile, it has one, and the product is a stream of weights.
-int expert_shape(const cfpp_seq* s, const LayerPlan& L, int n) {
+// tile, it has one (`once`), and the product is a stream of weights.  A stream hides the tiles' own time only in part: with 66 tokens
+// per expert, 64 experts of 2816 x 2048 take 159 us in tiles of 64 x 96, estimated at 118, and 151 us in tiles of 256 x 96, at 94.
+struct ExpertPlan { int shape, tokens, once; };
+ExpertPlan expert_plan(const cfpp_seq* s, const LayerPlan& L, int n) {
     const GemmShape* shapes = s->esize == 2 ? kShapes16 : kShapes32;
     const int count = s->esize == 2 ? (int)std::size(kShapes16) : (int)std::size(kShapes32);
     const double avg = (double)n * L.d.top / L.d.experts, live = L.d.experts * std::min(1.0, avg);
-    int best = 0;
+    const float stream = stream_cost(live * 2.0 * L.d.ff * s->xpitch);
+    ExpertPlan best{};
     float least = INFINITY;
     for (int i = 0; i < count; ++i) {
         const GemmShape& c = shapes[i];
-        const double per = avg + 1.5 * sqrt(avg) <= c.tokens ? 1.0 : std::max(1.0, avg / c.tokens + 0.5);
-        const float t = gemm_cost(c, live * per * ceil_div(2 * L.d.ff, c.rows), (float)s->xpitch / kRowBytes, s->cus, live * 2.0 * L.d.ff * s->xpitch);
-        if (t < least) {
-            least = t;
-            best = i;
+        const bool one = avg + 1.5 * sqrt(avg) <= c.tokens;
+        const double per = one ? 1.0 : std::max(1.0, avg / c.tokens + 0.5);
+        const float t = gemm_tiles_cost(c, live * per * ceil_div(2 * L.d.ff, c.rows), (float)s->xpitch / kRowBytes, s->cus);
+        const float cost = std::max(t, stream) + 0.3f * std::min(t, stream);
+        if (cost < least) {
+            least = cost;
+            best = {i, c.tokens, one};
         }
     }
     return best;
 }
-// tokens per tile of the expert products
-int expert_tile(const cfpp_seq* s, const LayerPlan& L, int n) { return (s->esize == 2 ? kShapes16 : kShapes32)[expert_shape(s, L, n)].tokens; }
 
 template <typename T, int EPI>
 void expert_gemm(const cfpp_seq* s, const LayerPlan& L, SeqGemm g, int n, hipStream_t st) {
     const SeqRoute& r = s->host_routes[L.route];
-    const int shape = expert_shape(s, L, n), slots = n * L.d.top;
+    const ExpertPlan plan = expert_plan(s, L, n);
+    const int slots = n * L.d.top;
     g.m = slots;
     g.tile_off = r.tile_off;
     g.row_off = r.row_off;
     g.slots = r.slots;
     g.experts = L.d.experts;
     g.splits = 1;
-    launch_shape<T, EPI>(g, shape, slots / expert_tile(s, L, n) + std::min(L.d.experts, slots), st);
+    g.once = plan.once;
+    launch_shape<T, EPI>(g, plan.shape, slots / plan.tokens + std::min(L.d.experts, slots), st);
 }
 
 // Columns of a workgroup and splits of the keys.  bf16: two column tiles per wave share the reads of keys and values; one, where that
@@ -1434,12 +1444,12 @@ int run_portion(cfpp_seq* s, int slot, int n, int pos, int n_want, float* logits
             for (; j < s->layers.size(); ++j) {
                 const LayerPlan& M = s->layers[j];
                 if (M.route < 0) continue;
-                if (expert_tile(s, M, n) != expert_tile(s, L, n)) break;
+                if (expert_plan(s, M, n).tokens != expert_plan(s, L, n).tokens) break;
                 ++count;
             }
             const size_t lds = (size_t)s->max_experts * 8;
             allow_lds(k_seq_route, lds);
-            hipLaunchKernelGGL(k_seq_route, dim3((unsigned)count), dim3(1024), lds, st, s->routes + L.route, s->tokens, n, expert_tile(s, L, n));
+            hipLaunchKernelGGL(k_seq_route, dim3((unsigned)count), dim3(1024), lds, st, s->routes + L.route, s->tokens, n, expert_plan(s, L, n).tokens);
             i = j - 1;
         }
     }
