@@ -267,11 +267,11 @@ __global__ __launch_bounds__(kWave* WR* WC) void k_seq_gemm(SeqGemm p) {
 }
 
 // 256 rows x 256 tokens, eight waves of 128 x 64 in two groups of four (waves i and i + 4 share a SIMD) that take turns: while one
-// group multiplies a quarter of its step's products, the other reads the operands of its next quarter from LDS and requests copies.
-// Group 1 runs one barrier behind.  The quarters of step k are (W half 0, A half 0), (W0, A1), (W1, A1), (W1, A0); a half is read by
-// all waves in the quarter that first needs it, and the copies of the same half two steps on (one step on for A1 and W1, which are read
-// late) go to its place two quarters later, when both groups have read it.  Requests go in the order in which the halves are
-// needed, always four halves ahead: 8 copies of a wave stay in flight behind each wait.
+// group multiplies a quarter of its step's products, the other reads operands from LDS and requests copies.  Group 1 runs one
+// barrier behind.  The quarters of step k are (W half 0, A half 0), (W0, A1), (W1, A1), (W1, A0); their reads are spread evenly, 8, 8, 4 and 4 per
+// wave: A0 and the second part of W0; A1 and the first part of W1; the rest of W1; the first part of the next W0 (12, 4, 8 and 0, as the
+// products need them, is 2 to 3 % slower: the longest turn decides).  The copies of a half two steps on go to its place one quarter after its
+// last read, when both groups have it; four or five halves stay in flight behind each wait.
 template <int EPI>
 __global__ __launch_bounds__(512, 2) void k_seq_gemm8(SeqGemm p) {
     constexpr int B = 256, kHalf = 128 * kRowBytes, kStep = 4 * kHalf;         // W0, W1, A0, A1
@@ -308,16 +308,16 @@ __global__ __launch_bounds__(512, 2) void k_seq_gemm8(SeqGemm p) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     const int col = lane & 15, g = lane >> 4;
-    u32x4 fw[4][2], fa0[2][2], fa1[2][2];
+    u32x4 fw0[4][2], fw1[4][2], fa0[2][2], fa1[2][2];
     const int u0 = (g ^ swz128(col)) * 16, u1 = ((4 + g) ^ swz128(col)) * 16;  // (16 rows on, the swizzle is the same)
     const char* lw = lds + (wr * 64 + col) * kRowBytes;
     const char* la = lds + A0 * kHalf + (wc * 32 + col) * kRowBytes;
-    auto read_w = [&](int k, int h) __attribute__((always_inline)) {
+    auto read_w = [&](u32x4 (&f)[4][2], int k, int h, int i0) __attribute__((always_inline)) {
         const char* b = lw + (k & 1) * kStep + h * kHalf;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            fw[i][0] = *reinterpret_cast<const u32x4*>(b + i * 16 * kRowBytes + u0);
-            fw[i][1] = *reinterpret_cast<const u32x4*>(b + i * 16 * kRowBytes + u1);
+        for (int i = i0; i < i0 + 2; ++i) {
+            f[i][0] = *reinterpret_cast<const u32x4*>(b + i * 16 * kRowBytes + u0);
+            f[i][1] = *reinterpret_cast<const u32x4*>(b + i * 16 * kRowBytes + u1);
         }
     };
     auto read_a = [&](u32x4 (&f)[2][2], int k, int h) __attribute__((always_inline)) {
@@ -334,8 +334,7 @@ __global__ __launch_bounds__(512, 2) void k_seq_gemm8(SeqGemm p) {
         __builtin_amdgcn_sched_barrier(0);
     };
     // the end of a quarter's reads, its products, and the end of its turn at the matrix cores
-    auto multiply = [&](int wh, const u32x4 (&f)[2][2], int ah) __attribute__((always_inline)) {
-        wait_vm<8>();                                    // the half that the next quarter reads has arrived
+    auto multiply = [&](int wh, const u32x4 (&w)[4][2], const u32x4 (&f)[2][2], int ah) __attribute__((always_inline)) {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         turn();
         __builtin_amdgcn_s_setprio(1);
@@ -344,7 +343,7 @@ __global__ __launch_bounds__(512, 2) void k_seq_gemm8(SeqGemm p) {
 #pragma unroll
             for (int i = 0; i < 4; ++i)
 #pragma unroll
-                for (int j = 0; j < 2; ++j) acc[wh * 4 + i][ah * 2 + j] = mma16<bf16_t>(fw[i][s], f[j][s], acc[wh * 4 + i][ah * 2 + j]);
+                for (int j = 0; j < 2; ++j) acc[wh * 4 + i][ah * 2 + j] = mma16<bf16_t>(w[i][s], f[j][s], acc[wh * 4 + i][ah * 2 + j]);
         __builtin_amdgcn_s_setprio(0);
         turn();
     };
@@ -354,22 +353,29 @@ __global__ __launch_bounds__(512, 2) void k_seq_gemm8(SeqGemm p) {
     request(W1, 0);
     request(W0, 1);
     request(A0, 1);
-    wait_vm<8>();
+    request(A1, 1);
+    wait_vm<10>();                                       // W0 and A0 of the first step
     turn();
     if (wr == 1) turn();
+    read_w(fw0, 0, 0, 0);
     for (int k = 0; k < n; ++k) {
-        read_w(k, 0);
         read_a(fa0, k, 0);
-        request(A1, k + 1);
-        multiply(0, fa0, 0);
-        read_a(fa1, k, 1);
+        read_w(fw0, k, 0, 2);
         request(W1, k + 1);
-        multiply(0, fa1, 1);
-        read_w(k, 1);
+        wait_vm<8>();                                    // (behind A1 and W1 of this step: W0, A0, A1, W1 of the next ones)
+        multiply(0, fw0, fa0, 0);
+        read_a(fa1, k, 1);
+        read_w(fw1, k, 1, 0);
         request(W0, k + 2);
-        multiply(1, fa1, 1);
+        multiply(0, fw0, fa1, 1);
+        read_w(fw1, k, 1, 2);
         request(A0, k + 2);
-        multiply(1, fa0, 0);
+        wait_vm<10>();                                   // (behind the next W0: A0, A1, W1, and W0, A0 of the step after it)
+        multiply(1, fw1, fa1, 1);
+        read_w(fw0, k + 1, 0, 0);
+        request(A1, k + 2);
+        wait_vm<10>();                                   // (behind the next A0)
+        multiply(1, fw1, fa0, 0);
     }
     if (wr == 0) turn();
     wait_vm<0>();                                        // (no copy is in flight when the workgroup's LDS goes to another)
