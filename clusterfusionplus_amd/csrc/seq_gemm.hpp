@@ -270,7 +270,7 @@ __global__ __launch_bounds__(kWave* WR* WC) void k_seq_gemm(SeqGemm p) {
 // group multiplies a quarter of its step's products, the other reads operands from LDS and requests copies.  Group 1 runs one
 // barrier behind.  The quarters of step k are (W half 0, A half 0), (W0, A1), (W1, A1), (W1, A0); their reads are spread evenly, 8, 8, 4 and 4 per
 // wave: A0 and the second part of W0; A1 and the first part of W1; the rest of W1; the first part of the next W0 (12, 4, 8 and 0, as the
-// products need them, is 2 to 3 % slower: the longest turn decides).  The copies of a half two steps on go to its place one quarter after its
+// products need them, is 2 to 4 % slower: the longest turn decides).  The copies of a half two steps on go to its place one quarter after its
 // last read, when both groups have it; four or five halves stay in flight behind each wait.
 template <int EPI>
 __global__ __launch_bounds__(512, 2) void k_seq_gemm8(SeqGemm p) {

@@ -1093,12 +1093,18 @@ void allow_lds(K kernel, size_t bytes) {
 // rows and k of 1408 to 14336 (bf16; fp32: 2 to 2000 tokens): a step of 128 bytes of k when a compute unit has one workgroup, the
 // share of a step when it has `resident` of them (the more of them, the more bytes in flight; past that they take turns), and
 // what a workgroup costs beside its steps.  The estimate below is within 10 % (root mean square) of the times measured, and what
-// it chooses is 2 % slower than the best choice on average, 20 % at worst.  (Two more tiles, 128 x 96 and 128 x 160, were within
-// 0.2 % of the others on average and are left out.)
+// it chooses is 2 % slower than the best choice on average, 20 % at worst.
+// The tiles from the ninth on are for 50 to 700 tokens, where a product is still a stream of weights, which tiles of few tokens read
+// two or three times: they hold the tokens in one tile or two, and their rings fill a compute unit's LDS.  22528 rows x 4096 without
+// -> with them: 64 tokens 44 -> 41 us, 100: 60 -> 42, 150: 63 -> 48, 300: 86 -> 67; over nine products of 2048 to 28672 rows and 37 to
+// 1000 tokens, the choice was 8.8 % behind the best tile measured and is 1.7 % behind it.  Eight layers of width 4096 in a model: 100
+// tokens 1460 -> 1305 us, 128: 1548 -> 1382, 256: 1865 -> 1702, 600: the same.
 struct GemmShape { int rows, tokens, resident; float step, share, fixed; };
 constexpr GemmShape kShapes16[] = {{64, 16, 2, 0.213f, 0.180f, 1.7f}, {64, 32, 2, 0.228f, 0.204f, 1.9f}, {64, 64, 2, 0.269f, 0.241f, 2.4f},
                                    {64, 96, 2, 0.304f, 0.282f, 2.9f}, {256, 96, 1, 0.804f, 0.804f, 5.5f}, {128, 128, 2, 0.618f, 0.618f, 5.3f},
-                                   {256, 128, 1, 0.919f, 0.919f, 6.9f}, {256, 256, 1, 1.098f, 1.098f, 13.9f}};
+                                   {256, 128, 1, 0.919f, 0.919f, 6.9f}, {256, 256, 1, 1.098f, 1.098f, 13.9f},
+                                   {128, 64, 2, 0.414f, 0.396f, 3.0f}, {96, 128, 1, 0.496f, 0.496f, 4.1f}, {128, 128, 1, 0.549f, 0.549f, 4.6f},
+                                   {128, 192, 1, 0.693f, 0.693f, 5.7f}, {192, 160, 1, 0.807f, 0.807f, 6.4f}, {96, 160, 1, 0.557f, 0.557f, 4.7f}};
 constexpr GemmShape kShapes32[] = {{64, 16, 2, 0.285f, 0.215f, 1.7f}, {64, 32, 2, 0.393f, 0.320f, 2.0f}, {64, 64, 3, 0.614f, 0.520f, 2.7f},
                                    {128, 128, 2, 1.865f, 1.957f, 5.9f}};
 struct GemmPlan { int shape, splits; };
@@ -1156,8 +1162,14 @@ void launch_shape(const SeqGemm& g, int shape, int tiles_t, hipStream_t st) {
             case 4: return launch_gemm<T, 256, 96, 8, 1, 3, EPI>(g, tiles_t, st);
             case 5: return launch_gemm<T, 128, 128, 2, 2, 2, EPI>(g, tiles_t, st);
             case 6: return launch_gemm<T, 256, 128, 4, 2, 3, EPI>(g, tiles_t, st);
+            case 8: return launch_gemm<T, 128, 64, 4, 2, 3, EPI>(g, tiles_t, st);
+            case 9: return launch_gemm<T, 96, 128, 2, 2, 5, EPI>(g, tiles_t, st);
+            case 10: return launch_gemm<T, 128, 128, 4, 2, 4, EPI>(g, tiles_t, st);
+            case 11: return launch_gemm<T, 128, 192, 4, 2, 3, EPI>(g, tiles_t, st);
+            case 12: return launch_gemm<T, 192, 160, 4, 2, 3, EPI>(g, tiles_t, st);
+            case 13: return launch_gemm<T, 96, 160, 2, 2, 4, EPI>(g, tiles_t, st);
         }
-        constexpr size_t lds = 2 * 512 * kRowBytes;
+        constexpr size_t lds = 2 * 512 * kRowBytes;     // 7
         allow_lds(k_seq_gemm8<EPI>, lds);
         hipLaunchKernelGGL(k_seq_gemm8<EPI>, dim3(ceil_div(g.n, 256) * tiles_t * g.splits), dim3(512), lds, st, g);
     } else {

@@ -19,12 +19,20 @@ DENSE = [(2, 300, 2001, 333),        # 64 x 16
          (33, 60, 20003, 51),        # 64 x 64, one step of k
          (64, 130, 20001, 51),
          (65, 60, 20001, 51),        # 64 x 96
-         (97, 130, 29999, 777),      # 128 x 128 (fp32 too)
+         (65, 60, 33001, 51),        # 256 x 96
+         (97, 130, 29999, 777),      # 128 x 64
+         (97, 260, 17001, 17001),    # 96 x 128, in the head as well
+         (97, 60, 33001, 51),        # 128 x 128, two per compute unit (fp32 too)
+         (97, 390, 25001, 51),       # 128 x 128, one
+         (129, 60, 22001, 22001),    # 96 x 160, in the head as well
+         (129, 60, 33001, 51),       # 192 x 160
+         (129, 130, 25001, 25001),   # 128 x 192, in the head as well
+         (193, 390, 25001, 51),      # 256 x 128
          (257, 60, 20000, 51),
-         (129, 520, 29999, 51),      # 256 x 128
-         (700, 300, 4001, 51),       # ... in the down rows, split
+         (129, 520, 29999, 51),
+         (700, 300, 4001, 51),       # 64 x 96 in the down rows, split
          (257, 520, 29999, 51),      # 256 x 256
-         (513, 130, 20001, 20001)]   # ... with one token and one row in the last tiles, in the head as well
+         (513, 130, 20001, 20001)]   # one token and one row in the last tiles
 
 
 @functools.lru_cache(maxsize=1)
