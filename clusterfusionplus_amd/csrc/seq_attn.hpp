@@ -66,8 +66,8 @@ template <typename T, int NK, int NT> struct AttnTile {
 // What bounds it: the matrix cores and the softmax's vector instructions, which take turns inside a wave and overlap with the other
 // wave of the SIMD.  So two workgroups per compute unit, one barrier per tile, and nothing is waited for but the tile itself: with
 // copies that the compiler knows of it waited for the next tile's before this tile's first read of LDS, and values took a detour
-// through registers to be transposed.  8000 tokens, 32 heads of 192 and 128: 1722 -> 1050 us; 2048 tokens, 128 and 128: 135 -> 98 us.
-// 37 tokens at 1990, 32 / 8 heads: 82 -> 12 us and 8 for the merge (24 workgroups became 360).
+// through registers to be transposed.  8000 tokens, 32 heads of 192 and 128: 1753 -> 1237 us; 2048 tokens, 128 and 128: 141 -> 103 us.
+// 37 tokens at 1990, 32 / 8 heads: 85 -> 12 us and 5 for the merge (24 workgroups became 384).
 // (NK: elements of a key row in LDS, NT: value columns.  The products run over all of them, without branches between the reads
 // of LDS: past the end of the query there are zeros, and of the columns past the end of a value nothing is stored.
 // SH: keys have a shared part)
