@@ -90,25 +90,31 @@ __device__ __forceinline__ void copy_to_lds16(const void* g, void* lds) {
 // waits until at most N of the wave's vector memory operations are still on their way
 template <int N> __device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
-// an address that is the same in all lanes, in scalar registers
+// An address that is the same in all lanes, in scalar registers that a scalar instruction has written.  The copies below may read such a
+// register at once; one that a vector instruction has written (a readfirstlane) they may read five wait states later only, which the
+// compiler does not see to, since it does not look into them.
 __device__ __forceinline__ const char* uniform(const char* p) {
     const uint64_t v = (uint64_t)(uintptr_t)p;
     const uint32_t lo = __builtin_amdgcn_readfirstlane((int)(uint32_t)v), hi = __builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
-    return (const char*)(uintptr_t)((uint64_t)hi << 32 | lo);
+    uint64_t r;
+    asm("s_mov_b64 %0, %1" : "=s"(r) : "s"((uint64_t)hi << 32 | lo));
+    return (const char*)(uintptr_t)r;
 }
 
-// 64 units of 16 bytes from `base` (wave-uniform) + the lanes' offsets, or from the lanes' addresses, to LDS from byte `lds`
-// (wave-uniform) on.  Written out: the compiler does not know of the copy, so that it puts no waits of its own for it; who reads the
-// tile waits with wait_vm or pipe_barrier.
+// 64 units of 16 bytes from `base` + the lanes' offsets, or from the lanes' addresses, to LDS from byte `lds` (wave-uniform) on.  `base`
+// comes from uniform(), or from such a base by scalar additions.  Written out: the compiler does not know of the copy, so that it puts no
+// waits of its own for it; who reads the tile waits with wait_vm or pipe_barrier.  The place goes to m0, which the compiler writes and
+// keeps account of; the wait state between that and the copy is in here.  (With all five wait states in here, whatever writes the
+// base, 700 tokens of a model with 64 experts take 1.8 % longer, 4412 -> 4492 us, and 37 of a dense one 0.7 %, 3574 -> 3599 us.)
 __device__ __forceinline__ void copy_to_lds16_at(uint32_t off, const void* base, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory");
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "{m0}"(lds) : "memory");
 }
 // ... of bytes that nobody reads again: they leave the caches to the others'
 __device__ __forceinline__ void copy_to_lds16_once(uint32_t off, const void* base, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(off), "s"(base), "s"(lds) : "memory");
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(off), "s"(base), "{m0}"(lds) : "memory");
 }
 __device__ __forceinline__ void copy_to_lds16_from(const void* p, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(p), "s"(lds) : "memory");
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(p), "{m0}"(lds) : "memory");
 }
 __device__ __forceinline__ uint32_t lds_address(const void* p) { return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)p; }
 // waits for all but the wave's N newest copies and for its reads of LDS, then for the other waves

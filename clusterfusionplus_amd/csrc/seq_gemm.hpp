@@ -200,8 +200,8 @@ __global__ __launch_bounds__(kWave* WR* WC) void k_seq_gemm(SeqGemm p) {
     GemmTile t;
     if (!gemm_tile<BW, BT>(p, t)) return;
     const int nk = p.kbytes / kRowBytes, kb = mul_div(nk, t.split, p.splits), n = mul_div(nk, t.split + 1, p.splits) - kb;
-    const char* bw = t.w + (size_t)t.tw * BW * p.kbytes + (size_t)kb * kRowBytes;
-    const char* ba = p.a + (p.tile_off != nullptr ? (size_t)0 : (size_t)t.tt * BT * p.lda) + (size_t)kb * kRowBytes;
+    const char* bw = uniform(t.w + (size_t)t.tw * BW * p.kbytes + (size_t)kb * kRowBytes);
+    const char* ba = uniform(p.a + (p.tile_off != nullptr ? (size_t)0 : (size_t)t.tt * BT * p.lda) + (size_t)kb * kRowBytes);
     uint32_t vw[WI], va[AI];
 #pragma unroll
     for (int i = 0; i < WI; ++i) {
@@ -281,8 +281,8 @@ __global__ __launch_bounds__(512, 2) void k_seq_gemm8(SeqGemm p) {
     GemmTile t;
     if (!gemm_tile<B, B>(p, t)) return;
     const int nk = p.kbytes / kRowBytes, kb = mul_div(nk, t.split, p.splits), n = mul_div(nk, t.split + 1, p.splits) - kb;
-    const char* bw = t.w + (size_t)t.tw * B * p.kbytes + (size_t)kb * kRowBytes;
-    const char* ba = p.a + (p.tile_off != nullptr ? (size_t)0 : (size_t)t.tt * B * p.lda) + (size_t)kb * kRowBytes;
+    const char* bw = uniform(t.w + (size_t)t.tw * B * p.kbytes + (size_t)kb * kRowBytes);
+    const char* ba = uniform(p.a + (p.tile_off != nullptr ? (size_t)0 : (size_t)t.tt * B * p.lda) + (size_t)kb * kRowBytes);
     // half h of W: rows wr * 128 + h * 64 + 0 .. 63 of both groups; half h of A: tokens wc * 64 + h * 32 + 0 .. 31 of the four columns
     uint32_t vw[2][2], va[2][2];
 #pragma unroll
