@@ -84,8 +84,8 @@ __global__ __launch_bounds__(kSeqThreads, (NT <= 128 ? 2 : 1)) void k_seq_attn(S
     if (((bx >> 3) & 1) && (bx | 7) < gx) bx ^= 7;
     const int c0 = (gx - 1 - bx) * 64 * CT;
 
-    // (its sign goes to the query; not zero, so that it keeps the scores of keys that are not seen at -infinity)
-    const float scale = fmaxf(fabsf(a.scale_log2), 1e-30f);
+    // (its sign goes to the query; not zero, so that it keeps the scores of keys that are not seen at -infinity; NaN stays NaN)
+    const float size = fabsf(a.scale_log2), scale = size < 1e-30f ? 1e-30f : size;
     int pq[CT], first[CT], tok[CT], head[CT];
     u32x4 qf[CT][KS];
     float m[CT], l[CT];                                  // running maximum (log2 domain), this lane's share of the denominator

@@ -41,6 +41,18 @@ def test_portions_far_into_a_sequence(name, dtype):
     assert pos == 1300
 
 
+# a scale that is no number: no logit is one, in one split of the keys and in several
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("kind", [grouped, latent])
+def test_scale_that_is_no_number(kind, dtype):
+    from clusterfusionplus_amd import kagapel, nibotar
+    M, cfg = kind(scale=float("nan"))
+    toks = M.prompt(cfg, 600, 6)
+    m = (nibotar if M is N else kagapel).from_tensors(cfg, M.weights(cfg, 5), dtype, capacity=600)
+    for pos, n in ((0, 30), (30, 560), (590, 5)):
+        assert m.forward(0, toks[pos:pos + n], pos, range(n)).isnan().all(), (pos, n)
+
+
 # projections of up to 8192 and 16384 values, and of more; heads that are no whole groups of four; values mixed; padded heads
 PROJECTIONS = {"12k": [N.attn(64, 16, 128, 128)], "17k": [N.attn(128, 4, 128, 128)], "mixed_12k": [N.attn(48, 12, 100, 132, v_mix=True, chunk=31), N.attn(48, 12, 100, 132, v_mix=True)],
                "no_fours": [N.attn(6, 2, 42, 30, v_mix=True), N.attn(6, 2, 40, 30, v_mix=True), N.attn(10, 5, 42, 12, v_mix=True)]}
