@@ -36,6 +36,7 @@
 #include "seq_device.hpp"
 #include "seq_gemm.hpp"
 #include "seq_latent.hpp"
+#include "seq_plan.hpp"
 
 using namespace cfpp;
 
@@ -1013,8 +1014,6 @@ __global__ void k_seq_rope_table(float2* t, const double* freq, double mul, int 
 // ================================================================================================
 // host side
 // ================================================================================================
-int up_to(int a, int b) { return (a + b - 1) / b * b; }
-int ceil_div(int a, int b) { return (a + b - 1) / b; }
 size_t pitch_of(int K, int esize) { return (size_t)up_to(K * esize, kRowBytes); }
 
 struct LayerPlan {
@@ -1234,17 +1233,12 @@ void expert_gemm(const cfpp_seq* s, const LayerPlan& L, SeqGemm g, int n, hipStr
     launch_shape<T, EPI>(g, plan.shape, slots / plan.tokens + std::min(L.d.experts, slots), st);
 }
 
-// Columns of a workgroup and splits of the keys.  bf16: two column tiles per wave share the reads of keys and values; one, where that
-// leaves fewer columns empty or where two workgroups per compute unit are not reached.  Splits fill the chip: two workgroups per
-// compute unit, each with two tiles at least.
 template <typename T, int NK, int NT>
 void launch_attn(SeqAttn a, int G, int cus, size_t room, float* part, hipStream_t st) {
     using L = AttnTile<T, NK, NT>;
-    const int cols = a.T * a.R, tiles = ceil_div(std::min(a.pos0 + a.T, a.chunk > 0 ? a.chunk : a.pos0 + a.T), L::keys);
-    const bool two = sizeof(T) == 2 && ceil_div(cols, 128) * G >= 2 * cus;       // (fp32: two column tiles do not fit the registers)
-    const int wgs = ceil_div(cols, two ? 128 : 64) * G, per_cu = NT <= 128 ? 2 : 1;
-    const size_t floats = (size_t)a.T * a.H * (a.vtiles * 16 + 2);
-    a.splits = std::max(1, (int)std::min<size_t>({(size_t)16, (size_t)(per_cu * cus / wgs), (size_t)(tiles / 2), room / floats}));
+    const int cols = a.T * a.R;
+    const AttnPlan plan = plan_attn({a.T, a.R, G, a.pos0, a.chunk, L::keys, sizeof(T) == 2, NT <= 128 ? 2 : 1, (size_t)a.T * a.H * (a.vtiles * 16 + 2)}, cus, room);
+    a.splits = plan.splits;
     a.part = part;
     a.ml = part + (size_t)a.splits * a.T * a.H * a.vtiles * 16;
     const size_t lds = 2 * L::size;
@@ -1256,7 +1250,7 @@ void launch_attn(SeqAttn a, int G, int cus, size_t room, float* part, hipStream_
     };
     auto pick = [&](auto sh) {
         if constexpr (sizeof(T) == 2) {
-            if (two) return go(std::integral_constant<int, 2>{}, sh);
+            if (plan.two) return go(std::integral_constant<int, 2>{}, sh);   // (fp32: two column tiles do not fit the registers)
         }
         go(std::integral_constant<int, 1>{}, sh);
     };

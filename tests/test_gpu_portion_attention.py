@@ -41,6 +41,21 @@ def test_portions_far_into_a_sequence(name, dtype):
     assert pos == 1300
 
 
+# short portions that begin with a chunk, just behind its edge and just before it: they see a tile or two, far into the sequence
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+def test_short_portions_at_the_edge_of_a_chunk(dtype):
+    from clusterfusionplus_amd import nibotar
+    cfg = grouped(chunk=400)[1]
+    w, toks = N.weights(cfg, 5), N.prompt(cfg, 1300, 6)
+    want = N.oracle(cfg, w, toks)
+    m = nibotar.from_tensors(cfg, w, dtype, capacity=1300)
+    pos = 0
+    for n in (400, 37, 63, 300, 2, 5, 130, 263, 3, 37, 60):
+        assert N.error(m.forward(0, toks[pos:pos + n], pos, range(n)), want[pos:pos + n]) < LIMIT[dtype], (pos, n)
+        pos += n
+    assert pos == 1300
+
+
 # a scale that is no number: no logit is one, in one split of the keys and in several
 @pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
 @pytest.mark.parametrize("kind", [grouped, latent])
