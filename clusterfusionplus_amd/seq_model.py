@@ -92,7 +92,9 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 
 def vector(v: torch.Tensor, device) -> torch.Tensor:
-    return v.detach().to(device=device, dtype=torch.float32).contiguous()
+    """fp32 on the device, contiguous and 16-byte aligned (a view into a larger tensor may begin anywhere)."""
+    v = v.detach().to(device=device, dtype=torch.float32).contiguous()
+    return v if v.data_ptr() % 16 == 0 else v.clone()
 
 
 @dataclass

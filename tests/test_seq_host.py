@@ -54,6 +54,19 @@ def test_packed_weights():
     assert f.layers[1].w_down.shape == (70, 64) and f.embed.shape == (41, 96)
 
 
+@pytest.mark.parametrize("module, cfg, models", [(nibotar, M.CASES["everything"], M), (kagapel, KM.CASES["everything"], KM)], ids=["nibotar", "kagapel"])
+def test_packed_tensors_are_aligned(module, cfg, models):
+    """What the kernels read in units of 16 bytes begins at one, also where the checkpoint's tensors are views into a larger one."""
+    w = {}
+    for name, t in models.weights(cfg).items():
+        buf = torch.empty(t.numel() + 1, dtype=t.dtype if t.dtype == torch.int32 else torch.float32)
+        buf[1:] = t.flatten()
+        w[name] = buf[1:].view(t.shape)
+    p = module.pack_weights(module.parse_config(cfg), w, torch.float32, "cpu")
+    tensors = [(f"{l}.{k}", v) for l, layer in enumerate(p.layers) for k, v in vars(layer).items() if k != "table"] + list(vars(p).items())
+    assert not [n for n, v in tensors if isinstance(v, torch.Tensor) and v.data_ptr() % 16]
+
+
 def test_missing_and_misshapen_tensors_are_named():
     cfg = M.CASES["everything"]
     for name, t in (("l1.mix.k.norm", None), ("l0.mlp.e3.down", torch.zeros(2, 2)), ("l3.mlp.table", M.weights(cfg)["l3.mlp.table"] + 9)):
