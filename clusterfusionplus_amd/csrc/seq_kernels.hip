@@ -23,7 +23,6 @@
 #include <string.h>
 
 #include <algorithm>
-#include <iterator>
 #include <map>
 #include <new>
 #include <tuple>
@@ -1088,60 +1087,6 @@ void allow_lds(K kernel, size_t bytes) {
 }
 
 // ---- portions ----------------------------------------------------------------------------------
-// The tiles of the matrix products and what they cost, in us, as measured on an MI355X over 2 to 4000 tokens, 1500 to 50432
-// rows and k of 1408 to 14336 (bf16; fp32: 2 to 2000 tokens): a step of 128 bytes of k when a compute unit has one workgroup, the
-// share of a step when it has `resident` of them (the more of them, the more bytes in flight; past that they take turns), and
-// what a workgroup costs beside its steps.  The estimate below is within 10 % (root mean square) of the times measured, and what
-// it chooses is 2 % slower than the best choice on average, 20 % at worst.
-// The tiles from the ninth on are for 50 to 700 tokens, where a product is still a stream of weights, which tiles of few tokens read
-// two or three times: they hold the tokens in one tile or two, and their rings fill a compute unit's LDS.  22528 rows x 4096 without
-// -> with them: 64 tokens 44 -> 41 us, 100: 60 -> 42, 150: 63 -> 48, 300: 86 -> 67; over nine products of 2048 to 28672 rows and 37 to
-// 1000 tokens, the choice was 8.8 % behind the best tile measured and is 1.7 % behind it.  Eight layers of width 4096 in a model: 100
-// tokens 1460 -> 1305 us, 128: 1548 -> 1382, 256: 1865 -> 1702, 600: the same.
-struct GemmShape { int rows, tokens, resident; float step, share, fixed; };
-constexpr GemmShape kShapes16[] = {{64, 16, 2, 0.213f, 0.180f, 1.7f}, {64, 32, 2, 0.228f, 0.204f, 1.9f}, {64, 64, 2, 0.269f, 0.241f, 2.4f},
-                                   {64, 96, 2, 0.304f, 0.282f, 2.9f}, {256, 96, 1, 0.804f, 0.804f, 5.5f}, {128, 128, 2, 0.618f, 0.618f, 5.3f},
-                                   {256, 128, 1, 0.919f, 0.919f, 6.9f}, {256, 256, 1, 1.098f, 1.098f, 13.9f},
-                                   {128, 64, 2, 0.414f, 0.396f, 3.0f}, {96, 128, 1, 0.496f, 0.496f, 4.1f}, {128, 128, 1, 0.549f, 0.549f, 4.6f},
-                                   {128, 192, 1, 0.693f, 0.693f, 5.7f}, {192, 160, 1, 0.807f, 0.807f, 6.4f}, {96, 160, 1, 0.557f, 0.557f, 4.7f}};
-constexpr GemmShape kShapes32[] = {{64, 16, 2, 0.285f, 0.215f, 1.7f}, {64, 32, 2, 0.393f, 0.320f, 2.0f}, {64, 64, 3, 0.614f, 0.520f, 2.7f},
-                                   {128, 128, 2, 1.865f, 1.957f, 5.9f}};
-struct GemmPlan { int shape, splits; };
-
-// `tiles` tiles of `steps` steps on `cus` compute units
-float gemm_tiles_cost(const GemmShape& c, double tiles, float steps, int cus) {
-    const int load = (int)ceil(tiles / cus), full = load / c.resident, rest = load % c.resident;
-    float t = full * (steps * std::max(c.step, c.resident * c.share) + c.fixed);
-    if (rest > 0) t += steps * std::max(c.step, rest * c.share) + c.fixed;
-    return t;
-}
-// what a stream of so many bytes takes at 5.8 TB/s
-float stream_cost(double bytes) { return (float)(bytes / 5.8e6); }
-
-// The cheapest tile, and with `room` floats for partial results the cheapest number of splits of k as well.  Reading a partial
-// result costs its bytes at 5 TB/s, and 0.3 us.  No split has fewer than three steps.
-template <typename T>
-GemmPlan plan_gemm(const cfpp_seq* s, const SeqGemm& g, size_t room) {
-    const GemmShape* shapes = sizeof(T) == 2 ? kShapes16 : kShapes32;
-    const int count = sizeof(T) == 2 ? (int)std::size(kShapes16) : (int)std::size(kShapes32);
-    static const int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16};
-    const int nk = g.kbytes / kRowBytes;
-    GemmPlan best{0, 1};
-    float least = INFINITY;
-    for (int i = 0; i < count; ++i)
-        for (int sp : kSplits) {
-            if (sp > 1 && (room == 0 || nk / sp < 3 || (size_t)sp * g.m * g.ldy > room)) break;
-            const double tiles = (double)ceil_div(g.n, shapes[i].rows) * ceil_div(g.m, shapes[i].tokens) * sp;
-            float t = std::max(gemm_tiles_cost(shapes[i], tiles, (float)nk / sp, s->cus), stream_cost((double)g.n * g.kbytes));
-            if (sp > 1) t += 0.3f + 4e-6f * sp * g.m * g.n / 5.0f;
-            if (t < least) {
-                least = t;
-                best = {i, sp};
-            }
-        }
-    return best;
-}
-
 template <typename T, int BW, int BT, int WR, int WC, int NB, int EPI>
 void launch_gemm(const SeqGemm& g, int tiles_t, hipStream_t st) {
     const size_t lds = (size_t)NB * (BW + BT) * kRowBytes;
@@ -1184,44 +1129,24 @@ void launch_shape(const SeqGemm& g, int shape, int tiles_t, hipStream_t st) {
 // `room`: floats behind g.yf for partial results; the number of those that the product leaves there
 template <typename T, int EPI>
 int gemm(const cfpp_seq* s, SeqGemm g, hipStream_t st, size_t room = 0) {
-    const GemmPlan plan = plan_gemm<T>(s, g, EPI == kEpiF32 ? room : 0);
+    const GemmPlan plan = plan_gemm({g.n, g.m, g.kbytes, g.ldy, EPI == kEpiF32 ? room : 0}, sizeof(T) == 2, s->cus);
     g.splits = plan.splits;
     g.split_stride = (size_t)g.m * g.ldy;
-    const int tiles_t = ceil_div(g.m, (sizeof(T) == 2 ? kShapes16 : kShapes32)[plan.shape].tokens);
+    const int tiles_t = ceil_div(g.m, shapes_of(sizeof(T) == 2)[plan.shape].tokens);
     g.once = tiles_t == 1;
     launch_shape<T, EPI>(g, plan.shape, tiles_t, st);
     return plan.splits;
 }
 
-// Tile of the expert products of a portion of n tokens (both use it).  An expert has avg +- sqrt(avg) of them; where that fits a
-// tile, it has one (`once`), and the product is a stream of weights.  A stream hides the tiles' own time only in part: with 66 tokens
-// per expert, 64 experts of 2816 x 2048 take 159 us in tiles of 64 x 96, estimated at 118, and 151 us in tiles of 256 x 96, at 94.
-struct ExpertPlan { int shape, tokens, once; };
+template <typename T>
 ExpertPlan expert_plan(const cfpp_seq* s, const LayerPlan& L, int n) {
-    const GemmShape* shapes = s->esize == 2 ? kShapes16 : kShapes32;
-    const int count = s->esize == 2 ? (int)std::size(kShapes16) : (int)std::size(kShapes32);
-    const double avg = (double)n * L.d.top / L.d.experts, live = L.d.experts * std::min(1.0, avg);
-    const float stream = stream_cost(live * 2.0 * L.d.ff * s->xpitch);
-    ExpertPlan best{};
-    float least = INFINITY;
-    for (int i = 0; i < count; ++i) {
-        const GemmShape& c = shapes[i];
-        const bool one = avg + 1.5 * sqrt(avg) <= c.tokens;
-        const double per = one ? 1.0 : std::max(1.0, avg / c.tokens + 0.5);
-        const float t = gemm_tiles_cost(c, live * per * ceil_div(2 * L.d.ff, c.rows), (float)s->xpitch / kRowBytes, s->cus);
-        const float cost = std::max(t, stream) + 0.3f * std::min(t, stream);
-        if (cost < least) {
-            least = cost;
-            best = {i, c.tokens, one};
-        }
-    }
-    return best;
+    return plan_experts({n, L.d.top, L.d.experts, L.d.ff, s->xpitch}, sizeof(T) == 2, s->cus);
 }
 
 template <typename T, int EPI>
 void expert_gemm(const cfpp_seq* s, const LayerPlan& L, SeqGemm g, int n, hipStream_t st) {
     const SeqRoute& r = s->host_routes[L.route];
-    const ExpertPlan plan = expert_plan(s, L, n);
+    const ExpertPlan plan = expert_plan<T>(s, L, n);
     const int slots = n * L.d.top;
     g.m = slots;
     g.tile_off = r.tile_off;
@@ -1450,12 +1375,12 @@ int run_portion(cfpp_seq* s, int slot, int n, int pos, int n_want, float* logits
             for (; j < s->layers.size(); ++j) {
                 const LayerPlan& M = s->layers[j];
                 if (M.route < 0) continue;
-                if (expert_plan(s, M, n).tokens != expert_plan(s, L, n).tokens) break;
+                if (expert_plan<T>(s, M, n).tokens != expert_plan<T>(s, L, n).tokens) break;
                 ++count;
             }
             const size_t lds = (size_t)s->max_experts * 8;
             allow_lds(k_seq_route, lds);
-            hipLaunchKernelGGL(k_seq_route, dim3((unsigned)count), dim3(1024), lds, st, s->routes + L.route, s->tokens, n, expert_plan(s, L, n).tokens);
+            hipLaunchKernelGGL(k_seq_route, dim3((unsigned)count), dim3(1024), lds, st, s->routes + L.route, s->tokens, n, expert_plan<T>(s, L, n).tokens);
             i = j - 1;
         }
     }

@@ -1,6 +1,7 @@
 // What the kernels of a portion of the sequence models are launched with, from sizes alone.  Plain C++ without the device's headers, so
 // that the choices can be looked at on the host.
 #pragma once
+#include <math.h>
 #include <stddef.h>
 
 #include <algorithm>
@@ -9,6 +10,100 @@ namespace cfpp {
 
 inline int up_to(int a, int b) { return (a + b - 1) / b * b; }
 inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
+
+// The tiles of the matrix products and what they cost, in us, as measured on an MI355X over 2 to 4000 tokens, 1500 to 50432
+// rows and k of 1408 to 14336 (bf16; fp32: 2 to 2000 tokens): a step of 128 bytes of k when a compute unit has one workgroup, the
+// share of a step when it has `resident` of them (the more of them, the more bytes in flight; past that they take turns), and
+// what a workgroup costs beside its steps.  The estimate below is within 10 % (root mean square) of the times measured, and what
+// it chooses is 2 % slower than the best choice on average, 20 % at worst.
+// The tiles from the ninth on are for 50 to 700 tokens, where a product is still a stream of weights, which tiles of few tokens read
+// two or three times: they hold the tokens in one tile or two, and their rings fill a compute unit's LDS.  22528 rows x 4096 without
+// -> with them: 64 tokens 44 -> 41 us, 100: 60 -> 42, 150: 63 -> 48, 300: 86 -> 67; over nine products of 2048 to 28672 rows and 37 to
+// 1000 tokens, the choice was 8.8 % behind the best tile measured and is 1.7 % behind it.  Eight layers of width 4096 in a model: 100
+// tokens 1460 -> 1305 us, 128: 1548 -> 1382, 256: 1865 -> 1702, 600: the same.
+struct GemmShape { int rows, tokens, resident; float step, share, fixed; };
+constexpr GemmShape kShapes16[] = {{64, 16, 2, 0.213f, 0.180f, 1.7f}, {64, 32, 2, 0.228f, 0.204f, 1.9f}, {64, 64, 2, 0.269f, 0.241f, 2.4f},
+                                   {64, 96, 2, 0.304f, 0.282f, 2.9f}, {256, 96, 1, 0.804f, 0.804f, 5.5f}, {128, 128, 2, 0.618f, 0.618f, 5.3f},
+                                   {256, 128, 1, 0.919f, 0.919f, 6.9f}, {256, 256, 1, 1.098f, 1.098f, 13.9f},
+                                   {128, 64, 2, 0.414f, 0.396f, 3.0f}, {96, 128, 1, 0.496f, 0.496f, 4.1f}, {128, 128, 1, 0.549f, 0.549f, 4.6f},
+                                   {128, 192, 1, 0.693f, 0.693f, 5.7f}, {192, 160, 1, 0.807f, 0.807f, 6.4f}, {96, 160, 1, 0.557f, 0.557f, 4.7f}};
+constexpr GemmShape kShapes32[] = {{64, 16, 2, 0.285f, 0.215f, 1.7f}, {64, 32, 2, 0.393f, 0.320f, 2.0f}, {64, 64, 3, 0.614f, 0.520f, 2.7f},
+                                   {128, 128, 2, 1.865f, 1.957f, 5.9f}};
+struct GemmShapes {
+    const GemmShape* first;
+    int count;
+    const GemmShape& operator[](int i) const { return first[i]; }
+};
+inline GemmShapes shapes_of(bool bf16) {
+    if (bf16) return {kShapes16, (int)(sizeof(kShapes16) / sizeof(kShapes16[0]))};
+    return {kShapes32, (int)(sizeof(kShapes32) / sizeof(kShapes32[0]))};
+}
+
+// `tiles` tiles of `steps` steps on `cus` compute units
+inline float gemm_tiles_cost(const GemmShape& c, double tiles, float steps, int cus) {
+    const int load = (int)ceil(tiles / cus), full = load / c.resident, rest = load % c.resident;
+    float t = full * (steps * std::max(c.step, c.resident * c.share) + c.fixed);
+    if (rest > 0) t += steps * std::max(c.step, rest * c.share) + c.fixed;
+    return t;
+}
+// what a stream of so many bytes takes at 5.8 TB/s
+inline float stream_cost(double bytes) { return (float)(bytes / 5.8e6); }
+
+// A plain product: n rows of kbytes bytes, m tokens; `room` floats for partial results of rows of ldy floats (0: k is not split).
+struct GemmSizes {
+    int n, m, kbytes, ldy;
+    size_t room;
+    int steps() const { return kbytes / 128; }
+};
+// Its time with one tile and one number of splits.  Reading a partial result costs its bytes at 5 TB/s, and 0.3 us.
+inline float gemm_cost(const GemmSizes& g, const GemmShape& c, int splits, int cus) {
+    const double tiles = (double)ceil_div(g.n, c.rows) * ceil_div(g.m, c.tokens) * splits;
+    float t = std::max(gemm_tiles_cost(c, tiles, (float)g.steps() / splits, cus), stream_cost((double)g.n * g.kbytes));
+    if (splits > 1) t += 0.3f + 4e-6f * splits * g.m * g.n / 5.0f;
+    return t;
+}
+// The cheapest tile, and with room for partial results the cheapest number of splits of k as well.  No split has fewer than three steps.
+struct GemmPlan { int shape, splits; };
+inline GemmPlan plan_gemm(const GemmSizes& g, bool bf16, int cus) {
+    const GemmShapes shapes = shapes_of(bf16);
+    GemmPlan best{0, 1};
+    float least = INFINITY;
+    for (int i = 0; i < shapes.count; ++i)
+        for (int sp : {1, 2, 3, 4, 6, 8, 12, 16}) {
+            if (sp > 1 && (g.room == 0 || g.steps() / sp < 3 || (size_t)sp * g.m * g.ldy > g.room)) break;
+            const float t = gemm_cost(g, shapes[i], sp, cus);
+            if (t < least) {
+                least = t;
+                best = {i, sp};
+            }
+        }
+    return best;
+}
+
+// Tile of the expert products of a portion of n tokens (both use it).  An expert has avg +- sqrt(avg) of them; where that fits a
+// tile, it has one (`once`), and the product is a stream of weights.  A stream hides the tiles' own time only in part: with 66 tokens
+// per expert, 64 experts of 2816 x 2048 take 159 us in tiles of 64 x 96, estimated at 118, and 151 us in tiles of 256 x 96, at 94.
+struct ExpertSizes { int n, top, experts, ff, xbytes; };     // tokens, experts of a token, experts, their inner size, bytes of an input row
+struct ExpertPlan { int shape, tokens, once; };
+inline ExpertPlan plan_experts(const ExpertSizes& e, bool bf16, int cus) {
+    const GemmShapes shapes = shapes_of(bf16);
+    const double avg = (double)e.n * e.top / e.experts, live = e.experts * std::min(1.0, avg);
+    const float stream = stream_cost(live * 2.0 * e.ff * e.xbytes);
+    ExpertPlan best{};
+    float least = INFINITY;
+    for (int i = 0; i < shapes.count; ++i) {
+        const GemmShape& c = shapes[i];
+        const bool one = avg + 1.5 * sqrt(avg) <= c.tokens;
+        const double per = one ? 1.0 : std::max(1.0, avg / c.tokens + 0.5);
+        const float t = gemm_tiles_cost(c, live * per * ceil_div(2 * e.ff, c.rows), (float)e.xbytes / 128, cus);
+        const float cost = std::max(t, stream) + 0.3f * std::min(t, stream);
+        if (cost < least) {
+            least = cost;
+            best = {i, c.tokens, one};
+        }
+    }
+    return best;
+}
 
 // Attention of a portion of T tokens at positions pos0 and on: R query heads for each of G key / value heads, `keys` of them in a tile.
 struct AttnSizes {

@@ -1,41 +1,19 @@
 """The choices that a portion's kernels are launched with (csrc/seq_plan.hpp), on the host."""
-import ctypes
-import os
 import random
-import subprocess
 
 import pytest
 
-from clusterfusionplus_amd import build
+from tests import seq_plan as P
+from tests import test_gpu_products as G
 
-CUS, PER_CU, ROOM = 256, 2, 1 << 24
-SOURCE = """
-#include "seq_plan.hpp"
-using namespace cfpp;
-extern "C" int attn_splits(int T, int R, int G, int pos0, int chunk, int keys, int bf16, int per_cu, long floats, int cus, long room, int* columns) {
-    const AttnPlan p = plan_attn({T, R, G, pos0, chunk, keys, bf16 != 0, per_cu, (size_t)floats}, cus, (size_t)room);
-    *columns = p.two ? 128 : 64;
-    return p.splits;
-}
-"""
+ROOM = 1 << 24
 
 
-@pytest.fixture(scope="module")
-def plan(tmp_path_factory):
-    d = tmp_path_factory.mktemp("plan")
-    (d / "plan.cpp").write_text(SOURCE)
-    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", f"-I{build.CSRC}", str(d / "plan.cpp"), "-o", str(d / "plan.so")], check=True)
-    lib = ctypes.CDLL(str(d / "plan.so"))
-    lib.attn_splits.argtypes = [ctypes.c_int] * 8 + [ctypes.c_long, ctypes.c_int, ctypes.c_long, ctypes.POINTER(ctypes.c_int)]
-    return lib
-
-
-def splits(plan, T, R, G, pos, chunk, keys=64, room=ROOM, vdim=128):
-    columns = ctypes.c_int()
+def splits(T, R, G, pos, chunk, keys=64, room=ROOM, vdim=128):
     floats = T * R * G * (vdim + 2)
-    n = plan.attn_splits(T, R, G, pos, chunk, keys, keys == 64, PER_CU, floats, CUS, room, ctypes.byref(columns))
+    n, columns = P.attention(T, R, G, pos, chunk, keys, floats, room)
     assert 1 <= n <= 16 and (n == 1 or n * floats <= room)
-    return n, columns.value
+    return n, columns
 
 
 def walks(T, R, pos, chunk, keys, columns):
@@ -49,16 +27,89 @@ def walks(T, R, pos, chunk, keys, columns):
 
 @pytest.mark.parametrize("pos, chunk, want", [(8192, 8192, 1), (8193, 8192, 1), (8192 + 219, 8192, 2), (1990, 8192, 16), (8192 + 1990, 8192, 16), (8150, 8192, 16),
                                               (8170, 8192, 16), (0, 0, 1), (1990, 0, 16), (100, 40, 1), (1000, 300, 1)])
-def test_splits_follow_what_a_short_portion_sees(plan, pos, chunk, want):
+def test_splits_follow_what_a_short_portion_sees(pos, chunk, want):
     """37 tokens, four query heads to each of eight key heads: a chunk's first tokens see that chunk only."""
-    assert splits(plan, 37, 4, 8, pos, chunk)[0] == want
+    assert splits(37, 4, 8, pos, chunk)[0] == want
 
 
-def test_every_split_of_the_longest_walk_has_two_tiles(plan):
+def test_every_split_of_the_longest_walk_has_two_tiles():
     rng = random.Random(3)
     for _ in range(3000):
         T, R, G = rng.choice([2, 5, 37, 64, 65, 150, 301, 700]), rng.choice([1, 2, 4, 8]), rng.choice([1, 2, 8, 16, 32])
         chunk, keys = rng.choice([0, 1, 7, 100, 1000, 8192]), rng.choice([32, 64])
         pos = rng.randrange(0, 20000)
-        n, columns = splits(plan, T, R, G, pos, chunk, keys)
+        n, columns = splits(T, R, G, pos, chunk, keys)
         assert n == 1 or n <= max(walks(T, R, pos, chunk, keys, columns)) // 2, (T, R, G, pos, chunk, keys, n)
+
+
+# ---- the tiles that the products' tests are for --------------------------------------------------------------------------
+
+@pytest.mark.parametrize("sizes, tile", list(zip(G.DENSE, G.DENSE_TILES)), ids=str)
+def test_tiles_of_up_rows(sizes, tile):
+    n, width, ff, vocab = sizes
+    if sizes == (700, 300, 4001, 51):                # (here it is the down rows)
+        assert P.product(width, n, ff, True, P.room(n, width))[:3] == tile
+    else:
+        assert P.product(ff, n, width, True) == (*tile, 1)
+        if vocab > 10000:
+            assert P.product(vocab, n, width, True) == (*tile, 1)
+
+
+@pytest.mark.parametrize("sizes, tile", G.SPLIT, ids=str)
+def test_tiles_of_split_rows(sizes, tile):
+    n, width, ff = sizes
+    assert P.product(width, n, ff, True, P.room(4 * n, width)) == tile
+    assert P.product(width, n, ff, False, P.room(4 * n, width))[3] > 1
+
+
+@pytest.mark.parametrize("sizes, tile", G.GATED, ids=str)
+def test_tiles_of_gated_rows(sizes, tile):
+    n, width, ff = sizes
+    assert P.product(2 * ff, n, width, True) == (*tile, 1)
+    down = P.product(width, n, ff, True, P.room(n, width))
+    assert down[3] > 1 and (width < 8000 or down[:2] == (256, 256))
+
+
+@pytest.mark.parametrize("sizes, tile", G.HEADS, ids=str)
+def test_tiles_of_keys_and_values(sizes, tile):
+    heads, dim, vdim, rank, n = sizes
+    assert P.product(heads * (dim + vdim), n, rank, True) == (*tile, 1)
+
+
+@pytest.mark.parametrize("sizes, tile", G.EXPERT_TILES, ids=str)
+def test_tiles_of_experts(sizes, tile):
+    assert P.experts(*sizes, True) == tile
+
+
+@pytest.mark.parametrize("sizes, tile", G.HEAD, ids=str)
+def test_tiles_of_the_head(sizes, tile):
+    n, width, vocab = sizes
+    assert P.product(vocab, n, width, True) == (*tile, 1)
+
+
+def test_every_tile_is_tested_in_every_kind_of_product():
+    tiles = {(64, 16, 2), (64, 32, 2), (64, 64, 2), (64, 96, 2), (256, 96, 1), (128, 128, 2), (256, 128, 1), (256, 256, 1), (128, 64, 2), (96, 128, 1), (128, 128, 1),
+             (128, 192, 1), (192, 160, 1), (96, 160, 1)}
+    assert {P.tile(i, True) for i in range(len(tiles))} == tiles
+    small = {(64, 16, 2)}                            # (what everything takes in the other tests' small models)
+    whole = {(128, 128, 2)}                          # (of its size, the tile that is alone on a compute unit is the one to split)
+    head = {t for s, t in zip(G.DENSE, G.DENSE_TILES) if s[3] > 10000}
+    for name, seen in (("up", set(G.DENSE_TILES)), ("split", {t[:3] for _, t in G.SPLIT} | whole), ("gated", {t for _, t in G.GATED} | small),
+                       ("keys and values", {t for _, t in G.HEADS} | small), ("experts", {t[:3] for _, t in G.EXPERT_TILES}), ("head", head | {t for _, t in G.HEAD} | small)):
+        assert seen == tiles, (name, tiles - seen)
+
+
+def test_split_rows_of_wide_models():
+    n, ff = G.ROWS
+    for width in G.WIDTHS + [w for w, _ in G.STREAMS]:
+        for bf16 in (True, False):
+            assert P.product(width, n, ff, bf16, P.room(100, width))[3] > 1, (width, bf16)
+
+
+def test_no_split_of_less_than_three_steps_or_more_than_its_room():
+    rng = random.Random(5)
+    for _ in range(3000):
+        n, m, k, bf16 = rng.randint(1, 60000), rng.choice([2, 3, 17, 65, 100, 300, 1000, 4000]), rng.randint(1, 16000), rng.random() < 0.5
+        floats = rng.choice([0, m * n, 4 * m * n, 16 << 20])
+        rows, tokens, resident, sp = P.product(n, m, k, bf16, floats)
+        assert sp == 1 or (sp * m * n <= floats and P.row_bytes(k, bf16) // 128 // sp >= 3)
