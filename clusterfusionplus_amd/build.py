@@ -88,9 +88,38 @@ def ensure_neox():
         build_ext()
 
 
+LDS_BYTES = 160 * 1024       # of a compute unit
+
+
+def launch_lds(kernel):
+    """(LDS bytes, waves) of a workgroup of a kernel whose LDS is set at its launch, as the launch sites in csrc/seq_kernels.hip do, from
+    the kernel's name and template arguments.  Bytes None: they depend on the model.  None: the compiler knows them."""
+    import re
+    m = re.match(r"(k_seq_\w+)(?:<(.*)>)?$", kernel)
+    if m is None:
+        return None
+    name, args = m[1], [a.strip() for a in (m[2] or "").split(",")]
+    num = [int(a) for a in args if a.isdigit()]
+    size = 2 if args[0] == "bf16" else 4
+    if name == "k_seq_gemm":
+        bw, bt, wr, wc, nb = num[:5]
+        return nb * (bw + bt) * 128, wr * wc
+    if name == "k_seq_gemm8":
+        return 2 * 512 * 128, 8
+    if name == "k_seq_attn":                     # two tiles of keys and values
+        return 2 * (64 if size == 2 else 32) * (num[0] + num[1]) * size, 4
+    if name == "k_seq_latent_attn":              # three tiles of latents with the rotated part, in whole copies of 4 KB
+        units = (num[0] + 128) * size // 16 + 1
+        return 3 * -(-(32 if size == 2 else 16) * units // 256) * 4096, 4
+    if name in ("k_seq_postnorm", "k_seq_streams", "k_seq_gemv", "k_seq_route"):
+        return None, 16 if name == "k_seq_route" else 4
+    return None
+
+
 def resource_report(out=None):
-    """Compiles the HIP libraries with the compiler's kernel-resource-usage remarks and returns one line per kernel:
-    VGPRs, AGPRs, scratch bytes per lane (register spills), static LDS bytes per workgroup, waves per SIMD."""
+    """Compiles the HIP libraries with the compiler's kernel-resource-usage remarks and returns one line per kernel: VGPRs, AGPRs,
+    scratch bytes per lane (register spills), LDS bytes per workgroup, waves per SIMD.  LDS that is set at the launch, which the
+    compiler does not see, is counted in both (where it depends on the model: "+", and the waves that the registers allow)."""
     import re
     import tempfile
     hipcc = os.path.join(ROCM, "bin", "hipcc")
@@ -126,8 +155,13 @@ def resource_report(out=None):
         def g(key):
             m = re.search(key + r": (\S+)", block)
             return m.group(1) if m else "?"
-        rows.append((nice, g("VGPRs"), g("AGPRs"), g(r"ScratchSize \[bytes/lane\]"), g(r"LDS Size \[bytes/block\]"),
-                     g(r"Occupancy \[waves/SIMD\]")))
+        lds, waves, at_launch = g(r"LDS Size \[bytes/block\]"), g(r"Occupancy \[waves/SIMD\]"), launch_lds(nice)
+        if at_launch is not None and at_launch[0] is None:
+            lds += "+"
+        elif at_launch is not None:
+            total = int(lds) + at_launch[0]
+            lds, waves = str(total), str(min(int(waves), max(1, LDS_BYTES // total * at_launch[1] // 4)))
+        rows.append((nice, g("VGPRs"), g("AGPRs"), g(r"ScratchSize \[bytes/lane\]"), lds, waves))
     lines = [f"{'kernel':44s} {'VGPRs':>6s} {'AGPRs':>6s} {'scratch B/lane':>15s} {'LDS B/workgroup':>16s} {'waves/SIMD':>11s}"]
     lines += [f"{n[:44]:44s} {v:>6s} {a:>6s} {sc:>15s} {l:>16s} {o:>11s}" for n, v, a, sc, l, o in rows]
     text = "\n".join(lines)

@@ -1,8 +1,11 @@
 """The choices that a portion's kernels are launched with (csrc/seq_plan.hpp), on the host."""
+import os
 import random
+import re
 
 import pytest
 
+from clusterfusionplus_amd import build
 from tests import seq_plan as P
 from tests import test_gpu_products as G
 
@@ -113,3 +116,25 @@ def test_no_split_of_less_than_three_steps_or_more_than_its_room():
         floats = rng.choice([0, m * n, 4 * m * n, 16 << 20])
         rows, tokens, resident, sp = P.product(n, m, k, bf16, floats)
         assert sp == 1 or (sp * m * n <= floats and P.row_bytes(k, bf16) // 128 // sp >= 3)
+
+
+def test_workgroups_that_share_a_compute_unit_fit_its_memory():
+    """The table's workgroups per compute unit, and the LDS that the launches ask for (the figures of the resource report)."""
+    with open(os.path.join(build.CSRC, "seq_kernels.hip")) as f:
+        text = f.read()
+    for bf16, part in ((True, text[text.index("switch (shape)"):text.index("} else {", text.index("switch (shape)"))]), (False, text[text.index("} else {", text.index("switch (shape)")):])):
+        launches = {int(i): args for i, args in re.findall(r"case (\d+): return launch_gemm<T, ([\d, ]+), EPI>", part)}
+        launches.setdefault(7 if bf16 else 3, None if bf16 else re.search(r"launch_gemm<T, (128, [\d, ]+), EPI>\(g", part)[1])
+        assert len(launches) == (14 if bf16 else 4)
+        for i, args in launches.items():
+            rows, tokens, resident = P.tile(i, bf16)
+            assert args is None or args.startswith(f"{rows}, {tokens}, ")
+            lds, waves = build.launch_lds(f"k_seq_gemm<{'bf16' if bf16 else 'float'}, {args}, 0>" if args else "k_seq_gemm8<0>")
+            assert resident * lds <= build.LDS_BYTES, (rows, tokens)
+
+
+def test_lds_of_launches():
+    assert build.launch_lds("k_seq_gemm<bf16, 96, 128, 2, 2, 5, 0>") == (143360, 4) and build.launch_lds("k_seq_gemm8<3>") == (131072, 8)
+    assert build.launch_lds("k_seq_attn<bf16, 192, 128, 2, true>") == (81920, 4) and build.launch_lds("k_seq_attn<float, 256, 256, 1, false>") == (131072, 4)
+    assert build.launch_lds("k_seq_latent_attn<bf16, 512, 4>") == (135168, 4)
+    assert build.launch_lds("k_seq_postnorm<bf16>")[0] is None and build.launch_lds("k_seq_postnorm4<bf16, 8>") is None and build.launch_lds("k_fused<1>") is None
