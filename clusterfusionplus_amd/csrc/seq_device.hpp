@@ -20,7 +20,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kRowBytes = 128;                    // matrix rows are padded to this
-constexpr int kSeqThreads = 256;                  // threads of every sequence kernel: four waves
+constexpr int kSeqThreads = 256;                  // threads of a workgroup: four waves (matrix products have tiles with eight)
 constexpr int kSeqWaves = kSeqThreads / kWave;
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kMasked = -3.0e38f;               // score of a key that is not seen: its exp2 is zero next to any other, and next

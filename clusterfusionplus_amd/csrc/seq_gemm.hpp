@@ -37,7 +37,10 @@ struct SeqGemm {
     int experts, slot_div;   // input row of slot s: s / slot_div
     size_t w_stride;
     // (k_seq_gemm) The weights are read by one tile of tokens only, as a stream past the caches, in which the inputs stay: 37 tokens x 14336 x 4096
-    // 27.1 -> 24.8 us, 64 experts of 2816 x 2048 with 66 tokens each 171 -> 159 us; with two token tiles it costs (36 -> 42 us).
+    // 27.1 -> 24.8 us, 64 experts of 2816 x 2048 with 66 tokens each 171 -> 159 us; with two token tiles it costs (36 -> 42 us).  Weights that
+    // stay in the 256 MB cache from call to call would come faster from there: a product of 4096 x 4096 for 37 tokens, called over 200 MB of
+    // such matrices, 7.9 -> 8.5 us, over 300 MB and more 8.9 -> 8.6.  In models this small the streams are too short to tell (199 MB of
+    // weights, 37 tokens: 198 to 203 us with, 198 to 201 without; 502 MB: 610 to 633 and 646 to 658), so the model's size is not asked.
     int once;
     int splits;              // of k (kEpiF32); the s-th partial result lies s * split_stride floats behind yf
     size_t split_stride;

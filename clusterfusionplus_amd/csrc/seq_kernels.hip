@@ -6,6 +6,7 @@
 //   k_seq_gemm (output rows) -> k_seq_postnorm ->
 //   k_seq_gemm (up rows with the activation) -> k_seq_gemm (down rows) -> k_seq_postnorm;
 //   table experts: the same two products over tiles of tokens sorted by expert (k_seq_route), plus the shared expert's.
+//   Tiles and splits are chosen in seq_plan.hpp.
 // Decode (one token): five launches per layer, each with its neighbours' work fused in:
 //   k_seq_gemv (residual sum + norm of the sublayer before | q, k, v rows + bias)
 //   k_seq_attn_decode (norms, rotation, value mixing, cache append, split-KV attention, merge)
@@ -201,7 +202,8 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_postnorm4(SeqPostNorm a) {
 // One workgroup per token: raw q | k | v rows (fp32, biases included) -> norm over all of q and all of k, rotation, value
 // mixing -> q [T][H][Dp], k [G][..][Dp] and v [G][..][Vp]: rows of the portion's buffers, or of the cache itself.
 struct SeqQkv {
-    float* qkv;              // partial results of `parts` splits, part_stride floats apart; the first becomes their sum
+    float* qkv;              // partial results of `parts` splits, part_stride floats apart (k_seq_qkv_finish leaves their sum in the
+                             // first, k_seq_qkv_finish4 leaves them as they are: nobody reads them afterwards)
     int ld, parts;
     size_t part_stride;
     const float *qn, *kn;
@@ -1080,7 +1082,8 @@ int last_error() {
     return e == hipSuccess ? CFPP_OK : (int)e;
 }
 
-// dynamic LDS beyond the default limit has to be asked for, once per kernel
+// Dynamic LDS beyond the default limit has to be asked for.  At every launch: the call takes 0.07 us of host time, and no record has to be
+// kept per kernel and device.
 template <typename K>
 void allow_lds(K kernel, size_t bytes) {
     if (bytes > 65536) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);

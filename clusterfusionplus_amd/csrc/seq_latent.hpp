@@ -572,7 +572,9 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_streams(SeqStreams a) {
 }
 
 // The same for rows of whole groups of four elements, up to 1024 U of them: the streams stay in registers, and everything is requested
-// before anything is used.
+// before anything is used.  That is for portions of few tokens, where a row is a chain of round trips; with many, both kernels are bound
+// by their bytes.  Four streams of 4096 values, 37 tokens: 12.7 -> 9.8 us, 150: 15.4 -> 12.0, 512: 25.8 -> 20.4, 1000: 34.7 and 34.8, 8000:
+// 220 and 213; two of 2048, 37 tokens: 7.9 -> 5.8 us, 512: 8.3 and 8.2, 8000: 57 and 59.
 template <typename T, int S, int U>
 __global__ __launch_bounds__(kSeqThreads) void k_seq_streams4(SeqStreams a) {
     __shared__ float red[kSeqWaves];

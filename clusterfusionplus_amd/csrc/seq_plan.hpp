@@ -14,12 +14,18 @@ inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 // The tiles of the matrix products and what they cost, in us, as measured on an MI355X over 2 to 4000 tokens, 1500 to 50432
 // rows and k of 1408 to 14336 (bf16; fp32: 2 to 2000 tokens): a step of 128 bytes of k when a compute unit has one workgroup, the
 // share of a step when it has `resident` of them (the more of them, the more bytes in flight; past that they take turns), and
-// what a workgroup costs beside its steps.  The estimate below is within 10 % (root mean square) of the times measured, and what
-// it chooses is 2 % slower than the best choice on average, 20 % at worst.
+// what a workgroup costs beside its steps.
+// The estimate below is there to compare tiles: a product takes longer than it says, 15 % on average for the tile chosen (root mean
+// square 18 %; fp32 9 and 17 %), most where it is a stream of weights: 22528 x 4096 estimated and measured 32 / 40 us for 64 tokens, 36 / 41
+// for 100, 40 / 47 for 150, 58 / 68 for 300, 84 / 84 for 512, 505 / 565 for 4000.  What it chooses is 1.8 % slower than the best tile and split
+// measured, on average over 14 products and 17 numbers of tokens, 28 % at worst (10816 x 4096 for 25 tokens); fp32 1.5 and 12 %.
+// A tile is in the table because it is missed where it is chosen; without it the next choice takes longer, on average and at most:
+// 64 x 16 2 / 5 %, 64 x 32 16 / 37, 64 x 64 5 / 19, 64 x 96 4 / 24, 256 x 96 3 / 5, 256 x 128 11 / 19, 256 x 256 22 / 55, 128 x 64 4 / 15, 96 x 128
+// 7 / 17, 128 x 128 alone on a compute unit 12 / 41, 128 x 192 10 / 32, 192 x 160 9 / 33, 96 x 160 13 / 25.  128 x 128 with two workgroups per
+// compute unit is for few steps of k (keys and values from latents of 200 values, 4000 positions) and for 128256 rows of a head.
 // The tiles from the ninth on are for 50 to 700 tokens, where a product is still a stream of weights, which tiles of few tokens read
 // two or three times: they hold the tokens in one tile or two, and their rings fill a compute unit's LDS.  22528 rows x 4096 without
-// -> with them: 64 tokens 44 -> 41 us, 100: 60 -> 42, 150: 63 -> 48, 300: 86 -> 67; over nine products of 2048 to 28672 rows and 37 to
-// 1000 tokens, the choice was 8.8 % behind the best tile measured and is 1.7 % behind it.  Eight layers of width 4096 in a model: 100
+// -> with them: 64 tokens 44 -> 41 us, 100: 60 -> 42, 150: 63 -> 48, 300: 86 -> 67.  Eight layers of width 4096 in a model: 100
 // tokens 1460 -> 1305 us, 128: 1548 -> 1382, 256: 1865 -> 1702, 600: the same.
 struct GemmShape { int rows, tokens, resident; float step, share, fixed; };
 constexpr GemmShape kShapes16[] = {{64, 16, 2, 0.213f, 0.180f, 1.7f}, {64, 32, 2, 0.228f, 0.204f, 1.9f}, {64, 64, 2, 0.269f, 0.241f, 2.4f},

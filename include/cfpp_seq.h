@@ -118,7 +118,8 @@ typedef struct cfpp_seq_desc {
     const void* head;                      /* T [vocab, width] */
     int32_t slots;                         /* sequences that can hold cache at a time */
     int32_t capacity;                      /* positions per sequence */
-    int32_t max_portion;                   /* prompt tokens per pass; longer inputs are cut into passes of this size */
+    int32_t max_portion;                   /* prompt tokens per pass; longer inputs are cut into passes of this size (with table
+                                              experts of fewer, where a pass' inputs of the expert products would reach 4 GiB) */
 } cfpp_seq_desc;
 
 typedef struct cfpp_seq cfpp_seq;          /* opaque */
@@ -128,7 +129,8 @@ size_t cfpp_seq_row_pitch(int32_t K, int32_t dtype);
 const char* cfpp_seq_version(void);
 
 /* Allocates the caches ([slots] x the rows a layer can see: min(chunk, capacity), or capacity without chunks), rotary
- * tables and scratch memory (latent mixers: keys and values of all heads for one sequence of `capacity` positions).  The layer array is copied, the tensors are not. */
+ * tables and scratch memory (latent mixers: keys and values of all heads for one sequence of `capacity` positions; partial results
+ * of split products: up to 128 MB).  The layer array is copied, the tensors are not. */
 int cfpp_seq_create(const cfpp_seq_desc* desc, cfpp_seq** out);
 int cfpp_seq_destroy(cfpp_seq* s);
 /* Device bytes held by the object (caches and scratch). */
