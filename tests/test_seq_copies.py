@@ -1,5 +1,5 @@
-"""The hand-written copies from memory to LDS, in the assembly that the compiler makes around them.  It sees neither that they write
-m0 nor which wait states they need: both have to hold inside them, wherever they are put."""
+"""The hand-written copies from memory to LDS, in the assembly that the compiler makes around them.  It does not look into them: m0 has
+to be an operand that it writes for each, and their base must not need wait states, which it would not put in front of them."""
 import os
 import re
 import shutil
