@@ -66,7 +66,8 @@ template <typename T, int NK, int NT> struct AttnTile {
 // What bounds it: the matrix cores and the softmax's vector instructions, which take turns inside a wave and overlap with the other
 // wave of the SIMD.  So two workgroups per compute unit, one barrier per tile, and nothing is waited for but the tile itself: with
 // copies that the compiler knows of it waited for the next tile's before this tile's first read of LDS, and values took a detour
-// through registers to be transposed.  8000 tokens, 32 heads of 192 and 128: 1753 -> 1237 us; 2048 tokens, 128 and 128: 141 -> 103 us.
+// through registers to be transposed.  8000 tokens, 32 heads of 192 and 128: 1753 -> 1237 us; 2048 tokens, 128 and 128: 141 -> 103 us
+// (before the order of the workgroups was changed, below).
 // 37 tokens at 1990, 32 / 8 heads: 85 -> 12 us and 5 for the merge (24 workgroups became 384).
 // (NK: elements of a key row in LDS, NT: value columns.  The products run over all of them, without branches between the reads
 // of LDS: past the end of the query there are zeros, and of the columns past the end of a value nothing is stored.
@@ -77,11 +78,10 @@ __global__ __launch_bounds__(kSeqThreads, (NT <= 128 ? 2 : 1)) void k_seq_attn(S
     constexpr int KT = L::keys, KS = L::kbytes / 64;
     extern __shared__ __align__(1024) char lds[];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 15, g = lane >> 4;
-    // the longest walks first; every second group of eight runs backwards, so that each XCD (workgroups go round them) gets as
-    // many long ones as the others
-    const int gq = blockIdx.y, ncols = a.T * a.R, gx = gridDim.x;
-    int bx = blockIdx.x;
-    if (((bx >> 3) & 1) && (bx | 7) < gx) bx ^= 7;
+    // The longest walks of all key heads first, so that the short ones fill the chip's last moments (head by head, a quarter of the compute
+    // units' time was a tail: 8000 tokens, 32 heads of 192 and 128: 1264 -> 956 us; 2048 tokens, 128 and 128: 104 -> 86 us); and where the heads are a
+    // multiple of eight, all workgroups of a head are on one XCD and walk its keys side by side.
+    const int ncols = a.T * a.R, gx = (ncols + 64 * CT - 1) / (64 * CT), G = a.H / a.R, bx = blockIdx.x / G, gq = blockIdx.x - bx * G;
     const int c0 = (gx - 1 - bx) * 64 * CT;
 
     // (its sign goes to the query; not zero, so that it keeps the scores of keys that are not seen at -infinity; NaN stays NaN)
@@ -119,7 +119,7 @@ __global__ __launch_bounds__(kSeqThreads, (NT <= 128 ? 2 : 1)) void k_seq_attn(S
 
     // tiles: [k_first, k_split) in the cache, then [k_split, k_end) in the buffer; this split's are t0 .. t1 - 1
     const int in_cache = max(0, min(k_end, a.k_split) - k_first), n_cached = (in_cache + KT - 1) / KT, new_first = max(k_first, a.k_split);
-    const int ntiles = n_cached + (max(0, k_end - new_first) + KT - 1) / KT, split = blockIdx.z;
+    const int ntiles = n_cached + (max(0, k_end - new_first) + KT - 1) / KT, split = blockIdx.y;
     const int t0 = mul_div(ntiles, split, a.splits), t1 = mul_div(ntiles, split + 1, a.splits);
     struct Tile { int k0, hi; const char *k, *v; };      // first key, end of its part, row of position 0
     auto tile_at = [&](int i) {

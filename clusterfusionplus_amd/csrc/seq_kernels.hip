@@ -1174,7 +1174,7 @@ void launch_attn(SeqAttn a, int G, int cus, size_t room, float* part, hipStream_
         constexpr int CT = decltype(n)::value;
         constexpr bool SH = decltype(sh)::value;
         allow_lds(k_seq_attn<T, NK, NT, CT, SH>, lds);
-        hipLaunchKernelGGL((k_seq_attn<T, NK, NT, CT, SH>), dim3(ceil_div(cols, 64 * CT), G, a.splits), dim3(kSeqThreads), lds, st, a);
+        hipLaunchKernelGGL((k_seq_attn<T, NK, NT, CT, SH>), dim3(ceil_div(cols, 64 * CT) * G, a.splits), dim3(kSeqThreads), lds, st, a);
     };
     auto pick = [&](auto sh) {
         if constexpr (sizeof(T) == 2) {
