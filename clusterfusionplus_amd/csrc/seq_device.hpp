@@ -370,6 +370,12 @@ __device__ __forceinline__ void split_weights(f32x4 a, f32x4 b, u32x4& hi, u32x4
     hi = u32x4{pack_bf16(a[0], a[1]), pack_bf16(a[2], a[3]), pack_bf16(b[0], b[1]), pack_bf16(b[2], b[3])};
     const float v[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
 #pragma unroll
+    for (int j = 0; j < 4; ++j) {                        // (the compiler would convert every second value twice)
+        uint32_t x = hi[j];
+        asm("" : "+v"(x));
+        hi[j] = x;
+    }
+#pragma unroll
     for (int j = 0; j < 4; ++j) lo[j] = pack_bf16(v[2 * j] - __uint_as_float(hi[j] << 16), v[2 * j + 1] - __uint_as_float(hi[j] & 0xffff0000u));
 }
 // A transposing read of LDS: lane i of a group of 16 gives the address of four bf16 of a row (rows of the group's lanes i / 4, columns

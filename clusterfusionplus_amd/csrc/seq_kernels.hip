@@ -1163,24 +1163,23 @@ void expert_gemm(const cfpp_seq* s, const LayerPlan& L, SeqGemm g, int n, hipStr
 
 template <typename T, int NK, int NT>
 void launch_attn(SeqAttn a, int G, int cus, size_t room, float* part, hipStream_t st) {
-    using L = AttnTile<T, NK, NT>;
     const int cols = a.T * a.R;
-    const AttnPlan plan = plan_attn({a.T, a.R, G, a.pos0, a.chunk, L::keys, sizeof(T) == 2, NT <= 128 ? 2 : 1, (size_t)a.T * a.H * (a.vtiles * 16 + 2)}, cus, room);
+    const AttnPlan plan = plan_attn({a.T, a.R, G, a.pos0, a.chunk, AttnTile<T, NK, NT, 16>::keys, sizeof(T) == 2, NT <= 128 ? 2 : 1, (size_t)a.T * a.H * (a.vtiles * 16 + 2)}, cus, room);
     a.splits = plan.splits;
     a.part = part;
     a.ml = part + (size_t)a.splits * a.T * a.H * a.vtiles * 16;
-    const size_t lds = 2 * L::size;
     auto go = [&](auto n, auto sh) {
-        constexpr int CT = decltype(n)::value;
+        constexpr int C = decltype(n)::value;
         constexpr bool SH = decltype(sh)::value;
-        allow_lds(k_seq_attn<T, NK, NT, CT, SH>, lds);
-        hipLaunchKernelGGL((k_seq_attn<T, NK, NT, CT, SH>), dim3(ceil_div(cols, 64 * CT) * G, a.splits), dim3(kSeqThreads), lds, st, a);
+        const size_t lds = 2 * AttnTile<T, NK, NT, C>::size;
+        allow_lds(k_seq_attn<T, NK, NT, C, SH>, lds);
+        hipLaunchKernelGGL((k_seq_attn<T, NK, NT, C, SH>), dim3(ceil_div(cols, C * kSeqWaves) * G, a.splits), dim3(kSeqThreads), lds, st, a);
     };
     auto pick = [&](auto sh) {
         if constexpr (sizeof(T) == 2) {
-            if (plan.two) return go(std::integral_constant<int, 2>{}, sh);   // (fp32: two column tiles do not fit the registers)
+            if (plan.two) return go(std::integral_constant<int, 32>{}, sh);  // (fp32: they do not fit the registers)
         }
-        go(std::integral_constant<int, 1>{}, sh);
+        go(std::integral_constant<int, 16>{}, sh);
     };
     if (a.runits > 0) pick(std::true_type{});
     else pick(std::false_type{});
@@ -1273,7 +1272,6 @@ void portion_grouped(cfpp_seq* s, const LayerPlan& L, int slot, int n, int pos, 
     a.T = n;
     a.H = d.heads;
     a.R = L.R;
-    a.dsteps = L.krow / 64;
     a.qrow = a.krow = L.krow;
     a.vrow = L.vrow;
     a.V = d.vdim;
@@ -1335,7 +1333,6 @@ void portion_latent(cfpp_seq* s, const LayerPlan& L, int slot, int n, int pos, i
     a.T = n;
     a.H = d.heads;
     a.R = 1;
-    a.dsteps = L.qrow / 64;
     a.qrow = L.qrow;
     a.krow = L.plain;
     a.runits = L.shared / 16;

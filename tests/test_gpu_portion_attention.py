@@ -83,3 +83,24 @@ def test_projection_sizes(name, dtype):
     m = nibotar.from_tensors(cfg, w, dtype, capacity=100)
     logits = torch.cat([m.forward(0, toks[:33], 0, range(33)), m.forward(0, toks[33:62], 33, range(29)), m.forward(0, toks[62:], 62, range(28))])
     assert N.error(logits, want) < LIMIT[dtype]
+
+
+# enough columns for blocks of 32 (512 workgroups of 128): every size of tile, heads that share keys, chunks, a last block that is not full, keys of
+# the portion and of the context before it, scores of either sign and scores that are no numbers
+BLOCKS = {"small": (N, N.attn(64, 64, 16, 32)), "middle": (N, N.attn(64, 64, 72, 80, rot=8)), "large": (N, N.attn(64, 64, 200, 250)),
+          "groups": (N, N.attn(96, 48, 40, 56, rot=8)), "chunks": (N, N.attn(64, 64, 40, 56, chunk=400)), "negative": (N, N.attn(64, 64, 40, 56, scale=-0.2)),
+          "latent": (K, K.gated(64, 40, 16, 56, 48)), "latent_wide": (K, K.sunk(64, 128, 64, 128, 96)), "nan": (N, N.attn(64, 64, 40, 56, scale=float("nan")))}
+
+
+@pytest.mark.parametrize("name", list(BLOCKS))
+def test_columns_in_blocks_of_32(name):
+    from clusterfusionplus_amd import kagapel, nibotar
+    M, mixer = BLOCKS[name]
+    cfg = M.model(64, 51, [mixer], positions=1900) if M is K else M.model(64, 51, [(mixer, None)])
+    w, toks = M.weights(cfg, 5), M.prompt(cfg, 1807, 6)
+    m = (nibotar if M is N else kagapel).from_tensors(cfg, w, torch.bfloat16, capacity=1807)
+    got = torch.cat([m.forward(0, toks[:900], 0, range(900)), m.forward(0, toks[900:], 900, range(907))])
+    if name == "nan":
+        assert got.isnan().all()
+    else:
+        assert N.error(got, M.oracle(cfg, w, toks)) < LIMIT[torch.bfloat16]
