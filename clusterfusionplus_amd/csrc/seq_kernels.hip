@@ -277,17 +277,18 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_qkv_finish(SeqQkv a) {
     }
 }
 
-// The same where heads are whole groups of four elements and the row fits U groups per thread: everything is read once, in one round
+// The same where heads are whole groups of four elements and the row has up to 16384 values: everything is read once, in one round
 // trip (partial results of a split product included), and stays in registers.  Bound by its bytes: 2048 tokens of 3 x 4096 values take
-// 50 us in k_seq_qkv_finish and 42 us here, 37 tokens of 6144 in four parts 13 and 8.6 us.
-template <typename T, int U>
+// 50 us in k_seq_qkv_finish and 42 us here.
+template <typename T>
 __global__ __launch_bounds__(kSeqThreads) void k_seq_qkv_finish4(SeqQkv a) {
+    constexpr int U = 16;
     __shared__ float2 red[kSeqWaves];
     const int t = blockIdx.x, tid = threadIdx.x, nq = a.H * a.D, nk = a.G * a.D, nv = a.G * a.V, n4 = (nq + nk + nv) / 4;
     f32x4 x[U];
 #pragma unroll
     for (int j = 0; j < U; ++j) x[j] = reinterpret_cast<const f32x4*>(a.qkv + (size_t)t * a.ld)[min(tid + j * kSeqThreads, n4 - 1)];
-    add_rows4<U, (U <= 8 ? 3 : 1)>(x, a.qkv + (size_t)t * a.ld + a.part_stride, a.parts - 1, a.part_stride, n4);
+    add_rows4<U, 1>(x, a.qkv + (size_t)t * a.ld + a.part_stride, a.parts - 1, a.part_stride, n4);
     float sq = 0.0f, sk = 0.0f;
 #pragma unroll
     for (int j = 0; j < U; ++j) {
@@ -334,6 +335,100 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_qkv_finish4(SeqQkv a) {
                 for (int r = 0; r < 4; ++r) y[r] = (1.0f - a.lambda) * y[r] + a.lambda * f[r];
             }
             store4<T>(vo + g * a.vhead + d * sizeof(T), y);
+        }
+    }
+    // zeros behind the heads: layers of other sizes share these buffers
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    const int dz = (a.Dp - a.D) / 4, vz = (a.Vp - a.V) / 4;
+    if (dz > 0)
+        for (int i = tid; i < (a.H + a.G) * dz; i += kSeqThreads) {
+            const int h = i / dz, d = a.D + (i - h * dz) * 4;
+            store4<T>((h < a.H ? qo + (size_t)h * a.Dp * sizeof(T) : ko + (h - a.H) * a.khead) + d * sizeof(T), zero);
+        }
+    if (vz > 0)
+        for (int i = tid; i < a.G * vz; i += kSeqThreads) {
+            const int g = i / vz, d = a.V + (i - g * vz) * 4;
+            store4<T>(vo + g * a.vhead + d * sizeof(T), zero);
+        }
+}
+
+// The same for rows of up to 8192 values, where there are registers for what the norms, the rotation and the mixing read, too: it is requested with
+// the row, not behind the sums (37 tokens of 6144 in four parts 6.9 -> 6.1 us, 700 of 3072 8.7 -> 6.8, 1990 of 6144 29 -> 22; rows of 12288, with
+// two waves of a SIMD instead of four, would take 66 us instead of 43).  C: parts requested together; a row that is whole needs no registers
+// for them.
+template <typename T, int C>
+__global__ __launch_bounds__(kSeqThreads) void k_seq_qkv_finish8(SeqQkv a) {
+    constexpr int U = 8;
+    __shared__ float2 red[kSeqWaves];
+    const int t = blockIdx.x, tid = threadIdx.x, nq = a.H * a.D, nk = a.G * a.D, nv = a.G * a.V, n4 = (nq + nk + nv) / 4;
+    f32x4 x[U];
+#pragma unroll
+    for (int j = 0; j < U; ++j) x[j] = reinterpret_cast<const f32x4*>(a.qkv + (size_t)t * a.ld)[min(tid + j * kSeqThreads, n4 - 1)];
+    const float2* cs = a.cs + (size_t)(a.pos0 + t) * (a.rot / 2);
+    const float rd = 1.0f / (float)a.D, rv = 1.0f / (float)a.V;
+    struct Place { int e, h, d; };                       // element of the queries (keys, values), head, element of the head
+    auto head_of = [&](int i) {
+        const int e = i < nq ? i : i < nq + nk ? i - nq : i - nq - nk, h = (int)(((float)e + 0.5f) * (i < nq + nk ? rd : rv));      // (e < 2^16: exact)
+        return Place{e, h, e - h * (i < nq + nk ? a.D : a.V)};
+    };
+    struct More { f32x4 w; float2 c[2]; };               // norm weights and pairs; of values w: what is mixed in
+    auto more = [&](int i) {
+        const Place at = head_of(i);
+        More m{f32x4{0.f, 0.f, 0.f, 0.f}, {make_float2(1.0f, 0.0f), make_float2(1.0f, 0.0f)}};
+        if (i < nq + nk) {
+            m.w = *reinterpret_cast<const f32x4*>((i < nq ? a.qn : a.kn) + at.e);
+#pragma unroll
+            for (int r = 0; r < 2; ++r)
+                if (at.d + 2 * r < a.rot) m.c[r] = cs[at.d / 2 + r];
+        } else if (a.v_role == 2) {
+            m.w = *reinterpret_cast<const f32x4*>(a.v_first + (size_t)t * nv + at.e);
+        }
+        return m;
+    };
+    More m[U];
+#pragma unroll
+    for (int j = 0; j < U; ++j) m[j] = more(min(tid + j * kSeqThreads, n4 - 1) * 4);
+    add_rows4<U, C>(x, a.qkv + (size_t)t * a.ld + a.part_stride, a.parts - 1, a.part_stride, n4);
+    float sq = 0.0f, sk = 0.0f;
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+        const int i = (tid + j * kSeqThreads) * 4;
+        float s = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s = fmadd(x[j][r], x[j][r], s);
+        sq += i < nq ? s : 0.0f;
+        sk += i >= nq && i < nq + nk ? s : 0.0f;
+    }
+    const float2 sums = block_sum2(sq, sk, red);
+    const float iq = inv_rms(sums.x, nq, a.eps), ik = inv_rms(sums.y, nk, a.eps);
+    char* qo = a.q + (size_t)t * a.H * a.Dp * sizeof(T);
+    char* ko = a.k + (size_t)t * a.Dp * sizeof(T);
+    char* vo = a.v + (size_t)t * a.Vp * sizeof(T);
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+        const int i = (tid + j * kSeqThreads) * 4;
+        if (i >= nq + nk + nv) continue;
+        const Place at = head_of(i);
+        if (i < nq + nk) {
+            const bool q = i < nq;
+            const float inv = q ? iq : ik;
+            f32x4 y;
+#pragma unroll
+            for (int r = 0; r < 4; r += 2) {
+                const float2 cc = m[j].c[r / 2];
+                const float u = x[j][r] * m[j].w[r], v = x[j][r + 1] * m[j].w[r + 1];
+                y[r] = rotate_finish(RotIn{u, v, cc.x, -cc.y}, inv);
+                y[r + 1] = rotate_finish(RotIn{v, u, cc.x, cc.y}, inv);
+            }
+            store4<T>((q ? qo + (size_t)at.h * a.Dp * sizeof(T) : ko + at.h * a.khead) + at.d * sizeof(T), y);
+        } else {
+            f32x4 y = x[j];
+            if (a.v_role == 1) *reinterpret_cast<f32x4*>(a.v_first + (size_t)t * nv + at.e) = y;
+            if (a.v_role == 2) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) y[r] = (1.0f - a.lambda) * y[r] + a.lambda * m[j].w[r];
+            }
+            store4<T>(vo + at.h * a.vhead + at.d * sizeof(T), y);
         }
     }
     // zeros behind the heads: layers of other sizes share these buffers
@@ -1257,8 +1352,10 @@ void portion_grouped(cfpp_seq* s, const LayerPlan& L, int slot, int n, int pos, 
              d.rot_dims, pos, (size_t)(direct ? L.rows : cap) * L.krow, (size_t)(direct ? L.rows : cap) * L.vrow, L.v_role, s->v_first, s->q,
              direct ? kc + (size_t)(pos - cs0) * L.krow : s->k, direct ? vc + (size_t)(pos - cs0) * L.vrow : s->v};
     auto finish = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(n), dim3(kSeqThreads), 0, st, f); };
-    if (d.dim % 4 == 0 && d.vdim % 4 == 0 && L.n_qkv <= 8 * 4 * kSeqThreads) finish(k_seq_qkv_finish4<T, 8>);
-    else if (d.dim % 4 == 0 && d.vdim % 4 == 0 && L.n_qkv <= 16 * 4 * kSeqThreads) finish(k_seq_qkv_finish4<T, 16>);
+    const bool fours = d.dim % 4 == 0 && d.vdim % 4 == 0;
+    if (fours && L.n_qkv <= 8 * 4 * kSeqThreads && parts > 1) finish(k_seq_qkv_finish8<T, 3>);
+    else if (fours && L.n_qkv <= 8 * 4 * kSeqThreads) finish(k_seq_qkv_finish8<T, 1>);
+    else if (fours && L.n_qkv <= 16 * 4 * kSeqThreads) finish(k_seq_qkv_finish4<T>);
     else finish(k_seq_qkv_finish<T>);
 
     SeqAttn a{};
@@ -1299,8 +1396,16 @@ template <typename T>
 void portion_latent(cfpp_seq* s, const LayerPlan& L, int slot, int n, int pos, int parts, hipStream_t st) {
     const cfpp_seq_layer& d = L.d;
     char* kc = L.kc + (size_t)slot * s->d.capacity * L.crow;
-    SeqLatentFinish f{s->qkv, s->ld_qkv, L.n_qkv, parts, (size_t)n * s->ld_qkv, L.own, latent_row_of<T>(s, L), L.cs, d.heads, d.dim, d.rot_dims, pos, L.plain, L.qrow, s->q, kc};
-    hipLaunchKernelGGL(k_seq_latent_finish<T>, dim3(n), dim3(kSeqThreads), 0, st, f);
+    const int made = d.heads * (d.dim + d.rot_dims) + (L.own ? d.kv_rank + d.rot_dims : 0);       // values in front of the gates
+    const int read = parts > 1 ? L.n_qkv : made;         // (of a row that is whole, the gates stay where they are)
+    SeqLatentFinish f{s->qkv, s->ld_qkv, read, made, parts, (size_t)n * s->ld_qkv, L.own, latent_row_of<T>(s, L), L.cs, d.heads, d.dim, d.rot_dims, pos, L.plain, L.qrow, s->q, kc};
+    auto finish = [&](auto kernel, size_t lds) { hipLaunchKernelGGL(kernel, dim3(n), dim3(kSeqThreads), lds, st, f); };
+    const bool fours = read % 4 == 0 && made % 4 == 0;
+    const size_t lds = (size_t)made * 4 + d.rot_dims * 4;
+    if (fours && read <= 8 * 4 * kSeqThreads && parts > 1) finish(k_seq_latent_finish4<T, 8, 3>, lds);
+    else if (fours && read <= 8 * 4 * kSeqThreads) finish(k_seq_latent_finish4<T, 8, 1>, lds);
+    else if (fours && read <= 12 * 4 * kSeqThreads) finish(k_seq_latent_finish4<T, 12, 1>, lds);
+    else finish(k_seq_latent_finish<T>, 0);
 
     const int ctx = pos + n, cap = s->d.capacity;
     SeqGemm g{};

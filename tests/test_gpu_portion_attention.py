@@ -104,3 +104,22 @@ def test_columns_in_blocks_of_32(name):
         assert got.isnan().all()
     else:
         assert N.error(got, M.oracle(cfg, w, toks)) < LIMIT[torch.bfloat16]
+
+
+# latent projections of up to 8192 and 12288 values, and of more; in one part (64 columns) and in several (512); rows and gates that are no whole groups
+# of four; a layer that reads the latents of another
+LATENTS = {"6k": (24, 128, 64, 56, 48), "12k": (48, 128, 64, 56, 48), "16k": (64, 128, 64, 56, 48), "no_fours": (3, 41, 16, 55, 49), "gates_no_fours": (3, 44, 16, 55, 48)}
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("width", [64, 512])
+@pytest.mark.parametrize("name", list(LATENTS))
+def test_latent_projection_sizes(name, width, dtype):
+    from clusterfusionplus_amd import kagapel
+    dims = LATENTS[name]
+    cfg = K.model(width, 51, [K.gated(*dims), K.sunk(*dims, kv_from=0), K.gated(*dims)])
+    w, toks = K.weights(cfg, 5), K.prompt(cfg, 90, 6)
+    want = K.oracle(cfg, w, toks)
+    m = kagapel.from_tensors(cfg, w, dtype, capacity=100)
+    logits = torch.cat([m.forward(0, toks[:33], 0, range(33)), m.forward(0, toks[33:62], 33, range(29)), m.forward(0, toks[62:], 62, range(28))])
+    assert N.error(logits, want) < LIMIT[dtype]
