@@ -203,7 +203,7 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_postnorm4(SeqPostNorm a) {
 // mixing -> q [T][H][Dp], k [G][..][Dp] and v [G][..][Vp]: rows of the portion's buffers, or of the cache itself.
 struct SeqQkv {
     float* qkv;              // partial results of `parts` splits, part_stride floats apart (k_seq_qkv_finish leaves their sum in the
-                             // first, k_seq_qkv_finish4 leaves them as they are: nobody reads them afterwards)
+                             // first, k_seq_qkv_finish4 and 8 leave them as they are: nobody reads them)
     int ld, parts;
     size_t part_stride;
     const float *qn, *kn;

@@ -114,12 +114,14 @@ inline ExpertPlan plan_experts(const ExpertSizes& e, bool bf16, int cus) {
 // Attention of a portion of T tokens at positions pos0 and on: R query heads for each of G key / value heads, `keys` of them in a tile.
 struct AttnSizes {
     int T, R, G, pos0, chunk, keys;
-    bool pairs;              // bf16: two column tiles per wave are possible
+    bool pairs;              // bf16: waves of 32 columns are possible
     int per_cu;              // workgroups that share a compute unit
     size_t floats;           // of a split's partial results
 };
-// Columns of a workgroup and splits of the keys.  bf16: two column tiles per wave share the reads of keys and values; one, where that
-// leaves fewer columns empty or where two workgroups per compute unit are not reached.  Splits fill the chip: two workgroups per
+// Columns of a workgroup and splits of the keys.  bf16: waves of 32 columns take fewer instructions per weight, those of 16 balance better
+// where there are few workgroups.  The line is at two workgroups of four such waves per compute unit (us with 16 / 32 columns, 32 heads of 128 and
+// 128: 1500 tokens, 384 workgroups 47 / 55, 2048 tokens, 512 workgroups 76.5 / 76, 3000 tokens 136 / 134; of 192 and 128: 1600 tokens 67 / 78,
+// 2048 90 / 96, 3000 171 / 168).  Splits fill the chip: two workgroups per
 // compute unit, with two tiles at least in each split of the longest walk, which begins at the chunk of the portion's first token (that
 // chunk counts and not the context: 37 tokens just behind a chunk of 8192 see one tile; shared by 16 splits, eight layers of 32 / 8 heads
 // of 128 took 1005 us, and take 957).
