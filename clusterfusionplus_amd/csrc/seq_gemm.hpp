@@ -302,12 +302,15 @@ __global__ __launch_bounds__(kWave* WR* WC) void k_seq_gemm(SeqGemm p) {
     GemmTile t;
     if (!gemm_tile<BW, BT>(p, t)) return;
     const int nk = p.kbytes / kRowBytes, kb = mul_div(nk, t.split, p.splits), n = mul_div(nk, t.split + 1, p.splits) - kb;
-    // Tiles of a weight stream begin at different steps and go round: workgroups that run side by side would otherwise ask for the same 128
-    // bytes of rows that are 4 KB apart, or a multiple of it, which lie in few of the memory's channels (the copies in flight cover less than 512
-    // bytes of a row).  64 experts of 2816 x 2048, 66 tokens each: 154 -> 140 us; 21888 gated rows x 2048, 150 tokens: 31.2 -> 28.1; 14336 x 4096, 37
+    // Tiles of a weight stream begin at different steps and go round (steps of 5 apart: of n steps every one is a start, or n / 5 of them where n
+    // is a multiple of 5).  Workgroups that run side by side would otherwise ask for the same 128 bytes of rows that are 4 KB apart, or a multiple of
+    // it; the copies in flight cover (NB - 1) x 128 <= 640 bytes of a row.  That these lie in few of the memory's channels is supposed, from the
+    // times alone: 64 experts of 2816 x 2048, 66 tokens each: 154 -> 140 us; 21888 gated rows x 2048, 150 tokens: 31.2 -> 28.1; 14336 x 4096, 37
     // tokens: 24.7 -> 24.2.  Not where several tiles of tokens share a weight's copy in the caches or the splits of k are apart by themselves (2 to 5 %
-    // slower), nor for a head, whose eight rounds of workgroups drift apart (1 % slower).
-    const int first = EPI != kEpiHead && p.once && p.splits == 1 ? t.tw * 5 % n : 0;
+    // slower), nor for a head, whose eight rounds of workgroups drift apart (1 % slower), nor in fp32 (14336 x 4096, 2 tokens 46 and 43 us, but 17
+    // tokens 56 and 58, 12 experts' 2816 x 2048 43 and 47).
+    constexpr bool kTurns = sizeof(T) == 2 && EPI != kEpiHead;
+    const int first = kTurns && p.once && p.splits == 1 ? t.tw * 5 % n : 0;
     const char* bw = uniform(t.w + (size_t)t.tw * BW * p.kbytes + (size_t)(kb + first) * kRowBytes);
     const char* ba = uniform(p.a + (p.tile_off != nullptr ? (size_t)0 : (size_t)t.tt * BT * p.lda) + (size_t)(kb + first) * kRowBytes);
     uint32_t vw[WI], va[AI];
@@ -333,13 +336,13 @@ __global__ __launch_bounds__(kWave* WR* WC) void k_seq_gemm(SeqGemm p) {
         }
 #pragma unroll
         for (int i = 0; i < AI; ++i) copy_to_lds16_at(va[i], ba, b + BW * kRowBytes + min(wave + i * NW, AC - 1) * 1024);
-        bw += kRowBytes;
-        ba += kRowBytes;
+        ++issued;
+        // (No branch: a step of a narrow tile takes 0.2 us, and a jump out of the loop's line costs 4 to 11 % of it.  Head of 4000 x 4096, one token:
+        // 16.5 us, with the jump 18.2; 1024 x 2048 in bf16, 300 tokens: 10.8 and 12.0; 14336 x 4096 in fp32, 17 tokens: 55.7 and 58.9.)
+        const int64_t on = kRowBytes - (kTurns && issued == n - first ? (int64_t)n * kRowBytes : 0);
+        bw += on;
+        ba += on;
         fill = next(fill);
-        if (++issued == n - first) {
-            bw -= (size_t)n * kRowBytes;
-            ba -= (size_t)n * kRowBytes;
-        }
     };
     f32x4 acc[MI][NI];
 #pragma unroll

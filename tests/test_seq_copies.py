@@ -95,18 +95,40 @@ def test_scalar_base_from_a_vector_instruction(kernels):
     assert too_early(code) == []
 
 
-def test_no_copy_of_the_library_reads_its_base_too_early(tmp_path):
+@pytest.fixture(scope="module")
+def library(tmp_path_factory):
+    """Name -> instructions of every kernel of the built library, in the order of their addresses."""
     objdump = os.path.join(build.ROCM, "lib", "llvm", "bin", "llvm-objdump")
     if shutil.which(objdump) is None:
         pytest.skip("no llvm-objdump")
     build.ensure_seq()
-    lib = shutil.copy(build.SEQ_LIB, tmp_path)
-    subprocess.run([objdump, "--offloading", lib], cwd=tmp_path, check=True, stdout=subprocess.DEVNULL)
-    device, = tmp_path.glob("*gfx950")
+    d = tmp_path_factory.mktemp("library")
+    lib = shutil.copy(build.SEQ_LIB, d)
+    subprocess.run([objdump, "--offloading", lib], cwd=d, check=True, stdout=subprocess.DEVNULL)
+    device, = d.glob("*gfx950")
     text = subprocess.run([objdump, "-d", "--no-show-raw-insn", str(device)], check=True, stdout=subprocess.PIPE, text=True).stdout
-    code = [line.split("//")[0].strip() for line in text.splitlines() if line.startswith("\t")]
+    out = {}
+    for part in re.split(r"\n(?=[0-9a-f]+ <)", text):
+        name = re.match(r"[0-9a-f]+ <(.*)>:", part)
+        if name:
+            out[name[1]] = [line.split("//")[0].strip() for line in part.splitlines()[1:] if line.startswith("\t")]
+    return out
+
+
+def test_no_copy_of_the_library_reads_its_base_too_early(library):
+    code = [t for kernel in library.values() for t in kernel]
     assert sum(t.startswith("global_load_lds_dwordx4") for t in code) > 1000
     assert too_early(code) == []
+
+
+def test_rings_step_on_without_a_jump(library):
+    """Between the last copy of a step's request and the step's first read of LDS there is no branch, in any of the products with a ring."""
+    rings = {name: code for name, code in library.items() if "k_seq_gemmI" in name}
+    assert len(rings) > 50
+    for name, code in rings.items():
+        read = next(i for i, t in enumerate(code) if t.startswith("ds_read_b128"))
+        copy = max(i for i in range(read) if code[i].startswith("global_load_lds_dwordx4"))
+        assert [t for t in code[copy:read] if t.startswith(("s_branch", "s_cbranch"))] == [], name
 
 
 @pytest.mark.parametrize("kind", [0, 1, 2], ids=["at", "once", "from"])
