@@ -352,13 +352,13 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_qkv_finish4(SeqQkv a) {
         }
 }
 
-// The same for rows of up to 8192 values, where there are registers for what the norms, the rotation and the mixing read, too: it is requested with
-// the row, not behind the sums (37 tokens of 6144 in four parts 6.9 -> 6.1 us, 700 of 3072 8.7 -> 6.8, 1990 of 6144 29 -> 22; rows of 12288, with
-// two waves of a SIMD instead of four, would take 66 us instead of 43).  C: parts requested together; a row that is whole needs no registers
-// for them.
-template <typename T, int C>
+// The same for rows of up to 1024 U <= 8192 values, where there are registers for what the norms, the rotation and the mixing read, too: it is
+// requested with the row, not behind the sums (37 tokens of 6144 in four parts 6.9 -> 6.1 us, 700 of 3072 8.7 -> 6.8, 1990 of 6144 29 -> 22; rows of
+// 12288, with two waves of a SIMD instead of four, would take 66 us instead of 43).  U = 4 where the row fits: places behind its end are requested
+// like others (150 tokens of 3072 in parts 5.4 -> 4.6 us, 300 of 3072 4.9 -> 4.1, 2 of 768 3.6 -> 2.9).  C: parts requested together; a row that is
+// whole needs no registers for them.
+template <typename T, int U, int C>
 __global__ __launch_bounds__(kSeqThreads) void k_seq_qkv_finish8(SeqQkv a) {
-    constexpr int U = 8;
     __shared__ float2 red[kSeqWaves];
     const int t = blockIdx.x, tid = threadIdx.x, nq = a.H * a.D, nk = a.G * a.D, nv = a.G * a.V, n4 = (nq + nk + nv) / 4;
     f32x4 x[U];
@@ -1353,8 +1353,10 @@ void portion_grouped(cfpp_seq* s, const LayerPlan& L, int slot, int n, int pos, 
              direct ? kc + (size_t)(pos - cs0) * L.krow : s->k, direct ? vc + (size_t)(pos - cs0) * L.vrow : s->v};
     auto finish = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(n), dim3(kSeqThreads), 0, st, f); };
     const bool fours = d.dim % 4 == 0 && d.vdim % 4 == 0;
-    if (fours && L.n_qkv <= 8 * 4 * kSeqThreads && parts > 1) finish(k_seq_qkv_finish8<T, 3>);
-    else if (fours && L.n_qkv <= 8 * 4 * kSeqThreads) finish(k_seq_qkv_finish8<T, 1>);
+    if (fours && L.n_qkv <= 4 * 4 * kSeqThreads && parts > 1) finish(k_seq_qkv_finish8<T, 4, 3>);
+    else if (fours && L.n_qkv <= 4 * 4 * kSeqThreads) finish(k_seq_qkv_finish8<T, 4, 1>);
+    else if (fours && L.n_qkv <= 8 * 4 * kSeqThreads && parts > 1) finish(k_seq_qkv_finish8<T, 8, 3>);
+    else if (fours && L.n_qkv <= 8 * 4 * kSeqThreads) finish(k_seq_qkv_finish8<T, 8, 1>);
     else if (fours && L.n_qkv <= 16 * 4 * kSeqThreads) finish(k_seq_qkv_finish4<T>);
     else finish(k_seq_qkv_finish<T>);
 

@@ -1,4 +1,6 @@
 """Attention of a portion: keys shared among workgroups, tiles of keys that begin and end anywhere, scores of either sign."""
+import functools
+
 import pytest
 import torch
 
@@ -123,3 +125,28 @@ def test_latent_projection_sizes(name, width, dtype):
     m = kagapel.from_tensors(cfg, w, dtype, capacity=100)
     logits = torch.cat([m.forward(0, toks[:33], 0, range(33)), m.forward(0, toks[33:62], 33, range(29)), m.forward(0, toks[62:], 62, range(28))])
     assert N.error(logits, want) < LIMIT[dtype]
+
+
+# projections of up to 4096, 8192 and more values whose products are split over k, by (values, width): partial rotation, padded heads, values kept by
+# the first layer and mixed in by the second; 2 to 8 parts over these portions (tests/test_seq_plan.py)
+PARTS_ROWS = {4096: (16, 8, 128, 128), 4100: (25, 5, 116, 124), 8192: (32, 16, 128, 128), 8196: (33, 3, 208, 236)}
+PARTS_WIDTHS, PARTS_TOKENS = (1024, 2048), (5, 17, 33)
+
+
+@functools.lru_cache(maxsize=1)
+def in_parts(values, width):
+    cfg = N.model(width, 51, [(N.attn(*PARTS_ROWS[values], rot=rot, v_mix=True), None) for rot in (64, 100)])
+    w, toks = N.weights(cfg, 5), N.prompt(cfg, sum(PARTS_TOKENS), 6)
+    return cfg, w, toks, N.oracle(cfg, w, toks)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("width", PARTS_WIDTHS)
+@pytest.mark.parametrize("values", list(PARTS_ROWS))
+def test_projections_in_parts(values, width, dtype):
+    from clusterfusionplus_amd import nibotar
+    cfg, w, toks, want = in_parts(values, width)
+    m, pos = nibotar.from_tensors(cfg, w, dtype, capacity=100), 0
+    for n in PARTS_TOKENS:
+        assert N.error(m.forward(0, toks[pos:pos + n], pos, range(n)), want[pos:pos + n]) < LIMIT[dtype], n
+        pos += n

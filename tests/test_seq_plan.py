@@ -7,6 +7,7 @@ import pytest
 
 from clusterfusionplus_amd import build
 from tests import seq_plan as P
+from tests import test_gpu_portion_attention as A
 from tests import test_gpu_products as G
 
 ROOM = 1 << 24
@@ -107,6 +108,15 @@ def test_split_rows_of_wide_models():
     for width in G.WIDTHS + [w for w, _ in G.STREAMS]:
         for bf16 in (True, False):
             assert P.product(width, n, ff, bf16, P.room(100, width))[3] > 1, (width, bf16)
+
+
+def test_projections_in_parts():
+    """The parts that every size of row has in its tests: some added in one round of three, some in two."""
+    for values, (heads, kv_heads, dim, vdim) in A.PARTS_ROWS.items():
+        assert heads * dim + kv_heads * (dim + vdim) == values
+        for bf16 in (True, False):
+            parts = {P.product(values, n, width, bf16, P.room(100, values))[3] for n in A.PARTS_TOKENS for width in A.PARTS_WIDTHS}
+            assert 1 not in parts and len(parts) > (values < 8192) and (values > 4100 or max(parts) > 4), (values, bf16, parts)
 
 
 def test_no_split_of_less_than_three_steps_or_more_than_its_room():
