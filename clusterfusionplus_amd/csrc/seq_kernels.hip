@@ -1404,7 +1404,9 @@ void portion_latent(cfpp_seq* s, const LayerPlan& L, int slot, int n, int pos, i
     auto finish = [&](auto kernel, size_t lds) { hipLaunchKernelGGL(kernel, dim3(n), dim3(kSeqThreads), lds, st, f); };
     const bool fours = read % 4 == 0 && made % 4 == 0;
     const size_t lds = (size_t)made * 4 + d.rot_dims * 4;
-    if (fours && read <= 8 * 4 * kSeqThreads && parts > 1) finish(k_seq_latent_finish4<T, 8, 3>, lds);
+    if (fours && read <= 4 * 4 * kSeqThreads && parts > 1) finish(k_seq_latent_finish4<T, 4, 3>, lds);
+    else if (fours && read <= 4 * 4 * kSeqThreads) finish(k_seq_latent_finish4<T, 4, 1>, lds);
+    else if (fours && read <= 8 * 4 * kSeqThreads && parts > 1) finish(k_seq_latent_finish4<T, 8, 3>, lds);
     else if (fours && read <= 8 * 4 * kSeqThreads) finish(k_seq_latent_finish4<T, 8, 1>, lds);
     else if (fours && read <= 12 * 4 * kSeqThreads) finish(k_seq_latent_finish4<T, 12, 1>, lds);
     else finish(k_seq_latent_finish<T>, 0);

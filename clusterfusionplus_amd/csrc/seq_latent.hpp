@@ -83,7 +83,8 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_latent_finish(SeqLatentFini
 
 // The same where the row is whole groups of four values, up to 1024 U of them: everything is requested at once (of C parts together), and the
 // row is read from LDS, where it took three or four round trips.  Gates are read only where they come in parts, and their sum goes back.
-// 8000 tokens of 6720 values and 4096 gates: 100 -> 71 us for 330 MB; 150 tokens of 3648 in parts: 8.1 -> 6.3.
+// 8000 tokens of 6720 values and 4096 gates: 100 -> 71 us for 330 MB.  U = 4 where the row fits, since places behind its end are requested like others:
+// 150 tokens of 3648 in parts 6.4 us, with 8 groups 5.6, with 4 5.0; 100 of 1120 in parts 4.5, 5.6 and 4.7.
 template <typename T, int U, int C>
 __global__ __launch_bounds__(kSeqThreads) void k_seq_latent_finish4(SeqLatentFinish a) {
     __shared__ float red[kSeqWaves];

@@ -108,9 +108,9 @@ def test_columns_in_blocks_of_32(name):
         assert N.error(got, M.oracle(cfg, w, toks)) < LIMIT[torch.bfloat16]
 
 
-# latent projections of up to 8192 and 12288 values, and of more; in one part (64 columns) and in several (512); rows and gates that are no whole groups
-# of four; a layer that reads the latents of another
-LATENTS = {"6k": (24, 128, 64, 56, 48), "12k": (48, 128, 64, 56, 48), "16k": (64, 128, 64, 56, 48), "no_fours": (3, 41, 16, 55, 49), "gates_no_fours": (3, 44, 16, 55, 48)}
+# latent projections of up to 4096, 8192 and 12288 values, and of more; in one part (64 columns) and in several (512); rows and gates that are no whole
+# groups of four; a layer that reads the latents of another
+LATENTS = {"1k": (5, 128, 64, 56, 48), "4k": (19, 128, 64, 56, 384), "4k_more": (19, 128, 64, 56, 388), "6k": (24, 128, 64, 56, 48), "12k": (48, 128, 64, 56, 48), "16k": (64, 128, 64, 56, 48), "no_fours": (3, 41, 16, 55, 49), "gates_no_fours": (3, 44, 16, 55, 48)}
 
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
@@ -119,7 +119,7 @@ LATENTS = {"6k": (24, 128, 64, 56, 48), "12k": (48, 128, 64, 56, 48), "16k": (64
 def test_latent_projection_sizes(name, width, dtype):
     from clusterfusionplus_amd import kagapel
     dims = LATENTS[name]
-    cfg = K.model(width, 51, [K.gated(*dims), K.sunk(*dims, kv_from=0), K.gated(*dims)])
+    cfg = K.model(width, 51, [K.gated(*dims), K.sunk(*dims, kv_from=0), K.gated(*dims), K.sunk(*dims)])
     w, toks = K.weights(cfg, 5), K.prompt(cfg, 90, 6)
     want = K.oracle(cfg, w, toks)
     m = kagapel.from_tensors(cfg, w, dtype, capacity=100)
