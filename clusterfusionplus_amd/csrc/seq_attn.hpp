@@ -323,16 +323,24 @@ __global__ __launch_bounds__(kSeqThreads, (NT <= 128 ? 2 : 1)) void k_seq_attn(S
                     __builtin_amdgcn_sched_barrier(0);
                 }
             } else {
+                // Values of four keys are read two products ahead: left to the compiler, each pair of reads is waited for right where it is used (700
+                // tokens at 1990, 16 / 4 heads of 128: 223 us with all reads hoisted, 232 with none, 207 two ahead).
+                constexpr int KV = KT / C, kSteps = NT / C * KV;
+                f32x4 f[3];
+                auto read_values = [&](int i) __attribute__((always_inline)) {
+                    const char* b = tile + (vat ^ (i / KV * L::block * 16)) + i % KV * C * L::vbytes;
 #pragma unroll
-                for (int i = 0; i < NT / C; ++i)
+                    for (int j = 0; j < 4; ++j) f[i % 3][j] = *reinterpret_cast<const float*>(b + j * L::vbytes);
+                };
+                read_values(0);
+                read_values(1);
 #pragma unroll
-                    for (int h = 0; h < KT / C; ++h) {
-                        const char* b = tile + (vat ^ (i * L::block * 16)) + h * C * L::vbytes;
-                        f32x4 f;
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) f[j] = *reinterpret_cast<const float*>(b + j * L::vbytes);
-                        acc[i] = attn_mma<T>(__builtin_bit_cast(u32x4, f), __builtin_bit_cast(u32x4, w[h]), acc[i]);
-                    }
+                for (int i = 0; i < kSteps; ++i) {
+                    if (i + 2 < kSteps) read_values(i + 2);
+                    __builtin_amdgcn_sched_barrier(0);
+                    acc[i / KV] = attn_mma<T>(__builtin_bit_cast(u32x4, f[i % 3]), __builtin_bit_cast(u32x4, w[i % KV]), acc[i / KV]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             }
         }
         t = tn;

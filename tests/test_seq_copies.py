@@ -131,6 +131,16 @@ def test_rings_step_on_without_a_jump(library):
         assert [t for t in code[copy:read] if t.startswith(("s_branch", "s_cbranch"))] == [], name
 
 
+def test_products_of_attention_have_their_reads_in_flight(library):
+    """No product of a portion's attention waits for every read of LDS, but where a phase begins or ends."""
+    kernels = {name: code for name, code in library.items() if re.search(r"k_seq_attnI", name)}
+    assert len(kernels) == 24
+    for name, code in kernels.items():
+        products = [i for i, t in enumerate(code) if t.startswith("v_mfma")]
+        waits = [i for i in products if any(re.match(r"s_waitcnt.*lgkmcnt\(0\)", t) for t in code[i - 2:i])]
+        assert len(products) >= 24 and len(waits) <= 8, (name, len(products), len(waits))
+
+
 @pytest.mark.parametrize("kind", [0, 1, 2], ids=["at", "once", "from"])
 def test_compiler_knows_that_m0_is_written(kernels, kind):
     """Every copy is preceded by a write of m0 of its own, and at least one instruction lies between them."""
