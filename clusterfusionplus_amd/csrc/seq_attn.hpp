@@ -3,6 +3,7 @@
 #include <type_traits>
 
 #include "seq_device.hpp"
+#include "seq_plan.hpp"
 
 namespace cfpp {
 
@@ -19,9 +20,9 @@ struct SeqAttn {
     char* out;
     const float* sink;       // nullable
     const float* gate;       // nullable: [T][ldg], the outputs are multiplied by its sigmoid
-    int T, H, R, qrow, krow, vrow, V, vtiles, pos0, chunk, cap, rows, ldo, k_split, runits, rrow, ldg;
+    int T, H, R, G, qrow, krow, vrow, V, vtiles, pos0, chunk, cap, rows, ldo, k_split, runits, rrow, ldg;
     float scale_log2;
-    int splits;
+    int splits, up;          // up: rows of workgroups that go from the last block of columns on (attn_block)
     float *part, *ml;        // splits > 1: [splits][T][H][16 vtiles], [splits][T][H][2]
 };
 template <int UN> __device__ __forceinline__ int swz_key(int row) { return UN % 16 ? (row >> 1) & 7 : row & 15; }
@@ -97,11 +98,13 @@ __global__ __launch_bounds__(kSeqThreads, (NT <= 128 ? 2 : 1)) void k_seq_attn(S
     constexpr int KT = L::keys, G = kWave / C, KS = L::ku / G, NE = C * C / kWave, kCols = C * kSeqWaves;      // lanes of a column, steps of a score, outputs of a lane
     extern __shared__ __align__(1024) char lds[];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane % C, g = lane / C;
-    // The longest walks of all key heads first, so that the short ones fill the chip's last moments (head by head, a quarter of the compute
-    // units' time was a tail: 8000 tokens, 32 heads of 192 and 128: 1264 -> 956 us; 2048 tokens, 128 and 128: 104 -> 86 us); and where the heads are a
-    // multiple of eight, all workgroups of a head are on one XCD and walk its keys side by side.
-    const int ncols = a.T * a.R, gx = (ncols + kCols - 1) / kCols, heads = a.H / a.R, bx = blockIdx.x / heads, gq = blockIdx.x - bx * heads;
-    const int c0 = (gx - 1 - bx) * kCols;
+    // Workgroups go row by row, a row being the same columns of all key heads and splits, with the longest walks first (attn_block), so that the short
+    // ones fill the chip's last moments (head by head, a quarter of the compute units' time was a tail: 8000 tokens, 32 heads of 192 and 128: 1264 -> 956 us;
+    // 2048 tokens, 128 and 128: 104 -> 86 us).  Where the heads are a multiple of eight, all workgroups of a head are on one XCD and walk its keys
+    // side by side.
+    // (one split: the grid has one dimension, which is not limited to 65535)
+    const int ncols = a.T * a.R, rows = (ncols + kCols - 1) / kCols, part = blockIdx.x / (unsigned)a.G, gq = blockIdx.x - part * a.G;
+    const int split = a.splits > 1 ? part : 0, c0 = attn_block(a.splits > 1 ? blockIdx.y : part, rows, a.up) * kCols;
 
     // (its sign goes to the query; not zero, so that it keeps the scores of keys that are not seen at -infinity; NaN stays NaN)
     const float size = fabsf(a.scale_log2), scale = size < 1e-30f ? 1e-30f : size;
@@ -131,7 +134,7 @@ __global__ __launch_bounds__(kSeqThreads, (NT <= 128 ? 2 : 1)) void k_seq_attn(S
 
     // tiles: [k_first, k_split) in the cache, then [k_split, k_end) in the buffer; this split's are t0 .. t1 - 1
     const int in_cache = max(0, min(k_end, a.k_split) - k_first), n_cached = (in_cache + KT - 1) / KT, new_first = max(k_first, a.k_split);
-    const int ntiles = n_cached + (max(0, k_end - new_first) + KT - 1) / KT, split = blockIdx.y;
+    const int ntiles = n_cached + (max(0, k_end - new_first) + KT - 1) / KT;
     const int t0 = mul_div(ntiles, split, a.splits), t1 = mul_div(ntiles, split + 1, a.splits);
     struct Tile { int k0, hi; const char *k, *v; };      // first key, end of its part, its rows
     auto tile_at = [&](int i) {

@@ -1260,15 +1260,19 @@ template <typename T, int NK, int NT>
 void launch_attn(SeqAttn a, int G, int cus, size_t room, float* part, hipStream_t st) {
     const int cols = a.T * a.R;
     const AttnPlan plan = plan_attn({a.T, a.R, G, a.pos0, a.chunk, AttnTile<T, NK, NT, 16>::keys, sizeof(T) == 2, NT <= 128 ? 2 : 1, (size_t)a.T * a.H * (a.vtiles * 16 + 2)}, cus, room);
+    a.G = G;
     a.splits = plan.splits;
+    a.up = plan.up;
     a.part = part;
     a.ml = part + (size_t)a.splits * a.T * a.H * a.vtiles * 16;
     auto go = [&](auto n, auto sh) {
         constexpr int C = decltype(n)::value;
         constexpr bool SH = decltype(sh)::value;
         const size_t lds = 2 * AttnTile<T, NK, NT, C>::size;
+        const int rows = ceil_div(cols, C * kSeqWaves);
+        const dim3 grid = a.splits > 1 ? dim3(G * a.splits, rows) : dim3(G * rows);
         allow_lds(k_seq_attn<T, NK, NT, C, SH>, lds);
-        hipLaunchKernelGGL((k_seq_attn<T, NK, NT, C, SH>), dim3(ceil_div(cols, C * kSeqWaves) * G, a.splits), dim3(kSeqThreads), lds, st, a);
+        hipLaunchKernelGGL((k_seq_attn<T, NK, NT, C, SH>), grid, dim3(kSeqThreads), lds, st, a);
     };
     auto pick = [&](auto sh) {
         if constexpr (sizeof(T) == 2) {

@@ -125,13 +125,24 @@ struct AttnSizes {
 // compute unit, with two tiles at least in each split of the longest walk, which begins at the chunk of the portion's first token (that
 // chunk counts and not the context: 37 tokens just behind a chunk of 8192 see one tile; shared by 16 splits, eight layers of 32 / 8 heads
 // of 128 took 1005 us, and take 957).
-struct AttnPlan { bool two; int splits; };
+//
+// The order of the workgroups.  A row of them is the same columns of all key heads and splits; rows go from the last block of columns, which walks
+// the most keys, to the first.  Where all are resident, two per compute unit, workgroups i and i + `cus` share one (the hardware places them in turn:
+// read from its registers, 512 workgroups of 64 KB), so the rows behind the first `cus` workgroups go upwards, and a long walk has a short one beside
+// it.  In us, head by head / downwards only / so, in fp32: 16 heads of 192 and 128, 1000 tokens 101 / 94 / 63; 32 / 8 heads of 128, 1000 tokens 129 /
+// 107 / 85; 10 / 5 heads of 64, 1500 tokens in two splits 52 / 57 / 43; 12 / 4 heads of 96 and 80, 700 tokens in three 38 / 43 / 31; bf16, where
+// a walk of so few workgroups is short: equal to 1 %.  With more workgroups the longest come first, since what is left over goes where a short walk
+// has ended (upwards in the second round too, 544 workgroups in bf16 take 217 us instead of 184).
+struct AttnPlan { bool two; int splits, up; };       // up: rows that go down
+constexpr int attn_block(int row, int rows, int up) { return row < up ? rows - 1 - row : row - up; }
 inline AttnPlan plan_attn(const AttnSizes& a, int cus, size_t room) {
     const int cols = a.T * a.R, behind = a.pos0 + a.T - (a.chunk > 0 ? a.pos0 / a.chunk * a.chunk : 0);
     const int tiles = ceil_div(a.chunk > 0 ? std::min(behind, a.chunk) : behind, a.keys);
     const bool two = a.pairs && ceil_div(cols, 128) * a.G >= 2 * cus;
     const int wgs = ceil_div(cols, two ? 128 : 64) * a.G;
-    return {two, std::max(1, (int)std::min<size_t>({(size_t)16, (size_t)(a.per_cu * cus / wgs), (size_t)(tiles / 2), room / a.floats}))};
+    const int splits = std::max(1, (int)std::min<size_t>({(size_t)16, (size_t)(a.per_cu * cus / wgs), (size_t)(tiles / 2), room / a.floats}));
+    const bool resident = a.per_cu >= 2 && wgs * splits <= 2 * cus;
+    return {two, splits, resident ? std::max(1, cus / (a.G * splits)) : wgs / a.G};
 }
 
 }  // namespace cfpp

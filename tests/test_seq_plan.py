@@ -46,6 +46,23 @@ def test_every_split_of_the_longest_walk_has_two_tiles():
         assert n == 1 or n <= max(walks(T, R, pos, chunk, keys, columns)) // 2, (T, R, G, pos, chunk, keys, n)
 
 
+def test_long_walks_have_short_ones_beside_them():
+    """Every row of workgroups is there once.  Workgroups i and i + 256 share a compute unit: where all are resident, two such walks are little longer
+    than the longest alone; where more follow, the longest are first."""
+    rng = random.Random(4)
+    for T, R, G, keys in [(1000, 1, 16, 32), (1000, 4, 8, 32), (1500, 2, 5, 32), (700, 3, 4, 32), (2048, 1, 4, 64), (700, 1, 12, 64), (3000, 1, 300, 64)] + \
+            [(rng.randint(2, 4000), rng.choice([1, 2, 4, 8]), rng.choice([1, 2, 3, 5, 8, 12, 16, 32, 40]), rng.choice([32, 64])) for _ in range(300)]:
+        n, columns, order = P.attention_plan(T, R, G, 0, 0, keys, T * R * G * 130, ROOM)
+        rows = len(order)
+        assert sorted(order) == list(range(rows)), (T, R, G, keys)
+        lengths = [block + 1 for block in order for _ in range(G * n)]
+        if len(lengths) > 2 * P.CUS:
+            assert n == 1 and lengths == sorted(lengths, reverse=True), (T, R, G, keys)
+        else:
+            together = [lengths[i] + sum(lengths[i + P.CUS:i + P.CUS + 1]) for i in range(min(P.CUS, len(lengths)))]
+            assert max(together) <= rows + 2, (T, R, G, keys, max(together), rows)
+
+
 # ---- the tiles that the products' tests are for --------------------------------------------------------------------------
 
 @pytest.mark.parametrize("sizes, tile", list(zip(G.DENSE, G.DENSE_TILES)), ids=str)
