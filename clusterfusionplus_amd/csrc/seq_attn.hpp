@@ -22,7 +22,7 @@ struct SeqAttn {
     const float* gate;       // nullable: [T][ldg], the outputs are multiplied by its sigmoid
     int T, H, R, G, qrow, krow, vrow, V, vtiles, pos0, chunk, cap, rows, ldo, k_split, runits, rrow, ldg;
     float scale_log2;
-    int splits, up;          // up: rows of workgroups that go from the last block of columns on (attn_block)
+    int splits, up, swap;    // (of attn_block)
     float *part, *ml;        // splits > 1: [splits][T][H][16 vtiles], [splits][T][H][2]
 };
 template <int UN> __device__ __forceinline__ int swz_key(int row) { return UN % 16 ? (row >> 1) & 7 : row & 15; }
@@ -104,7 +104,7 @@ __global__ __launch_bounds__(kSeqThreads, (NT <= 128 ? 2 : 1)) void k_seq_attn(S
     // side by side.
     // (one split: the grid has one dimension, which is not limited to 65535)
     const int ncols = a.T * a.R, rows = (ncols + kCols - 1) / kCols, part = blockIdx.x / (unsigned)a.G, gq = blockIdx.x - part * a.G;
-    const int split = a.splits > 1 ? part : 0, c0 = attn_block(a.splits > 1 ? blockIdx.y : part, rows, a.up) * kCols;
+    const int split = a.splits > 1 ? part : 0, c0 = attn_block(a.splits > 1 ? blockIdx.y : part, rows, a.up, a.swap) * kCols;
 
     // (its sign goes to the query; not zero, so that it keeps the scores of keys that are not seen at -infinity; NaN stays NaN)
     const float size = fabsf(a.scale_log2), scale = size < 1e-30f ? 1e-30f : size;

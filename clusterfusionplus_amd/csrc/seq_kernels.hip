@@ -1263,6 +1263,7 @@ void launch_attn(SeqAttn a, int G, int cus, size_t room, float* part, hipStream_
     a.G = G;
     a.splits = plan.splits;
     a.up = plan.up;
+    a.swap = plan.swap;
     a.part = part;
     a.ml = part + (size_t)a.splits * a.T * a.H * a.vtiles * 16;
     auto go = [&](auto n, auto sh) {

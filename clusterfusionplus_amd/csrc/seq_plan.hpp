@@ -131,18 +131,27 @@ struct AttnSizes {
 // read from its registers, 512 workgroups of 64 KB), so the rows behind the first `cus` workgroups go upwards, and a long walk has a short one beside
 // it.  In us, head by head / downwards only / so, in fp32: 16 heads of 192 and 128, 1000 tokens 101 / 94 / 63; 32 / 8 heads of 128, 1000 tokens 129 /
 // 107 / 85; 10 / 5 heads of 64, 1500 tokens in two splits 52 / 57 / 43; 12 / 4 heads of 96 and 80, 700 tokens in three 38 / 43 / 31; bf16, where
-// a walk of so few workgroups is short: equal to 1 %.  With more workgroups the longest come first, since what is left over goes where a short walk
-// has ended (upwards in the second round too, 544 workgroups in bf16 take 217 us instead of 184).
-struct AttnPlan { bool two; int splits, up; };       // up: rows that go down
-constexpr int attn_block(int row, int rows, int up) { return row < up ? rows - 1 - row : row - up; }
+// a walk of so few workgroups is short: equal to 1 %.  With more workgroups the longest come first, since what is left over goes where a walk has
+// ended.  Two that share a compute unit should not end together: then two that are left over go there, and other units stay idle.  The older one
+// of the two is served first, so a somewhat longer one ends with the younger (768 workgroups, 1500 tokens at 1990, fp32: on 128 units within 10 us,
+// and four workgroups on each of these, two on the others).  So where there is less than one left over per unit, and the walks are alike, the
+// younger are the longer ones: 32 heads of 192 and 128, 1150 tokens at 1990, fp32 731 -> 585 us, 1500 tokens 848 -> 701 (610 and 729 when reads
+// of values were waited for and the older one ended first), bf16 133 -> 116 and 153 -> 139.  Alike: at least half as many keys in front of the portion
+// as in it, and no chunk that begins inside (2100 tokens at 0 in bf16 would take 83 us instead of 73).
+struct AttnPlan { bool two; int splits, up, swap; };         // rows that go down; so many rows come behind as many that follow them
+constexpr int attn_block(int row, int rows, int up, int swap) {
+    return row >= up ? row - up : rows - 1 - (row < swap ? row + swap : row < 2 * swap ? row - swap : row);
+}
 inline AttnPlan plan_attn(const AttnSizes& a, int cus, size_t room) {
     const int cols = a.T * a.R, behind = a.pos0 + a.T - (a.chunk > 0 ? a.pos0 / a.chunk * a.chunk : 0);
     const int tiles = ceil_div(a.chunk > 0 ? std::min(behind, a.chunk) : behind, a.keys);
     const bool two = a.pairs && ceil_div(cols, 128) * a.G >= 2 * cus;
     const int wgs = ceil_div(cols, two ? 128 : 64) * a.G;
     const int splits = std::max(1, (int)std::min<size_t>({(size_t)16, (size_t)(a.per_cu * cus / wgs), (size_t)(tiles / 2), room / a.floats}));
-    const bool resident = a.per_cu >= 2 && wgs * splits <= 2 * cus;
-    return {two, splits, resident ? std::max(1, cus / (a.G * splits)) : wgs / a.G};
+    const int rows = wgs / a.G, some = std::max(1, cus / (a.G * splits)), total = wgs * splits;
+    if (a.per_cu >= 2 && total <= 2 * cus) return {two, splits, some, 0};
+    const bool alike = 2 * (behind - a.T) >= a.T && (a.chunk == 0 || behind <= a.chunk);
+    return {two, splits, rows, a.per_cu >= 2 && total <= 3 * cus && alike ? some : 0};
 }
 
 }  // namespace cfpp

@@ -12,13 +12,14 @@ SOURCE = """
 #include "seq_plan.hpp"
 using namespace cfpp;
 static int code(int shape, int splits, bool bf16) { const GemmShape& s = shapes_of(bf16)[shape]; return ((s.rows * 1024 + s.tokens) * 4 + s.resident) * 32 + splits; }
-extern "C" int attn(int T, int R, int G, int pos0, int chunk, int keys, int bf16, int per_cu, long floats, int cus, long room, int* columns, int* up) {
+extern "C" int attn(int T, int R, int G, int pos0, int chunk, int keys, int bf16, int per_cu, long floats, int cus, long room, int* columns, int* up, int* swap) {
     const AttnPlan p = plan_attn({T, R, G, pos0, chunk, keys, bf16 != 0, per_cu, (size_t)floats}, cus, (size_t)room);
     *columns = p.two ? 128 : 64;
     *up = p.up;
+    *swap = p.swap;
     return p.splits;
 }
-extern "C" int block(int row, int rows, int up) { return attn_block(row, rows, up); }
+extern "C" int block(int row, int rows, int up, int swap) { return attn_block(row, rows, up, swap); }
 extern "C" int product(int n, int m, int kbytes, int ldy, long room, int bf16, int cus) {
     const GemmPlan p = plan_gemm({n, m, kbytes, ldy, (size_t)room}, bf16 != 0, cus);
     return code(p.shape, p.splits, bf16);
@@ -42,8 +43,8 @@ def lib():
         subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", f"-I{build.CSRC}", src, "-o", so], check=True)
         lib = ctypes.CDLL(so)
     i, l, p = ctypes.c_int, ctypes.c_long, ctypes.POINTER(ctypes.c_int)
-    lib.attn.argtypes = [i] * 8 + [l, i, l, p, p]
-    lib.block.argtypes = [i] * 3
+    lib.attn.argtypes = [i] * 8 + [l, i, l, p, p, p]
+    lib.block.argtypes = [i] * 4
     lib.product.argtypes = [i] * 4 + [l, i, i]
     lib.experts.argtypes = [i] * 7 + [p]
     lib.tile.argtypes = [i, i]
@@ -58,10 +59,10 @@ def attention(T, R, G, pos, chunk, keys, floats, room, per_cu=2):
 
 def attention_plan(T, R, G, pos, chunk, keys, floats, room, per_cu=2):
     """(splits of the keys, columns of a workgroup, blocks of columns in the order of the workgroups' rows)"""
-    columns, up = ctypes.c_int(), ctypes.c_int()
-    splits = lib().attn(T, R, G, pos, chunk, keys, keys == 64, per_cu, floats, CUS, room, ctypes.byref(columns), ctypes.byref(up))
+    columns, up, swap = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+    splits = lib().attn(T, R, G, pos, chunk, keys, keys == 64, per_cu, floats, CUS, room, ctypes.byref(columns), ctypes.byref(up), ctypes.byref(swap))
     rows = -(-T * R // columns.value)
-    return splits, columns.value, [lib().block(row, rows, up.value) for row in range(rows)]
+    return splits, columns.value, [lib().block(row, rows, up.value, swap.value) for row in range(rows)]
 
 
 def _decode(code):

@@ -108,6 +108,24 @@ def test_columns_in_blocks_of_32(name):
         assert N.error(got, M.oracle(cfg, w, toks)) < LIMIT[torch.bfloat16]
 
 
+# more workgroups than are resident, by less than one per compute unit: 10 rows of 64 heads; 5 of them in front
+LEFT_OVER = {"grouped": (N, N.attn(64, 64, 40, 56, rot=8)), "chunks": (N, N.attn(64, 64, 40, 56, chunk=1000)), "latent": (K, K.sunk(64, 40, 16, 56, 48)), "middle": (N, N.attn(64, 64, 128, 128))}
+LEFT_OVER_TOKENS = (320, 625)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("name", list(LEFT_OVER))
+def test_workgroups_left_over(name, dtype):
+    from clusterfusionplus_amd import kagapel, nibotar
+    M, mixer = LEFT_OVER[name]
+    first, n = LEFT_OVER_TOKENS
+    cfg = M.model(64, 51, [mixer], positions=1000) if M is K else M.model(64, 51, [(mixer, None)])
+    w, toks = M.weights(cfg, 5), M.prompt(cfg, first + n, 6)
+    m = (nibotar if M is N else kagapel).from_tensors(cfg, w, dtype, capacity=first + n)
+    got = torch.cat([m.forward(0, toks[:first], 0, range(first)), m.forward(0, toks[first:], first, range(n))])
+    assert N.error(got, M.oracle(cfg, w, toks)) < LIMIT[dtype]
+
+
 # latent projections of up to 4096, 8192 and 12288 values, and of more; in one part (64 columns) and in several (512); rows and gates that are no whole
 # groups of four; a layer that reads the latents of another
 LATENTS = {"1k": (5, 128, 64, 56, 48), "4k": (19, 128, 64, 56, 384), "4k_more": (19, 128, 64, 56, 388), "6k": (24, 128, 64, 56, 48), "12k": (48, 128, 64, 56, 48), "16k": (64, 128, 64, 56, 48), "no_fours": (3, 41, 16, 55, 49), "gates_no_fours": (3, 44, 16, 55, 48)}

@@ -46,21 +46,38 @@ def test_every_split_of_the_longest_walk_has_two_tiles():
         assert n == 1 or n <= max(walks(T, R, pos, chunk, keys, columns)) // 2, (T, R, G, pos, chunk, keys, n)
 
 
-def test_long_walks_have_short_ones_beside_them():
+def test_order_of_the_workgroups():
     """Every row of workgroups is there once.  Workgroups i and i + 256 share a compute unit: where all are resident, two such walks are little longer
-    than the longest alone; where more follow, the longest are first."""
-    rng = random.Random(4)
-    for T, R, G, keys in [(1000, 1, 16, 32), (1000, 4, 8, 32), (1500, 2, 5, 32), (700, 3, 4, 32), (2048, 1, 4, 64), (700, 1, 12, 64), (3000, 1, 300, 64)] + \
-            [(rng.randint(2, 4000), rng.choice([1, 2, 4, 8]), rng.choice([1, 2, 3, 5, 8, 12, 16, 32, 40]), rng.choice([32, 64])) for _ in range(300)]:
-        n, columns, order = P.attention_plan(T, R, G, 0, 0, keys, T * R * G * 130, ROOM)
-        rows = len(order)
-        assert sorted(order) == list(range(rows)), (T, R, G, keys)
-        lengths = [block + 1 for block in order for _ in range(G * n)]
-        if len(lengths) > 2 * P.CUS:
-            assert n == 1 and lengths == sorted(lengths, reverse=True), (T, R, G, keys)
+    than the longest alone; where less than one per unit is left over and walks are alike, the younger of the two is the longer one and the shortest
+    are left over; otherwise the longest are first."""
+    rng, kinds = random.Random(4), set()
+    for T, R, G, keys, pos, chunk in [(1000, 1, 16, 32, 0, 0), (1000, 4, 8, 32, 0, 0), (1500, 2, 5, 32, 0, 0), (700, 3, 4, 32, 0, 0), (3000, 1, 300, 64, 0, 0), (1150, 1, 32, 32, 1990, 0),
+                                      (1500, 1, 32, 32, 1990, 0), (1500, 1, 32, 32, 1990, 3000), (1500, 1, 32, 32, 1990, 3490), (1500, 1, 32, 32, 749, 0), (1100, 1, 40, 64, 550, 0), (66, 1, 300, 64, 64, 0)] + \
+            [(rng.randint(2, 4000), rng.choice([1, 2, 4, 8]), rng.choice([1, 2, 3, 5, 8, 12, 16, 32, 40]), rng.choice([32, 64]), rng.choice([0, 100, 1000, 3000]), rng.choice([0, 0, 2000, 8192])) for _ in range(600)]:
+        n, columns, order = P.attention_plan(T, R, G, pos, chunk, keys, T * R * G * 130, ROOM)
+        rows, what = len(order), (T, R, G, keys, pos, chunk)
+        assert sorted(order) == list(range(rows)), what
+        blocks = [block for block in order for _ in range(G * n)]
+        alike = 2 * (pos - (pos // chunk * chunk if chunk else 0)) >= T and not (chunk and pos // chunk != (pos + T - 1) // chunk)
+        if len(blocks) <= 2 * P.CUS:
+            kinds.add("resident")
+            assert max(blocks[i] + sum(blocks[i + P.CUS:i + P.CUS + 1]) for i in range(min(P.CUS, len(blocks)))) <= rows, what
+        elif len(blocks) <= 3 * P.CUS and alike:
+            kinds.add("left over")
+            some = P.CUS // G * G or G
+            assert n == 1 and all(blocks[i] < blocks[i + some] for i in range(some)) and max(blocks[2 * some:], default=-1) < min(blocks[:2 * some]), what
         else:
-            together = [lengths[i] + sum(lengths[i + P.CUS:i + P.CUS + 1]) for i in range(min(P.CUS, len(lengths)))]
-            assert max(together) <= rows + 2, (T, R, G, keys, max(together), rows)
+            kinds.add("many")
+            assert n == 1 and blocks == sorted(blocks, reverse=True), what
+    assert len(kinds) == 3
+
+
+def test_attention_with_workgroups_left_over():
+    """What its test is for."""
+    first, n = A.LEFT_OVER_TOKENS
+    for keys in (32, 64):
+        for chunk in (0, 1000):
+            assert P.attention_plan(n, 1, 64, first, chunk, keys, n * 64 * 130, ROOM) == (1, 64, [5, 4, 3, 2, 9, 8, 7, 6, 1, 0])
 
 
 # ---- the tiles that the products' tests are for --------------------------------------------------------------------------
