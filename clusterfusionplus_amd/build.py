@@ -93,7 +93,7 @@ LDS_BYTES = 160 * 1024       # of a compute unit
 
 def launch_lds(kernel):
     """(LDS bytes, waves) of a workgroup of a kernel whose LDS is set at its launch, as the launch sites in csrc/seq_kernels.hip do, from
-    the kernel's name and template arguments.  Bytes None: they depend on the model.  None: the compiler knows them."""
+    the kernel's name and template arguments (the most that it takes, where a row's length counts).  Bytes None: they depend on the model.  None: the compiler knows them."""
     import re
     m = re.match(r"(k_seq_\w+)(?:<(.*)>)?$", kernel)
     if m is None:
@@ -111,6 +111,8 @@ def launch_lds(kernel):
     if name == "k_seq_latent_attn":              # three tiles of latents with the rotated part, in whole copies of 4 KB
         units = (num[0] + 128) * size // 16 + 1
         return 3 * -(-(32 if size == 2 else 16) * units // 256) * 4096, 4
+    if name == "k_seq_latent_finish4":           # the row in front of its gates, up to 1024 values per group of a thread, and a position's pairs
+        return 1024 * num[0] * 4 + 512, 4
     if name in ("k_seq_postnorm", "k_seq_streams", "k_seq_gemv", "k_seq_route"):
         return None, 16 if name == "k_seq_route" else 4
     return None

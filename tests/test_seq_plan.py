@@ -179,6 +179,7 @@ def test_workgroups_that_share_a_compute_unit_fit_its_memory():
 
 def test_lds_of_launches():
     assert build.launch_lds("k_seq_gemm<bf16, 96, 128, 2, 2, 5, 0>") == (143360, 4) and build.launch_lds("k_seq_gemm8<3>") == (131072, 8)
-    assert build.launch_lds("k_seq_attn<bf16, 192, 128, 2, true>") == (81920, 4) and build.launch_lds("k_seq_attn<float, 256, 256, 1, false>") == (131072, 4)
+    assert build.launch_lds("k_seq_attn<bf16, 192, 128, 32, true>") == (81920, 4) and build.launch_lds("k_seq_attn<float, 256, 256, 16, false>") == (131072, 4)
     assert build.launch_lds("k_seq_latent_attn<bf16, 512, 4>") == (135168, 4)
+    assert build.launch_lds("k_seq_latent_finish4<bf16, 12, 1>") == (49664, 4) and build.launch_lds("k_seq_latent_finish4<float, 4, 3>") == (16896, 4)
     assert build.launch_lds("k_seq_postnorm<bf16>")[0] is None and build.launch_lds("k_seq_postnorm4<bf16, 8>") is None and build.launch_lds("k_fused<1>") is None
