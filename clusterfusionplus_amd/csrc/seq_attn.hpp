@@ -104,7 +104,8 @@ __global__ __launch_bounds__(kSeqThreads, (NT <= 128 ? 2 : 1)) void k_seq_attn(S
     // side by side.
     // (one split: the grid has one dimension, which is not limited to 65535)
     const int ncols = a.T * a.R, rows = (ncols + kCols - 1) / kCols, part = blockIdx.x / (unsigned)a.G, gq = blockIdx.x - part * a.G;
-    const int split = a.splits > 1 ? part : 0, c0 = attn_block(a.splits > 1 ? blockIdx.y : part, rows, a.up, a.swap) * kCols;
+    const bool in_parts = C == 16 && a.splits > 1;       // (portions with blocks of 32 fill the chip)
+    const int split = in_parts ? part : 0, c0 = attn_block(in_parts ? blockIdx.y : part, rows, a.up, a.swap) * kCols;
 
     // (its sign goes to the query; not zero, so that it keeps the scores of keys that are not seen at -infinity; NaN stays NaN)
     const float size = fabsf(a.scale_log2), scale = size < 1e-30f ? 1e-30f : size;
@@ -135,7 +136,7 @@ __global__ __launch_bounds__(kSeqThreads, (NT <= 128 ? 2 : 1)) void k_seq_attn(S
     // tiles: [k_first, k_split) in the cache, then [k_split, k_end) in the buffer; this split's are t0 .. t1 - 1
     const int in_cache = max(0, min(k_end, a.k_split) - k_first), n_cached = (in_cache + KT - 1) / KT, new_first = max(k_first, a.k_split);
     const int ntiles = n_cached + (max(0, k_end - new_first) + KT - 1) / KT;
-    const int t0 = mul_div(ntiles, split, a.splits), t1 = mul_div(ntiles, split + 1, a.splits);
+    const int t0 = in_parts ? mul_div(ntiles, split, a.splits) : 0, t1 = in_parts ? mul_div(ntiles, split + 1, a.splits) : ntiles;
     struct Tile { int k0, hi; const char *k, *v; };      // first key, end of its part, its rows
     auto tile_at = [&](int i) {
         const bool cached = i < n_cached;
@@ -352,7 +353,7 @@ __global__ __launch_bounds__(kSeqThreads, (NT <= 128 ? 2 : 1)) void k_seq_attn(S
     if (c0 + wave * C + col >= ncols) return;
     auto four = [&](int v) { return f32x4{acc[v / C][v % C / 8 * 4], acc[v / C][v % C / 8 * 4 + 1], acc[v / C][v % C / 8 * 4 + 2], acc[v / C][v % C / 8 * 4 + 3]}; };      // outputs v + 4 g ..
     constexpr int kOut = 4 * G;                          // outputs of a column from one of a lane's four to the next
-    if (a.splits > 1) {
+    if (in_parts) {
         const size_t row = ((size_t)split * a.T + tok) * a.H + head;
         if (g == 0) *reinterpret_cast<float2*>(a.ml + row * 2) = make_float2(m, lw);
         float* p = a.part + row * (a.vtiles * 16) + g * 4;

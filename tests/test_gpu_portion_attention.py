@@ -87,11 +87,12 @@ def test_projection_sizes(name, dtype):
     assert N.error(logits, want) < LIMIT[dtype]
 
 
-# enough columns for blocks of 32 (512 workgroups of 128): every size of tile, heads that share keys, chunks, a last block that is not full, keys of
+# enough columns for blocks of 32 (512 workgroups of 128; tests/test_seq_plan.py): every size of tile, heads that share keys, chunks, a last block that is not full, keys of
 # the portion and of the context before it, scores of either sign and scores that are no numbers
 BLOCKS = {"small": (N, N.attn(64, 64, 16, 32)), "middle": (N, N.attn(64, 64, 72, 80, rot=8)), "large": (N, N.attn(64, 64, 200, 250)),
           "groups": (N, N.attn(96, 48, 40, 56, rot=8)), "chunks": (N, N.attn(64, 64, 40, 56, chunk=400)), "negative": (N, N.attn(64, 64, 40, 56, scale=-0.2)),
-          "latent": (K, K.gated(64, 40, 16, 56, 48)), "latent_wide": (K, K.sunk(64, 128, 64, 128, 96)), "nan": (N, N.attn(64, 64, 40, 56, scale=float("nan")))}
+          "keys_192": (N, N.attn(64, 64, 160, 96)), "latent": (K, K.gated(64, 40, 16, 56, 48)), "latent_middle": (K, K.sunk(64, 72, 32, 88, 48)),
+          "latent_wide": (K, K.sunk(64, 128, 64, 128, 96)), "latent_large": (K, K.gated(64, 160, 64, 200, 96)), "nan": (N, N.attn(64, 64, 40, 56, scale=float("nan")))}
 
 
 @pytest.mark.parametrize("name", list(BLOCKS))

@@ -72,6 +72,24 @@ def test_order_of_the_workgroups():
     assert len(kinds) == 3
 
 
+def test_attention_in_blocks_of_32():
+    """The cases of its test take them, in every size of tile, and their keys are never split."""
+    seen = set()
+    for name, (model, mixer) in A.BLOCKS.items():
+        m = mixer.get("mixer", mixer)
+        R, G = (1, m["heads"]) if "mixer" in mixer else (m["heads"] // m["kv_heads"], m["kv_heads"])
+        for n, pos in ((900, 0), (907, 900)):
+            assert splits(n, R, G, pos, m.get("mask", {}).get("size", 0), vdim=m["vdim"])[1] == 128, name
+        keys, values = m["dim"] + m.get("rot_dim", 0), m["vdim"]
+        tile = next(t for t in ((64, 64), (128, 128), (192, 128), (256, 256)) if keys <= t[0] and values <= t[1])
+        seen.add((*tile, "mixer" in mixer))
+    assert seen == {(*t, latent) for t in ((64, 64), (128, 128), (192, 128), (256, 256)) for latent in (False, True)}
+    rng = random.Random(6)
+    for _ in range(500):
+        n, columns = splits(rng.randint(2, 8000), rng.choice([1, 2, 4]), rng.choice([1, 8, 16, 32, 128]), rng.randrange(0, 9000), rng.choice([0, 8192]))
+        assert columns == 64 or n == 1
+
+
 def test_attention_with_workgroups_left_over():
     """What its test is for."""
     first, n = A.LEFT_OVER_TOKENS
