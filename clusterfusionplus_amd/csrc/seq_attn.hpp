@@ -86,8 +86,10 @@ template <typename T, int NK, int NT, int C> struct AttnTile {
 // 2 x 16 935 / 79, sums that are rescaled for maxima that move by 2^8 only and no value converted twice 895 / 73, addresses that are carried from
 // tile to tile 887 / 70.
 // 37 tokens at 1990, 32 / 8 heads: 85 -> 12 us and 5 for the merge (24 workgroups became 384).
-// Tried and slower: two groups of four waves that take turns at products and softmax (1000 against 875), the scores of the next tile
-// beside the softmax with tiles of 32 keys (1318).
+// Tried and slower, on blocks of 16 with fragments read ahead, which took 875 us on that card (8000 tokens): two groups of four waves that take turns at
+// products and softmax (1000), the scores of the next tile beside the softmax with tiles of 32 keys (1318).
+// Reading ahead takes heads of up to 64 from 79 to 103 registers, four waves of a SIMD instead of five: 16 heads, 1500 tokens at 0 / at 1990 take 29.6 /
+// 66.4 us without and 24.6 / 55.2 with it and the order of the workgroups, 100 tokens 6.5 and 6.5.
 // (NK: elements of a key row in LDS, NT: value columns.  The products run over all of them, without branches between the reads
 // of LDS: past the end of the query there are zeros, and of the columns past the end of a value nothing is stored.
 // C: columns of a wave; SH: keys have a shared part)

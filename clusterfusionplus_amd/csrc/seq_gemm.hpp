@@ -110,7 +110,8 @@ __device__ __forceinline__ void gemm_store(const SeqGemm& p, const GemmTile& t, 
         rp = k ? p.kp : p.vp;
         return (k ? p.yt + h * p.kh : p.yv + h * p.vh) + (m - h * d) * (int)sizeof(T);
     };
-    // bf16 outputs leave in units of 16 bytes (gated, two tiles only: 8): as a lane has them, 4 or 2 outputs of a token, a store of the wave takes 16
+    // bf16 outputs leave in units of 16 bytes (gated, two tiles only: 8) where a wave has an even number of tiles of rows (64 x 16, 64 x 32, 96 x 128,
+    // 96 x 160 and 192 x 160 have one or three, and store 4 or 8 bytes below): as a lane has them, 4 or 2 outputs of a token, a store of the wave takes 16
     // lines of memory for 512 or 256 bytes.  Lane group g of every two tiles' four (gated, four tiles: of all four) takes a row's next outputs from
     // the groups beside it.  256 x 256 tiles: keys and values from latents of 512 values, 3151 positions 24.6 -> 20.4 us, 8000 103 -> 82;
     // 16384 x 4096, 2048 tokens 238 -> 220; 22528 gated rows, 8000 tokens 1089 -> 1059.

@@ -119,12 +119,13 @@ struct AttnSizes {
     size_t floats;           // of a split's partial results
 };
 // Columns of a workgroup and splits of the keys.  bf16: waves of 32 columns take fewer instructions per weight, those of 16 balance better
-// where there are few workgroups.  The line is at two workgroups of four such waves per compute unit (us with 16 / 32 columns, 32 heads of 128 and
-// 128: 1500 tokens, 384 workgroups 47 / 55, 2048 tokens, 512 workgroups 76.5 / 76, 3000 tokens 136 / 134; of 192 and 128: 1600 tokens 67 / 78,
-// 2048 90 / 96, 3000 171 / 168).  Splits fill the chip: two workgroups per
-// compute unit, with two tiles at least in each split of the longest walk, which begins at the chunk of the portion's first token (that
-// chunk counts and not the context: 37 tokens just behind a chunk of 8192 see one tile; shared by 16 splits, eight layers of 32 / 8 heads
-// of 128 took 1005 us, and take 957).
+// where there are few workgroups.  The line is at two workgroups of four such waves per compute unit, which is where it belongs for 32 heads of 128
+// (us with 16 / 32 columns: 1500 tokens, 384 workgroups 43 / 52, 2048 tokens, 512 workgroups 67 / 68, 3000 122 / 126; behind 1990 positions 114 / 122,
+// 156 / 150, 262 / 248).  Of keys of 192 it is early for prompts (2048 tokens 74 / 76, 2300 88 / 95, 3000 140 / 133; at 1990 183 / 171), of heads of
+// 64 more so (2048 39 / 45, 3000 69 / 71; at 1990 96 / 89), and of 256 late for 32 heads (1500 110 / 93, 2048 167 / 143; at 1990 421 / 333).
+// Splits fill the chip: two workgroups per compute unit, with two tiles at least in each split of the longest walk, which begins at the chunk of the
+// portion's first token (that chunk counts and not the context: 37 tokens just behind a chunk of 8192 see one tile; shared by 16 splits, eight layers
+// of 32 / 8 heads of 128 took 1005 us, and take 957).
 //
 // The order of the workgroups.  A row of them is the same columns of all key heads and splits; rows go from the last block of columns, which walks
 // the most keys, to the first.  Where all are resident, two per compute unit, workgroups i and i + `cus` share one (the hardware places them in turn:
