@@ -152,7 +152,7 @@ inline AttnPlan plan_attn(const AttnSizes& a, int cus, size_t room) {
     const int rows = wgs / a.G, some = std::max(1, cus / (a.G * splits)), total = wgs * splits;
     if (a.per_cu >= 2 && total <= 2 * cus) return {two, splits, some, 0};
     const bool alike = 2 * (behind - a.T) >= a.T && (a.chunk == 0 || behind <= a.chunk);
-    return {two, splits, rows, a.per_cu >= 2 && total <= 3 * cus && alike ? some : 0};
+    return {two, splits, rows, a.per_cu >= 2 && total <= 3 * cus && alike ? std::min(some, rows / 2) : 0};
 }
 
 }  // namespace cfpp

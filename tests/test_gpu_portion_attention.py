@@ -127,6 +127,19 @@ def test_workgroups_left_over(name, dtype):
     assert N.error(got, M.oracle(cfg, w, toks)) < LIMIT[dtype]
 
 
+# more heads than workgroups are resident: one row of them
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("kind", ["grouped", "latent"])
+def test_one_row_of_many_heads(kind, dtype):
+    from clusterfusionplus_amd import kagapel, nibotar
+    cfg = K.model(64, 51, [K.sunk(600, 8, 8, 8, 16)]) if kind == "latent" else N.model(64, 51, [(N.attn(600, 600, 8, 8), None)])
+    M, make = (K, kagapel) if kind == "latent" else (N, nibotar)
+    w, toks = M.weights(cfg, 5), M.prompt(cfg, 30, 6)
+    m = make.from_tensors(cfg, w, dtype, capacity=30)
+    got = torch.cat([m.forward(0, toks[:20], 0, range(20)), m.forward(0, toks[20:], 20, range(10))])
+    assert N.error(got, M.oracle(cfg, w, toks)) < LIMIT[dtype]
+
+
 # latent projections of up to 4096, 8192 and 12288 values, and of more; in one part (64 columns) and in several (512); rows and gates that are no whole
 # groups of four; a layer that reads the latents of another
 LATENTS = {"1k": (5, 128, 64, 56, 48), "4k": (19, 128, 64, 56, 384), "4k_more": (19, 128, 64, 56, 388), "6k": (24, 128, 64, 56, 48), "12k": (48, 128, 64, 56, 48), "16k": (64, 128, 64, 56, 48), "no_fours": (3, 41, 16, 55, 49), "gates_no_fours": (3, 44, 16, 55, 48)}

@@ -52,8 +52,9 @@ def test_order_of_the_workgroups():
     are left over; otherwise the longest are first."""
     rng, kinds = random.Random(4), set()
     for T, R, G, keys, pos, chunk in [(1000, 1, 16, 32, 0, 0), (1000, 4, 8, 32, 0, 0), (1500, 2, 5, 32, 0, 0), (700, 3, 4, 32, 0, 0), (3000, 1, 300, 64, 0, 0), (1150, 1, 32, 32, 1990, 0),
-                                      (1500, 1, 32, 32, 1990, 0), (1500, 1, 32, 32, 1990, 3000), (1500, 1, 32, 32, 1990, 3490), (1500, 1, 32, 32, 749, 0), (1100, 1, 40, 64, 550, 0), (66, 1, 300, 64, 64, 0)] + \
-            [(rng.randint(2, 4000), rng.choice([1, 2, 4, 8]), rng.choice([1, 2, 3, 5, 8, 12, 16, 32, 40]), rng.choice([32, 64]), rng.choice([0, 100, 1000, 3000]), rng.choice([0, 0, 2000, 8192])) for _ in range(600)]:
+                                      (1500, 1, 32, 32, 1990, 0), (1500, 1, 32, 32, 1990, 3000), (1500, 1, 32, 32, 1990, 3490), (1500, 1, 32, 32, 749, 0), (1100, 1, 40, 64, 550, 0), (66, 1, 300, 64, 64, 0), (10, 1, 600, 64, 20, 0), (64, 1, 768, 32, 64, 0), (65, 1, 257, 32, 64, 0), (100, 1, 384, 64, 64, 0)] + \
+            [(rng.randint(2, 4000), rng.choice([1, 2, 4, 8]), rng.choice([1, 2, 3, 5, 8, 12, 16, 32, 40]), rng.choice([32, 64]), rng.choice([0, 100, 1000, 3000]), rng.choice([0, 0, 2000, 8192])) for _ in range(600)] + \
+            [(rng.randint(2, 200), 1, rng.randint(100, 4096), rng.choice([32, 64]), rng.choice([0, 100, 3000]), 0) for _ in range(300)]:
         n, columns, order = P.attention_plan(T, R, G, pos, chunk, keys, T * R * G * 130, ROOM)
         rows, what = len(order), (T, R, G, keys, pos, chunk)
         assert sorted(order) == list(range(rows)), what
@@ -64,8 +65,8 @@ def test_order_of_the_workgroups():
             assert max(blocks[i] + sum(blocks[i + P.CUS:i + P.CUS + 1]) for i in range(min(P.CUS, len(blocks)))) <= rows, what
         elif len(blocks) <= 3 * P.CUS and alike:
             kinds.add("left over")
-            some = P.CUS // G * G or G
-            assert n == 1 and all(blocks[i] < blocks[i + some] for i in range(some)) and max(blocks[2 * some:], default=-1) < min(blocks[:2 * some]), what
+            some = min(P.CUS // G or 1, rows // 2) * G
+            assert n == 1 and all(blocks[i] < blocks[i + some] for i in range(some)) and max(blocks[2 * some:], default=-1) < min(blocks[:2 * some], default=rows), what
         else:
             kinds.add("many")
             assert n == 1 and blocks == sorted(blocks, reverse=True), what
