@@ -1,7 +1,7 @@
 """fp32 products of 64 tokens and more, whose values are taken apart into bf16 parts: every tile in every kind of product, one to many steps of k,
 values that bf16 does not hold, infinities and NaN.
 
-Limit: a product's value is kept to 2^-26 and sums are rounded in fp32, which over the sums of these sizes gives 1e-6 of the outputs' spread in
+Limit: a product's value is kept to 2^-24 and sums are rounded in fp32, which over the sums of these sizes gives 1e-6 of the outputs' spread in
 the products alone; attention and norms, in fp32 as before, add as much."""
 import functools
 
@@ -114,3 +114,33 @@ def test_values_of_the_head(sizes, what):
         keep = [i for i in range(vocab) if i not in rows]
         got, want = got[:, keep], want[:, keep]
     assert M.error(got, want) < LIMIT
+
+
+def by_row(got, want):
+    """Root mean square of the difference of each row of the head, in units of its own spread."""
+    d = got.double() - want
+    return (d.pow(2).mean(0).sqrt() / want.std(0)).max().item()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("what", ["rows", "inputs of 1e30", "inputs of 1e37", "inputs of 1e-7", "all small"])
+@pytest.mark.parametrize("sizes", [s for s, _ in HEAD], ids=str)
+def test_small_values_beside_others(sizes, what):
+    """A value's error goes with the value: small rows of weights between ordinary ones, a column of inputs that are large where the weights are small,
+    or the other way round, inputs and weights that are all small.  (2^-24 is the least that a final norm's factor 1 + w can be but for zero.)"""
+    n, width, vocab = sizes
+    cfg, w, toks, _, _ = dense(n, width, 0, vocab, None)
+    w = dict(w, head=w["head"].clone())
+    w["final.norm"] = w["final.norm"].clone()
+    if what == "rows":
+        for row, scale in zip([0, 1, 70, 71, vocab // 2, vocab - 1], [1e-30, 1e-33, 1e-35, 1e-36, 1e-34, 1e-37]):
+            w["head"][row] *= scale
+    elif what == "all small":
+        w["final.norm"][:] = -1 + 2.0 ** -24
+        w["head"] *= 1e-29
+    else:
+        factor = 2.0 ** -24 if what == "inputs of 1e-7" else float(what.split()[-1])
+        w["final.norm"][width // 3] = factor if factor > 1 else factor - 1
+        w["head"][:, width // 3] /= factor
+    got, want = nibotar(cfg, w, n).forward(0, toks, 0, range(n)).cpu(), M.oracle(cfg, w, toks)
+    assert by_row(got, want) < LIMIT
