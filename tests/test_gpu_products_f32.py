@@ -20,6 +20,7 @@ DOWN = [((97, 1030, 4100), (*S, 6)), ((193, 3000, 700), (*T, 2)), ((129, 3000, 1
 GATED = [((129, 60, 5001), S), ((97, 130, 5001), T), ((65, 93, 12001), B)]
 HEADS = [((24, 100, 72, 512, 129), S), ((24, 192, 200, 130, 97), T), ((24, 192, 200, 60, 200), B)]
 EXPERTS = [((200, 2, 8, 2000, 29), S), ((200, 2, 3, 2000, 61), S), ((150, 1, 3, 4001, 125), T), ((300, 1, 2, 2000, 125), T), ((150, 2, 3, 4001, 29), B), ((300, 2, 3, 2000, 29), B)]
+UP_SIZES = [s for s, _ in UP]
 HEAD = [((97, 61, 16001), S), ((97, 125, 10001), T), ((97, 29, 20001), B)]
 
 
@@ -144,3 +145,29 @@ def test_small_values_beside_others(sizes, what):
         w["head"][:, width // 3] /= factor
     got, want = nibotar(cfg, w, n).forward(0, toks, 0, range(n)).cpu(), M.oracle(cfg, w, toks)
     assert by_row(got, want) < LIMIT
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes", [s for s, _ in UP[::2] + GATED] + [(n, 64, None, mixer) for *mixer, n in [s for s, _ in HEADS]] + [s for s, _ in EXPERTS[::3]], ids=str)
+def test_a_token_that_is_no_number(sizes):
+    """Every kind of product: it and the tokens behind it, which see its key, are no numbers; those before it are as they are, but for the ones
+    whose keys share its tile of 32 in the attention (their weights for it are zero, and zero times its values is no number)."""
+    if len(sizes) == 5:
+        n, top, experts, ff, width = sizes
+        cfg, made, lib = M.model(width, 64, [(M.attn(2, 1, 16, 16), M.moe(ff, experts, top))]), M, "nibotar"
+    elif sizes in UP_SIZES:
+        n, width, ff = sizes
+        cfg, made, lib = M.model(width, 51, [(M.attn(2, 1, 16, 16), M.dense(ff))]), M, "nibotar"
+    else:
+        n, width, ff, (heads, dim, vdim, rank) = (*sizes, (2, 16, 16, 24))[:4]
+        cfg, made, lib = K.model(width, 51, [K.gated(heads, dim, 16, vdim, rank, ff=ff)], streams=2, positions=n), K, "kagapel"
+    import importlib
+    lib = importlib.import_module(f"clusterfusionplus_amd.{lib}")
+    w = fp32(made.weights(cfg, 9))
+    w["embed"][0] = float("nan")
+    toks, bad = [t or 1 for t in M.prompt(cfg, n, 10)], 2 * n // 3
+    toks[bad] = 0
+    got = lib.from_tensors(cfg, w, torch.float32, capacity=n).forward(0, toks, 0, range(n)).cpu()
+    assert got[bad:].isnan().all()
+    clean = bad // 32 * 32
+    assert M.error(got[:clean], made.oracle(cfg, w, toks[:clean])) < LIMIT
