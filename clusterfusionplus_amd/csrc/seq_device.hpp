@@ -308,6 +308,20 @@ __device__ __forceinline__ void vt_request(u32x4 (&r)[N][4], int vunits, int tid
         for (int j = 0; j < 4; ++j) r[b][j] = ld16(rowp(kg * 4 + j) + (size_t)vc * 16);
     }
 }
+// ... the offsets of what is requested from the tile's first row, of which `left` follow; in registers from here on
+template <typename T, int KT, int NTHREADS, int FIRST, int N>
+__device__ __forceinline__ void vt_place(uint32_t (&at)[N][4], int vunits, int tid, int left, int vrow) {
+    constexpr int KG = KT / 4;
+#pragma unroll
+    for (int b = 0; b < N; ++b) {
+        const int idx = tid + (FIRST + b) * NTHREADS, kg = idx % KG, vc = min(idx / KG, vunits - 1);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            at[b][j] = (uint32_t)(min(kg * 4 + j, left) * vrow) + vc * 16;
+            asm volatile("" : "+v"(at[b][j]));
+        }
+    }
+}
 // ... the keys from `from` on get the row at `row` instead
 template <typename T, int KT, int NTHREADS, int FIRST, int N>
 __device__ __forceinline__ void vt_replace(u32x4 (&r)[N][4], int vunits, int tid, int from, const char* row) {

@@ -41,3 +41,17 @@ def test_more_splits_than_travel_together(dtype):
     m.forward(0, toks[:4195], 0, [4194])
     got = torch.cat([m.forward(0, [toks[i]], i, [0]) for i in range(4195, 4198)])
     assert M.error(got, want[4195:]) < LIMIT[dtype]
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("heads, dim, vdim", [(128, 24, 20), (128, 72, 88), (128, 136, 72)], ids=str)
+def test_several_tiles_per_wave(heads, dim, vdim, dtype):
+    """So many heads that the keys are in few splits: every wave goes on to further tiles, the last of them short, in rows that do not fill the columns."""
+    cfg = M.model(64, 97, [(M.attn(heads, heads, dim, vdim), M.dense(64))])
+    w, toks = M.weights(cfg, 5), M.prompt(cfg, 1101, 6)
+    want = M.oracle(cfg, w, toks)
+    m = build(cfg, w, dtype, capacity=1110, max_portion=1110)
+    for first in (700, 1023, 1097):
+        m.forward(0, toks[:first], 0, [first - 1])
+        got = torch.cat([m.forward(0, [toks[i]], i, [0]) for i in range(first, first + 4)])
+        assert M.error(got, want[first:first + 4]) < LIMIT[dtype], f"from position {first}"
