@@ -399,10 +399,9 @@ __global__ __launch_bounds__(kSeqThreads, 1) void k_seq_latent_attn(SeqLatentAtt
 // Workgroup (head, kLatentOut of its outputs; the head runs fastest, which keeps the workgroups of one head, who read the same
 // partial results, on few XCDs): merges the splits of the head, then its rows of W_uv, four per wave, in fp32, and
 // the output gate.
-// It is bound by the partial results, which every workgroup of a head reads: 32 heads of 512 latents behind 4096 positions, 65 splits, 133 KB.  In one
-// round trip, the maxima ahead of them, instead of three of 16 loads: 6.9 -> 6.1 us from the first start to the last end.  (kM: loads in flight per
-// thread.  36 of them leave room for two workgroups per compute unit; where there are more, as with 128 heads, they hide each other's waits: 8 layers
-// behind 2048 positions 1606 us with 16, 1620 with 36.)
+// It is bound by the partial results, which every workgroup of a head reads: 32 heads of 512 latents behind 4096 positions, 65 splits, 133 KB.  The splits'
+// maxima go ahead of them: a step of 32 such layers 3048 -> 3020 us.  (kM: loads in flight per thread.  With 36, one round trip for 65 splits, 3027; over nine models
+// and nine contexts between 2.5 % less, for 8 heads behind 8000 positions, and 4 % more, for 48 heads behind 4096: two workgroups per compute unit instead of four.)
 constexpr int kLatentOut = 16;
 constexpr int kLatentSplits = kSeqThreads;
 struct SeqLatentOut {
@@ -414,7 +413,7 @@ struct SeqLatentOut {
     char* out;               // T [H * V]
     int H, V, pitch, ns, least, rp;
 };
-template <typename T, int kM>
+template <typename T>
 __global__ __launch_bounds__(kSeqThreads) void k_seq_latent_out(SeqLatentOut a) {
     constexpr int U = Unit<T>::n, RPW = kLatentOut / kSeqWaves, NC = sizeof(T) == 2 ? 1 : 2;     // rows per wave, 1 KB loads per row
     __shared__ float f[kLatentSplits], red[kSeqWaves];
@@ -437,6 +436,7 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_latent_out(SeqLatentOut a) 
     const int r4 = a.rp / 4, nsg = kSeqThreads / r4, sg = tid / r4, x = tid - sg * r4;
     const float* p = a.acc + (size_t)h * a.rp + x * 4;
     const size_t split_stride = (size_t)a.H * a.rp;
+    constexpr int kM = 16;
     f32x4 t[kM];
     auto request = [&](int s0) __attribute__((always_inline)) {
 #pragma unroll

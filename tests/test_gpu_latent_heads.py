@@ -1,4 +1,4 @@
-"""One token's latent attention with so many heads that k_seq_latent_out's workgroups share compute units in another way (more than 512 of them)."""
+"""One token's latent attention with many heads: on both sides of two workgroups of k_seq_latent_out per compute unit (512), heads of more outputs than a workgroup has."""
 import pytest
 import torch
 
