@@ -89,7 +89,7 @@ def ensure_neox():
 
 
 LDS_BYTES = 160 * 1024       # of a compute unit
-FEEDERS = 4                  # waves of k_seq_gemm (but in tiles of 128 x 64) and k_seq_gemm_beside that copy
+FEEDERS = 4                  # waves of k_seq_gemm and k_seq_gemm_beside that copy
 
 
 def launch_lds(kernel):
@@ -166,7 +166,7 @@ def resource_report(out=None):
         if at_launch is not None and at_launch[0] is None:
             lds += "+"
         elif at_launch is not None:
-            total, in_all = int(lds) + at_launch[0], at_launch[1] + (FEEDERS if nice.startswith(("k_seq_gemm<", "k_seq_gemm_beside<")) and ", 128, 64," not in nice else 0)
+            total, in_all = int(lds) + at_launch[0], at_launch[1] + (FEEDERS if nice.startswith(("k_seq_gemm<", "k_seq_gemm_beside<")) else 0)
             lds, waves = str(total), str(min(int(waves), max(1, LDS_BYTES // total * in_all // 4)))
         rows.append((nice, g("VGPRs"), g("AGPRs"), g(r"ScratchSize \[bytes/lane\]"), lds, waves))
     lines = [f"{'kernel':44s} {'VGPRs':>6s} {'AGPRs':>6s} {'scratch B/lane':>15s} {'LDS B/workgroup':>16s} {'waves/SIMD':>11s}"]
