@@ -144,6 +144,21 @@ def test_tiles_of_the_head(sizes, tile):
     assert P.product(vocab, n, width, True) == (*tile, 1)
 
 
+def test_tiles_of_two_products_in_a_launch():
+    """Every tile in which the shared expert's product is put beside the experts' has kernels for both, in either kind of product."""
+    with open(build.SEQ_LIB, "rb") as f:
+        kernels = {(m[1] != b"f", int(m[2]), int(m[3])) for m in re.finditer(rb"k_seq_gemm_besideI(\w+?)Li(\d+)ELi(\d+)E", f.read())}
+    rng, beside = random.Random(7), set()
+    for _ in range(4000):
+        n, top, count = rng.choice([2, 5, 16, 17, 40, 64, 65, 129, 150, 300, 700, 2000]), rng.randint(1, 8), rng.choice([1, 2, 3, 8, 24, 64])
+        ff, shared, width, bf16 = rng.choice([60, 700, 1408, 4000]), rng.choice([1, 60, 700, 2816, 6000]), rng.choice([60, 192, 2048, 4096]), rng.random() < 0.5
+        a = (n, min(top, count), count, ff, P.row_bytes(width, bf16))
+        for sizes in ((2 * ff, a[4], 2 * shared, a[4], 0, 0), (width, P.row_bytes(ff, bf16), width, P.row_bytes(shared, bf16), width, P.room(n, width))):
+            if P.lib().beside(*a, *sizes, bf16, P.CUS):
+                beside.add((bf16, *P.experts(n, a[1], count, ff, width, bf16)[:2]))
+    assert beside == kernels, beside ^ kernels
+
+
 def test_every_tile_is_tested_in_every_kind_of_product():
     tiles = {(64, 16, 2), (64, 32, 2), (64, 64, 2), (64, 96, 2), (256, 96, 1), (128, 128, 2), (256, 128, 1), (256, 256, 1), (128, 64, 2), (96, 128, 1), (128, 128, 1),
              (128, 192, 1), (192, 160, 1), (96, 160, 1)}
