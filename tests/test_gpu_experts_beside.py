@@ -1,4 +1,5 @@
-"""The shared expert's products in the experts' launches and behind them: the same results by either way."""
+"""The shared expert's products in the experts' launches and behind them: the oracle's results by either way.  Which way each case takes
+stands with it; tests/test_seq_plan.py holds the table to the plan."""
 import functools
 
 import pytest
@@ -9,15 +10,18 @@ from tests import seq_plan as P
 from tests.test_gpu_nibotar import DTYPES, IDS, LIMIT, build
 
 pytestmark = pytest.mark.gpu
-WIDTH, FF, EXPERTS, TOP = 192, 72, 24, 3
+WIDTH, FF, EXPERTS, TOP, PORTION = 192, 72, 24, 3, 1300
+TOKENS = (2, 15, 16, 17, 64, 65, 129, 500, 1200)
+# (the shared expert's inner size, bf16): for each of the counts, b: both of its products are beside the experts', u: the up rows only, -: neither
+WAYS = {(1, True): "bbbbbbbbb", (40, True): "bbbbbbbbb", (72, True): "bbbbbbbbb", (900, True): "uuuuuuuu-", (2500, True): "uuuuuuu--",
+        (1, False): "bbbbbbbbb", (40, False): "bbbbbbbbb", (72, False): "bbbbbbbbb", (900, False): "uuuuuuu-u", (2500, False): "uuuuuuu--"}
 
 
-def besides(n, shared, size):
-    """(up, down): whether a portion of n tokens has the shared expert's product in the experts' launch"""
-    pitch = lambda k: -(-k * size // 128) * 128
-    a = (n, TOP, EXPERTS, FF, pitch(WIDTH))
-    return tuple(bool(P.lib().beside(*a, rows, kb, srows, skb, ldy, 0, size == 2, P.CUS))
-                 for rows, kb, srows, skb, ldy in ((2 * FF, pitch(WIDTH), 2 * shared, pitch(WIDTH), 0), (WIDTH, pitch(FF), WIDTH, pitch(shared), WIDTH)))
+def way(n, shared, bf16):
+    """What the library decides for a portion of n tokens."""
+    x, h, hs = (P.row_bytes(k, bf16) for k in (WIDTH, FF, shared))
+    up, down = (bool(P.lib().beside(n, TOP, EXPERTS, FF, x, *sizes, bf16, P.CUS)) for sizes in ((2 * FF, x, 2 * shared, x, 0, 0), (WIDTH, h, WIDTH, hs, WIDTH, P.room(PORTION, WIDTH))))
+    return {(True, True): "b", (True, False): "u", (False, False): "-", (False, True): "d"}[up, down]
 
 
 @functools.lru_cache(maxsize=None)
@@ -28,12 +32,9 @@ def reference(shared):
 
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
-@pytest.mark.parametrize("shared", [1, 40, 72, 900])
+@pytest.mark.parametrize("shared", sorted({shared for shared, _ in WAYS}))
 def test_shared_beside_and_behind(shared, dtype):
     cfg, w, toks, want = reference(shared)
-    m = build(cfg, w, dtype, capacity=1300, max_portion=1300)
-    ways = set()
-    for n in (2, 15, 16, 17, 64, 65, 129, 500, 1200):
-        ways.add(besides(n, shared, 4 if dtype == torch.float32 else 2))
+    m = build(cfg, w, dtype, capacity=PORTION, max_portion=PORTION)
+    for n in TOKENS:
         assert M.error(m.forward(0, toks[:n], 0, range(n)), want[:n]) < LIMIT[dtype], f"{n} tokens"
-    assert ((True, True) if shared <= 72 else (True, False)) in ways

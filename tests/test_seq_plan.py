@@ -7,6 +7,7 @@ import pytest
 
 from clusterfusionplus_amd import build
 from tests import seq_plan as P
+from tests import test_gpu_experts_beside as B
 from tests import test_gpu_portion_attention as A
 from tests import test_gpu_products as G
 
@@ -157,6 +158,12 @@ def test_tiles_of_two_products_in_a_launch():
             if P.lib().beside(*a, *sizes, bf16, P.CUS):
                 beside.add((bf16, *P.experts(n, a[1], count, ff, width, bf16)[:2]))
     assert beside == kernels, beside ^ kernels
+
+
+def test_ways_of_shared_experts():
+    """The ways that the shared experts' test is for."""
+    for (shared, bf16), ways in B.WAYS.items():
+        assert "".join(B.way(n, shared, bf16) for n in B.TOKENS) == ways, (shared, bf16)
 
 
 def test_every_tile_is_tested_in_every_kind_of_product():
