@@ -15,7 +15,7 @@ inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 // rows and k of 1408 to 14336 (bf16; fp32: 17 to 1500 tokens): a step of 128 bytes of k when a compute unit has one workgroup, the
 // share of a step when it has `resident` of them (the more of them, the more bytes in flight; past that they take turns), and
 // what a workgroup costs beside its steps.  (bf16: with all waves copying.  Since four waves do, steps are up to 17 % shorter in all tiles but those of
-// weight streams; a table fitted to that chose tiles that are 0.7 % better on their own and none better in a model, so it stays.)
+// weight streams; a table fitted to that chose tiles that are 0.7 % better on their own and up to 2 % worse in a model, so it stays.)
 // The estimate below is there to compare tiles: a product takes longer than it says, 10 % on average for the tile chosen (root mean
 // square 16 %; fp32 15 and 20 %), most where it is a stream of weights: 22528 x 4096 estimated and measured 36 / 35 us for 66 tokens, 36 / 38
 // for 100, 40 / 44 for 150, 58 / 63 for 300, 84 / 87 for 512, 253 / 272 for 2048.  What it chooses is 1.7 % slower than the best tile and split
@@ -24,7 +24,7 @@ inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 // A tile is in the table because it is missed where it is chosen; without it the next choice takes longer, on average and at most:
 // 64 x 16 2 / 24 %, 64 x 32 7 / 29, 64 x 64 6 / 13, 64 x 96 11 / 34, 256 x 96 0 / 9, 256 x 128 19 / 34,
 // 256 x 256 11 / 27, 128 x 64 3 / 11, 96 x 128 11 / 31, 128 x 128 alone on a compute unit 16 / 48, 128 x 192 10 / 21, 192 x 160 8 / 31, 96 x 160 10 / 17.
-// 128 x 128 with two workgroups per compute unit is for few steps of k (keys and values from latents of 200 values, 4000 positions) and for 128256 rows of
+// (256 x 96, which a product alone can do without, is for the experts' rows: see plan_experts.)  128 x 128 with two workgroups per compute unit is for few steps of k (keys and values from latents of 200 values, 4000 positions) and for 128256 rows of
 // a head.
 // The tiles from the ninth on are for 50 to 700 tokens, where a product is still a stream of weights, which tiles of few tokens read
 // two or three times: they hold the tokens in one tile or two, and their rings fill a compute unit's LDS.
