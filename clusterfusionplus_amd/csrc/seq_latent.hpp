@@ -400,7 +400,7 @@ __global__ __launch_bounds__(kSeqThreads, 1) void k_seq_latent_attn(SeqLatentAtt
 // partial results, on few XCDs): merges the splits of the head, then its rows of W_uv, four per wave, in fp32, and
 // the output gate.
 // It is bound by the partial results, which every workgroup of a head reads: 32 heads of 512 latents behind 4096 positions, 65 splits, 133 KB.  The splits'
-// maxima go ahead of them: a step of 32 such layers 3048 -> 3020 us.  (kM: loads in flight per thread.  With 36, one round trip for 65 splits, 3027; over nine models
+// maxima go ahead of them: a step of 32 such layers 3049 -> 3027 us.  (kM: loads in flight per thread.  With 36, one round trip for 65 splits, 3022; over nine models
 // and nine contexts between 2.5 % less, for 8 heads behind 8000 positions, and 4 % more, for 48 heads behind 4096: two workgroups per compute unit instead of four.)
 constexpr int kLatentOut = 16;
 constexpr int kLatentSplits = kSeqThreads;
