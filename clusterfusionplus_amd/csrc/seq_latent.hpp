@@ -4,6 +4,8 @@
 // it, the rotated key part that all heads share.
 //   Portions: the plain keys and the values of all heads are made from the cached latents by one matrix product
 //   (kEpiHeads) and attention runs over them head by head; the rotated part is read from the cache rows as it is.
+//   Portions of few tokens behind many positions (plan_latent_turn): as in decode, for all columns (token, head) side by side (k_seq_latent_absorb,
+//   k_seq_latent_block, k_seq_latent_turn_out).
 //   Decode: the query is taken into the latent space instead, q' = W_uk^T q (k_seq_latent_q), all heads attend to the cache
 //   rows themselves, as keys and as values (k_seq_latent_attn), and W_uv turns the weighted latents into the heads' outputs
 //   (k_seq_latent_out, which also merges the splits).  A step reads the cache once instead of making keys and values.
@@ -506,6 +508,384 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_latent_out(SeqLatentOut a) 
         if (v < a.V) {
             if (a.gate != nullptr) o *= sigmoid(a.gate[h * a.V + v]);
             reinterpret_cast<T*>(a.out)[h * a.V + v] = from_f32<T>(o);
+        }
+    }
+}
+
+// ---- portions of few tokens behind many positions ----------------------------------------------
+// The same three passes as for one token, for the columns (token, head) of a portion, head fastest: the cache is read as it is, and no keys and
+// values are made of it.  A column costs a portion's products of kv_rank instead of dim and vdim values for every key, so it is for few tokens (plan_latent_turn).  What it
+// replaces at 3000 positions: 16 heads 20 us for the keys and values, 12 for the attention and 5 for its merge; 128 heads 90, 60 and 8.
+
+// Queries into the latent space: workgroup (head, 64 latent columns, tokens), W_uk^T q from the rows that k_seq_latent_finish has made.  A wave owns 16
+// of the columns; W_uk, whose rows are dimensions, is taken through LDS, where a product's operand is read down its columns.
+struct SeqLatentAbsorb {
+    const char* q;           // T [tokens][H][qrow bytes]: plain part, at `plain` bytes the rotated part
+    const char* w_uk;        // T [H * D][pitch bytes]
+    char* out;               // T [tokens][H][crow bytes]: q' padded to `pitch` bytes, then the rotated part
+    int n, pitch, H, D, R, ncb, qrow, plain, crow;
+};
+constexpr int kAbsorbDims = 128, kAbsorbSets = 2;        // dimensions in LDS at a time, sets of 16 tokens of a workgroup
+template <typename T>
+__global__ __launch_bounds__(kSeqThreads) void k_seq_latent_absorb(SeqLatentAbsorb a) {
+    constexpr int U = Unit<T>::n, kCols = 64, kUnits = kCols / U, P = kCols + 2 * U, KS = 4 * U;      // units of a row in LDS, its elements, dimensions of a product
+    constexpr int kLoads = kAbsorbDims * kUnits / kSeqThreads, kSteps = kAbsorbDims / KS;
+    __shared__ __align__(16) T w[kAbsorbDims * P];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 15, g = lane >> 4;
+    const int h = blockIdx.x / a.ncb, c0 = (blockIdx.x - h * a.ncb) * kCols, t0 = blockIdx.y * 16 * kAbsorbSets, columns = a.pitch / (int)sizeof(T);
+    const char* from = a.w_uk + (size_t)h * a.D * a.pitch + (size_t)c0 * sizeof(T);
+    const int units = min(kUnits, (columns - c0) / U);
+    f32x4 acc[kAbsorbSets];
+#pragma unroll
+    for (int s = 0; s < kAbsorbSets; ++s) acc[s] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int d0 = 0; d0 < a.D; d0 += kAbsorbDims) {
+        // one round trip for everything; behind the last dimension there are zeros (of a query others would begin there)
+        u32x4 b[kLoads], x[kAbsorbSets][kSteps];
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) {
+            const int r = (tid + i * kSeqThreads) / kUnits, u = (tid + i * kSeqThreads) % kUnits;
+            b[i] = ld16(from + (size_t)min(d0 + r, a.D - 1) * a.pitch + min(u, units - 1) * 16);
+            if (d0 + r >= a.D || u >= units) b[i] = u32x4{0, 0, 0, 0};
+        }
+#pragma unroll
+        for (int s = 0; s < kAbsorbSets; ++s) {
+            const char* q = a.q + ((size_t)min(t0 + s * 16 + col, a.n - 1) * a.H + h) * a.qrow;
+#pragma unroll
+            for (int k = 0; k < kSteps; ++k) {
+                const int at = (d0 + k * KS + g * U) * (int)sizeof(T);
+                x[s][k] = ld16(q + min(at, a.plain - 16));
+                if (at >= a.plain) x[s][k] = u32x4{0, 0, 0, 0};
+            }
+        }
+        if (d0 > 0) __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) {
+            const int r = (tid + i * kSeqThreads) / kUnits, u = (tid + i * kSeqThreads) % kUnits;
+            *reinterpret_cast<u32x4*>(w + r * P + u * U) = b[i];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kSteps; ++k) {
+            T f[U];
+#pragma unroll
+            for (int e = 0; e < U; ++e) f[e] = w[(k * KS + g * U + e) * P + wave * 16 + col];
+            u32x4 fw;
+            __builtin_memcpy(&fw, f, 16);
+#pragma unroll
+            for (int s = 0; s < kAbsorbSets; ++s) acc[s] = mma16<T>(fw, x[s][k], acc[s]);
+        }
+    }
+    const int c = c0 + wave * 16 + g * 4;
+#pragma unroll
+    for (int s = 0; s < kAbsorbSets; ++s) {
+        const int t = t0 + s * 16 + col;
+        if (t < a.n && c < columns) store4<T>(a.out + ((size_t)t * a.H + h) * a.crow + (size_t)c * sizeof(T), acc[s]);
+    }
+    if (c0 != 0) return;
+    const int tail = (a.crow - a.pitch) / (int)sizeof(T), tokens = min(16 * kAbsorbSets, a.n - t0);  // rotated values, zeros behind them
+    for (int i = tid; i < tokens * tail; i += kSeqThreads) {
+        const int t = i / tail, j = i - t * tail;
+        const size_t row = (size_t)(t0 + t) * a.H + h;
+        reinterpret_cast<T*>(a.out + row * a.crow + a.pitch)[j] = j < a.R ? reinterpret_cast<const T*>(a.q + row * a.qrow + a.plain)[j] : from_f32<T>(0.0f);
+    }
+}
+
+// Workgroup (split, block of 16 S columns).  As k_seq_latent_attn, but every wave takes its part of S sets of columns at a time, so that a tile is read from
+// LDS once for all of them: a tile is a chain of barrier, reads, products, exchange of scores and softmax, which takes 1.4 us for one set,
+// 1.65 for two and 2.3 for four.  What bounds it is that chain.  128 heads, 40 tokens at 3000, 5120 columns: a workgroup of four waves per token and 32
+// heads 141 us; blocks of four sets whose softmax every wave does for itself 139, each set's softmax in one wave, the weights through LDS, 107; eight waves, two
+// on a SIMD, the score's products of different sets in turn and copies that the compiler does not wait for 79 (390 TFLOP/s with the weights' two parts).
+// Two buffers: the next tile's copies have the whole of this one's time.
+struct SeqLatentBlock {
+    const char* q;           // T [columns][crow bytes]
+    const char* kc;          // cache row of position 0
+    float *acc, *ml;         // [ns][columns][rp], [ns][columns][2]
+    float scale_log2;
+    int n, H, pos0, crow, ns, rp;
+};
+// Waves: KP of them share a score's dimensions, KG have keys of their own; each has NW latent columns of the sums.
+template <typename T, int NR> struct BlockWaves {
+    static constexpr int waves = NR >= 512 ? 8 : 4, kf = LatentTile<T>::keys / 16, groups = waves == 8 ? kf : 1, kp = waves / groups, keys = kf / groups;
+    static constexpr int columns = NR / waves, steps = LatentLds<T, NR>::ksteps / kp;
+    static_assert(LatentLds<T, NR>::ksteps % kp == 0 && columns % 32 == 0, "");
+};
+template <typename T, int NR, int S>
+__global__ __launch_bounds__((kWave * BlockWaves<T, NR>::waves)) void k_seq_latent_block(SeqLatentBlock a) {
+    using L = LatentLds<T, NR>;
+    using B = BlockWaves<T, NR>;
+    constexpr int KT = LatentTile<T>::keys, KF = B::kf, W = B::waves, KP = B::kp, KS = B::steps, KW = B::keys, NW = B::columns;
+    constexpr int kWeights = sizeof(T) == 2 ? 2 : 1;     // 16-byte units of a lane's weights
+    static_assert(S <= W, "");
+    extern __shared__ __align__(1024) char tiles[];
+    __shared__ f32x4 parts[S * KP * KF * kWave];         // scores of one part of the dimensions
+    __shared__ u32x4 weights[S * kWeights * kWave];
+    __shared__ float moved[S * 16];                      // what a column's sums are multiplied by
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 15, g = lane >> 4;
+    const int kp = wave % KP, key0 = wave / KP * KW;     // the wave's dimensions, and its first set of 16 keys
+    const int ncols = a.n * a.H, c0 = (int)blockIdx.y * 16 * S, sp = blockIdx.x;
+    const int end = a.pos0 + min(c0 + 16 * S - 1, ncols - 1) / a.H + 1, ntiles = (end + KT - 1) / KT;      // keys that the block's last token sees
+    const int k0 = mul_div(ntiles, sp, a.ns) * KT, k1 = min(mul_div(ntiles, sp + 1, a.ns) * KT, end);
+    const int ksteps = a.crow / 64, units = a.crow / 16;
+    auto stage = [&](uint32_t tile, int kb) __attribute__((always_inline)) {  // 64 units of the tile per copy, the waves in turn
+        constexpr int kCopies = L::copies * kSeqWaves;
+#pragma unroll
+        for (int i = 0; i < (kCopies + W - 1) / W; ++i) {
+            const int c = i * W + wave, l = c * 64 + lane, r = l / L::up, u = l - r * L::up;
+            if (c < kCopies) copy_to_lds16_from(a.kc + (size_t)min(kb + r, k1 - 1) * a.crow + min(u, units - 1) * 16, tile + c * 1024);
+        }
+    };
+    const uint32_t l0 = lds_address(tiles);
+    if (k0 < k1) stage(l0, k0);
+    u32x4 qf[S][KS];
+    f32x4 acc[S][NW / 16];
+    // wave s has the maxima and denominators of set s
+    float m = kNegBig, l = 0.0f;
+    const int seen = min(k1, a.pos0 + min(c0 + min(wave, S - 1) * 16 + col, ncols - 1) / a.H + 1);    // end of the keys that the column sees
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        const int c = min(c0 + s * 16 + col, ncols - 1);
+        const char* qr = a.q + (size_t)c * a.crow + g * 16;
+#pragma unroll
+        for (int d = 0; d < KS; ++d) {
+            qf[s][d] = ld16(qr + min(kp * KS + d, ksteps - 1) * 64);
+            if (kp * KS + d >= ksteps) qf[s][d] = u32x4{0, 0, 0, 0};
+        }
+#pragma unroll
+        for (int i = 0; i < NW / 16; ++i) acc[s][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    int buf = 0;
+    for (int kb = k0; kb < k1; kb += KT, buf ^= 1) {
+        // the tile is there, and nobody reads the other buffer any more
+        wait_vm<0>();
+        lds_barrier();
+        const char* const tile = tiles + buf * L::tile;
+        if (kb + KT < k1) stage(l0 + (buf ^ 1) * L::tile, kb + KT);
+        u32x4 kf[KS][KW];
+#pragma unroll
+        for (int d = 0; d < KS; ++d)
+#pragma unroll
+            for (int kt = 0; kt < KW; ++kt)
+                kf[d][kt] = *reinterpret_cast<const u32x4*>(tile + (((key0 + kt) * 16 + col) * L::up + (kp * KS + d) * 4 + g) * 16);
+        __builtin_amdgcn_sched_barrier(0);               // (all reads are requested before the first product waits for one)
+        f32x4 w[S][KW];
+#pragma unroll
+        for (int d = 0; d < KS; ++d)
+#pragma unroll
+            for (int kt = 0; kt < KW; ++kt)
+#pragma unroll
+                for (int s = 0; s < S; ++s) w[s][kt] = mma16<T>(kf[d][kt], qf[s][d], d == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : w[s][kt]);
+        __builtin_amdgcn_sched_barrier(0);               // (chains side by side, not one behind the other)
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+#pragma unroll
+            for (int kt = 0; kt < KW; ++kt) parts[((s * KP + kp) * KF + key0 + kt) * kWave + lane] = w[s][kt];
+        lds_barrier();
+        if (wave < S) {
+            f32x4 x[KF], p[KF][KP];
+            float top = kNegBig, sum = 0.0f;
+#pragma unroll
+            for (int kt = 0; kt < KF; ++kt)
+#pragma unroll
+                for (int v = 0; v < KP; ++v) p[kt][v] = parts[((wave * KP + v) * KF + kt) * kWave + lane];
+#pragma unroll
+            for (int kt = 0; kt < KF; ++kt) {
+                x[kt] = p[kt][0];
+#pragma unroll
+                for (int v = 1; v < KP; ++v) x[kt] += p[kt][v];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    x[kt][r] = kb + kt * 16 + g * 4 + r < seen ? x[kt][r] * a.scale_log2 : kMasked;
+                    top = fmaxf(top, x[kt][r]);
+                }
+            }
+            top = fmaxf(m, rows_max<16>(top));
+            const float c = fast_exp2(m - top);
+            m = top;
+#pragma unroll
+            for (int kt = 0; kt < KF; ++kt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    x[kt][r] = fast_exp2(x[kt][r] - m);
+                    sum += x[kt][r];
+                }
+            l = l * c + rows_sum<16>(sum);
+            if (g == 0) moved[wave * 16 + col] = c;
+            u32x4* const to = weights + wave * kWeights * kWave + lane;
+            if constexpr (sizeof(T) == 2) {
+                u32x4 hi, lo;
+                split_weights(x[0], x[1], hi, lo);
+                to[0] = hi;
+                to[kWave] = lo;
+            } else {
+                to[0] = __builtin_bit_cast(u32x4, x[0]);
+            }
+        }
+        lds_barrier();
+        u32x4 hi[S], lo[S];
+        float c[S];
+        bool any = false;
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            c[s] = moved[s * 16 + col];
+            hi[s] = weights[s * kWeights * kWave + lane];
+            if constexpr (kWeights == 2) lo[s] = weights[(s * kWeights + 1) * kWave + lane];
+        }
+#pragma unroll
+        for (int s = 0; s < S; ++s) any = any || c[s] != 1.0f;
+        if (__builtin_amdgcn_ballot_w64(any) != 0) {
+#pragma unroll
+            for (int s = 0; s < S; ++s)
+#pragma unroll
+                for (int i = 0; i < NW / 16; ++i) acc[s][i] *= c[s];
+        }
+        if constexpr (sizeof(T) == 2) {
+            constexpr int R = NW / 16 >= 8 ? 8 : 2;      // sets of 16 columns read together
+            const uint32_t v = (uint32_t)(uintptr_t)(tile + (4 * g + (col >> 2)) * L::up * 16 + wave * NW * 2 + (col & 3) * 8);
+#pragma unroll
+            for (int i = 0; i < NW / 16; i += R) {
+                TrCols f[R];
+                if constexpr (R == 8) tr_read8(f, v + i * 32, v + i * 32 + 16 * L::up * 16);
+                else tr_read2(f, v + i * 32, v + i * 32 + 16 * L::up * 16);
+#pragma unroll
+                for (int part = 0; part < 2; ++part)
+#pragma unroll
+                    for (int j = 0; j < R; ++j)
+#pragma unroll
+                        for (int s = 0; s < S; ++s)
+                            acc[s][i + j] = mma16<T>(u32x4{f[j].x.x, f[j].x.y, f[j].y.x, f[j].y.y}, part == 0 ? hi[s] : lo[s], acc[s][i + j]);
+            }
+        } else {
+            const char* v = tile + 4 * g * L::up * 16 + (wave * NW + col) * 4;
+#pragma unroll
+            for (int i = 0; i < NW / 16; ++i) {
+                f32x4 f;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) f[j] = *reinterpret_cast<const float*>(v + j * L::up * 16 + i * 64);
+#pragma unroll
+                for (int s = 0; s < S; ++s) acc[s][i] = mma16<T>(__builtin_bit_cast(u32x4, f), hi[s], acc[s][i]);
+            }
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        const int c = c0 + s * 16 + col;
+        if (c >= ncols) continue;
+        const size_t row = (size_t)sp * ncols + c;
+        if (wave == s && g == 0) *reinterpret_cast<float2*>(a.ml + row * 2) = make_float2(m, l);
+#pragma unroll
+        for (int i = 0; i < NW / 16; ++i)
+            if (wave * NW + i * 16 < a.rp) *reinterpret_cast<f32x4*>(a.acc + row * a.rp + wave * NW + i * 16 + g * 4) = acc[s][i];
+    }
+}
+
+// Workgroup (head, up to 16 tokens, `rows` of the head's outputs): merges the splits of these columns, then its rows of W_uv, and the output gate.  The
+// latents lie in LDS as fp32 or as two bf16 parts, which keep 16 of their bits.  Bound by round trips and, with many columns, by the partial results, which
+// the workgroups of a head read once each (half of V): 16 heads, 8 tokens in 64 splits 9 us, 128 heads, 40 tokens in 3 splits 23 us.  A workgroup for
+// each token and 16 outputs, as for one token, took 22 and, with 128 heads, 149 us for 40 tokens.
+constexpr int kTurnSplits = 64;
+struct SeqLatentTurnOut {
+    const float *acc, *ml;
+    const float* sink;       // nullable
+    const float* gate;       // nullable: [tokens][ldg] before the sigmoid
+    const char* w_uv;        // T [H * V][pitch bytes]
+    char* out;               // T [tokens][ldo bytes]
+    int n, tokens, H, V, rows, pitch, ns, rp, ldg, ldo;      // tokens: of a workgroup
+};
+template <typename T>
+__global__ __launch_bounds__(kSeqThreads) void k_seq_latent_turn_out(SeqLatentTurnOut a) {
+    constexpr int U = Unit<T>::n, kParts = sizeof(T) == 2 ? 2 : 1, kM = 16, kW = 16;
+    __shared__ float f[16][kTurnSplits];
+    extern __shared__ __align__(16) char lat[];          // [kParts][16][pitch + 16 bytes]
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 15, g = lane >> 4, h = blockIdx.x;
+    const int t0 = blockIdx.y * a.tokens, nt = min(a.tokens, a.n - t0), lrow = a.pitch + 16, ncols = a.n * a.H;
+    const float snk = a.sink != nullptr ? a.sink[h] * kLog2e : kNegBig;
+    // the wave's first rows of W_uv are on their way beside the merge
+    const int steps = a.pitch / 64, v1 = min(a.V, ((int)blockIdx.z + 1) * a.rows);
+    u32x4 fw[kW];
+    auto rows_at = [&](int v0) { return a.w_uv + ((size_t)h * a.V + min(v0 + col, a.V - 1)) * a.pitch + g * 16; };
+    auto request = [&](const char* w, int k) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < kW; ++i) fw[i] = ld16(w + min(k + i, steps - 1) * 64);
+    };
+    const int first = blockIdx.z * a.rows + wave * 16;
+    const int r4 = a.rp / 4, c4 = a.pitch / (int)sizeof(T) / 4;      // groups of four latents, of four columns of a row of W_uv
+    f32x4 y[kM];
+    auto ask = [&](int i, int s0) __attribute__((always_inline)) {
+        const int t = i / c4, x = i - t * c4;
+        const float* p = a.acc + ((size_t)(t0 + min(t, nt - 1)) * a.H + h) * a.rp + min(x, r4 - 1) * 4;
+#pragma unroll
+        for (int j = 0; j < kM; ++j) {
+            if (j % 4 == 0 && s0 + j >= a.ns) break;     // (the same for the workgroup)
+            y[j] = *reinterpret_cast<const f32x4*>(p + (size_t)min(s0 + j, a.ns - 1) * ncols * a.rp);
+        }
+    };
+    // (a lane has a split)
+    constexpr int kT = 16 / kSeqWaves;
+    float2 ml[kT];
+#pragma unroll
+    for (int j = 0; j < kT; ++j)
+        ml[j] = *reinterpret_cast<const float2*>(a.ml + ((size_t)min(lane, a.ns - 1) * ncols + (size_t)(t0 + min(wave + j * kSeqWaves, nt - 1)) * a.H + h) * 2);
+    ask(tid, 0);
+    request(rows_at(first), 0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < kT; ++j) {
+        const int t = wave + j * kSeqWaves;
+        if (t >= nt) break;
+        const float2 z = lane < a.ns ? ml[j] : make_float2(kNegBig, 0.0f);
+        const float m = wave_max(fmaxf(z.x, snk)), e = fast_exp2(z.x - m);
+        const float l = wave_sum(z.y * e) + (a.sink != nullptr ? fast_exp2(snk - m) : 0.0f);
+        f[t][lane] = e / l;
+    }
+    __syncthreads();
+    for (int i = tid; i < nt * c4; i += kSeqThreads) {
+        const int t = i / c4, x = i - t * c4;
+        f32x4 s = {0.f, 0.f, 0.f, 0.f};
+        if (i != tid) ask(i, 0);
+        for (int s0 = 0;;) {
+#pragma unroll
+            for (int j = 0; j < kM; ++j) {
+                if (j % 4 == 0 && s0 + j >= a.ns) break;
+                const bool live = s0 + j < a.ns && x < r4;           // (a split's values may be infinite: not times zero)
+                const float w = f[t][min(s0 + j, a.ns - 1)];
+#pragma unroll
+                for (int c = 0; c < 4; ++c) s[c] = live ? fmadd(y[j][c], w, s[c]) : s[c];
+            }
+            s0 += kM;
+            if (s0 >= a.ns) break;
+            ask(i, s0);
+        }
+        char* to = lat + t * lrow + x * 4 * (int)sizeof(T);
+        if constexpr (kParts == 2) {
+            const u32x2 hi = {pack_bf16(s[0], s[1]), pack_bf16(s[2], s[3])};
+            *reinterpret_cast<u32x2*>(to) = hi;
+            *reinterpret_cast<u32x2*>(to + 16 * lrow) = u32x2{pack_bf16(s[0] - __uint_as_float(hi.x << 16), s[1] - __uint_as_float(hi.x & 0xffff0000u)),
+                                                             pack_bf16(s[2] - __uint_as_float(hi.y << 16), s[3] - __uint_as_float(hi.y & 0xffff0000u))};
+        } else {
+            *reinterpret_cast<f32x4*>(to) = s;
+        }
+    }
+    __syncthreads();
+    const char* x = lat + min(col, nt - 1) * lrow + g * 16;
+    for (int v0 = first; v0 < v1; v0 += 16 * kSeqWaves) {
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        for (int k = 0; k < steps; k += kW) {
+            if (v0 != first || k > 0) request(rows_at(v0), k);
+#pragma unroll
+            for (int i = 0; i < kW; ++i) {
+                if (k + i >= steps) break;
+#pragma unroll
+                for (int j = 0; j < kParts; ++j) acc = mma16<T>(fw[i], *reinterpret_cast<const u32x4*>(x + j * 16 * lrow + (k + i) * 64), acc);
+            }
+        }
+        if (col < nt) {
+            T* o = reinterpret_cast<T*>(a.out + (size_t)(t0 + col) * a.ldo) + (size_t)h * a.V;
+            const float* gate = a.gate + (size_t)(t0 + col) * a.ldg + (size_t)h * a.V;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int v = v0 + g * 4 + r;
+                if (v < v1) o[v] = from_f32<T>(a.gate != nullptr ? acc[r] * sigmoid(gate[v]) : acc[r]);
+            }
         }
     }
 }

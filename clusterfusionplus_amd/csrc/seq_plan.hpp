@@ -174,4 +174,46 @@ inline AttnPlan plan_attn(const AttnSizes& a, int cus, size_t room) {
     return {two, splits, rows, a.per_cu >= 2 && total <= 3 * cus && alike ? std::min(some, rows / 2) : 0};
 }
 
+// A portion of few tokens behind many positions: latent attention may read the cached latents themselves instead of the keys and values that are
+// made of them.  A column (token, head) then takes products of `rank` values with every key instead of dim and vdim of them, and leaves sums of `rank` values
+// for each split; keys and values cost the same for one token as for a hundred.  Where the line is follows from an estimate of both, with
+// coefficients fitted to the difference measured over latent_2b, latent_6b9, latent_wide and a small uneven model (16, 32, 128 and 12 heads), 2 to 150 tokens at
+// 200, 1000, 3000 and 4000 (bf16: 128 differences, 6 us off on average; fp32: the uneven model alone).  In us per layer, made and read: 16 heads at 3000,
+// 2 tokens 108 / 91, 20 110 / 104, 40 113 / 112, 64 118 / 124; 128 heads at 3000, 2 tokens 411 / 282, 20 429 / 342, 64 480 / 469, 100 514 / 588; at 1000,
+// 20 333 / 319, 64 406 / 409; at 200, 10 300 / 302; 12 heads in fp32 at 3000, 2 tokens 111 / 85, 20 121 / 110, 64 139 / 164.  Not chosen within 4 us, which
+// is what the estimate misses small models by.  n tokens at pos and on; dim, rot, vdim: values of a head's key (plain, rotated) and value; bytes of a latent row, latents of it.
+struct LatentSizes {
+    int n, pos, heads, dim, rot, vdim, kbytes, rank;
+    bool bf16;
+    size_t room;             // floats for partial results
+};
+// splits 0: keys and values are made.  sets: of 16 columns in a block; tokens, rows: of a workgroup that merges and multiplies by W_uv.
+struct LatentTurn { int splits, sets, tokens, rows; };
+inline LatentTurn plan_latent_turn(const LatentSizes& z, int cus) {
+    if (z.n > 256) return {};                            // (not measured, and never near the line)
+    const int keys = z.bf16 ? 32 : 16, cols = z.n * z.heads, ctx = z.pos + z.n, tiles = ceil_div(ctx, keys), esize = z.bf16 ? 2 : 4;
+    const GemmSizes g{z.heads * (z.dim + z.vdim), ctx, z.kbytes, 0, 0};
+    const GemmPlan made = plan_gemm(g, z.bf16, cus);
+    const float gemm = gemm_cost(g, shapes_of(z.bf16)[made.shape], made.splits, cus);
+    const float mb = 1e-6f * ctx * g.n * esize, gflop = 2e-9f * ctx * cols * (z.dim + z.rot + z.vdim);
+    const float least = z.bf16 ? 14.0f + 0.86f * gemm + 0.067f * mb + 1.3f * gflop : 1.0f + 0.7f * gemm + 0.26f * mb + 0.3f * gflop;
+    LatentTurn best{};
+    float cost = least - 4.0f;                           // (of what is chosen: a round of workgroups, its tiles, partial results, columns)
+    const int most = (int)std::min<size_t>({(size_t)64, z.room / ((size_t)cols * (z.rank + 2)), (size_t)ceil_div(tiles, 2)});
+    for (int sets : {1, 2, 4}) {
+        const float tile = sets == 1 ? 1.4f : sets == 2 ? 1.65f : 2.3f;
+        for (int splits = 1; splits <= most; ++splits) {
+            const float rounds = (float)ceil_div(ceil_div(cols, 16 * sets) * splits, cus), walk = rounds * ceil_div(tiles, splits) * tile;
+            const float parts = 4e-6f * cols * splits * z.rank;
+            const float t = z.bf16 ? 16.0f * rounds + 0.83f * walk + 0.44f * parts + 3.2e-3f * cols : 0.6f * rounds + 1.3f * walk + 0.6f * parts + 4e-3f * cols;
+            if (t < cost) {
+                cost = t;
+                best = {splits, sets, 16, 64};
+            }
+        }
+    }
+    while (best.tokens > 2 && z.heads * ceil_div(z.vdim, best.rows) * ceil_div(z.n, best.tokens) < cus) best.tokens /= 2;
+    return best;
+}
+
 }  // namespace cfpp
