@@ -910,6 +910,8 @@ struct SeqStreams {
     int pitch;
     float* copy;             // nullable: receives the sum of the streams
     const int* rows;         // nullable: take token rows[t], write input t
+    int way;                 // k_seq_streams4: one of kStreams..
+    const float *y0, *mix0, *out0;       // ... kStreamsAgain: the update that was not stored
     // the start
     const int* tokens;       // null: not the start
     const int* state;        // not null: one token, its position from here instead of pos0 + t
@@ -1022,18 +1024,28 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_streams(SeqStreams a) {
 // before anything is used.  That is for portions of few tokens, where a row is a chain of round trips; with many, both kernels are bound
 // by their bytes.  Four streams of 4096 values, 37 tokens: 12.7 -> 9.8 us, 150: 15.4 -> 12.0, 512: 25.8 -> 20.4, 1000: 34.7 and 34.8, 8000:
 // 220 and 213; two of 2048, 37 tokens: 7.9 -> 5.8 us, 512: 8.3 and 8.2, 8000: 57 and 59.
-template <typename T, int S, int U>
+//
+// Portions of many tokens are bound by their bytes, most of which are the streams (M: what the kernel does with them, kStreamsStay and kStreamsAgain where
+// streams_later says so).  The update after a mixer is not stored: only the next input is needed of it.  The update after the feed-forward makes it again,
+// from the same values in the same order, and reads one row more for that, where a row for each stream is not written.  The streams go past the caches,
+// which leaves those to the sublayers' outputs.  Four streams of 4096 values, 8000 tokens: 220 + 220 us -> 140 + 269 (5.1 TB/s); without the latter 160 + 276.
+enum : int { kStreamsKept = 0, kStreamsStay = 1, kStreamsAgain = 2 };
+template <typename T, int S, int U, int M>
 __global__ __launch_bounds__(kSeqThreads) void k_seq_streams4(SeqStreams a) {
     __shared__ float red[kSeqWaves];
     const int t = a.rows != nullptr ? a.rows[blockIdx.x] : (int)blockIdx.x, tid = threadIdx.x, n4 = a.width / 4;
     float* x = a.x + (size_t)t * a.streams * a.width;
-    f32x4 o[S][U], w[U], y[U];
+    f32x4 o[S][U], w[U], y[U], z[M == kStreamsAgain ? U : 1];
+    auto load_stream = [](const float* p, int i) __attribute__((always_inline)) {
+        if constexpr (M != kStreamsKept) return __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p) + i);
+        else return reinterpret_cast<const f32x4*>(p)[i];
+    };
 #pragma unroll
     for (int j = 0; j < U; ++j) {
         const int i = min(tid + j * kSeqThreads, n4 - 1);
         if (a.tokens == nullptr) {
 #pragma unroll
-            for (int s = 0; s < S; ++s) o[s][j] = reinterpret_cast<const f32x4*>(x + (size_t)min(s, a.streams - 1) * a.width)[i];
+            for (int s = 0; s < S; ++s) o[s][j] = load_stream(x + (size_t)min(s, a.streams - 1) * a.width, i);
         } else {
             const T* e = reinterpret_cast<const T*>(a.embed + (size_t)a.tokens[t] * a.embed_pitch) + i * 4;
             const T* p = a.pos != nullptr ? reinterpret_cast<const T*>(a.pos + (size_t)(a.state != nullptr ? a.state[1] : a.pos0 + t) * a.embed_pitch) + i * 4 : nullptr;
@@ -1044,6 +1056,7 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_streams4(SeqStreams a) {
         }
         w[j] = a.w != nullptr ? reinterpret_cast<const f32x4*>(a.w)[i] : f32x4{0.f, 0.f, 0.f, 0.f};
         y[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if constexpr (M == kStreamsAgain) z[j] = reinterpret_cast<const f32x4*>(a.y0 + (size_t)t * a.width)[i];
     }
     if (a.ys != nullptr) {
         add_rows4<U, 2>(y, a.ys + (size_t)t * a.top * a.width, a.top, a.width, n4);
@@ -1055,23 +1068,25 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_streams4(SeqStreams a) {
 #pragma unroll
     for (int j = 0; j < U; ++j) {
         const int i = tid + j * kSeqThreads;
-        if (a.tokens == nullptr && a.mix != nullptr) {
+        auto update = [&](const float* mix, const float* out, f32x4 y) __attribute__((always_inline)) {
             f32x4 v[S];
 #pragma unroll
             for (int s = 0; s < S; ++s) {
                 const bool live = s < a.streams;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) v[s][r] = (live ? a.out[s] : 0.0f) * y[j][r];
+                for (int r = 0; r < 4; ++r) v[s][r] = (live ? out[s] : 0.0f) * y[r];
 #pragma unroll
                 for (int k = 0; k < S; ++k) {
-                    const float m = live && k < a.streams ? a.mix[k * a.streams + s] : 0.0f;
+                    const float m = live && k < a.streams ? mix[k * a.streams + s] : 0.0f;
 #pragma unroll
                     for (int r = 0; r < 4; ++r) v[s][r] = fmadd(m, o[k][j][r], v[s][r]);
                 }
             }
 #pragma unroll
             for (int s = 0; s < S; ++s) o[s][j] = v[s];
-        }
+        };
+        if constexpr (M == kStreamsAgain) update(a.mix0, a.out0, z[j]);
+        if (a.tokens == nullptr && a.mix != nullptr) update(a.mix, a.out, y[j]);
         f32x4 u = {0.f, 0.f, 0.f, 0.f}, all = u;
 #pragma unroll
         for (int s = 0; s < S; ++s)
@@ -1082,10 +1097,13 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_streams4(SeqStreams a) {
                 all += o[s][j];
             }
         if (i < n4) {
-            if (a.rows == nullptr) {
+            if (a.rows == nullptr && M != kStreamsStay) {
 #pragma unroll
                 for (int s = 0; s < S; ++s)
-                    if (s < a.streams) reinterpret_cast<f32x4*>(x + (size_t)s * a.width)[i] = o[s][j];
+                    if (s < a.streams) {
+                        if constexpr (M == kStreamsAgain) __builtin_nontemporal_store(o[s][j], reinterpret_cast<f32x4*>(x + (size_t)s * a.width) + i);
+                        else reinterpret_cast<f32x4*>(x + (size_t)s * a.width)[i] = o[s][j];
+                    }
             }
             if (a.copy != nullptr) reinterpret_cast<f32x4*>(a.copy + (size_t)t * a.width)[i] = all;
 #pragma unroll
