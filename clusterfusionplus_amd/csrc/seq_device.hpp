@@ -194,6 +194,11 @@ template <typename T> __device__ __forceinline__ void store4(void* p, f32x4 v) {
         *reinterpret_cast<u32x2*>(p) = u32x2{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
     }
 }
+// Four values of a row; `once`: nobody reads them again, and they leave the caches to the others'.
+template <bool once> __device__ __forceinline__ f32x4 load_row4(const float* row, int i) {
+    if constexpr (once) return __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(row) + i);
+    else return reinterpret_cast<const f32x4*>(row)[i];
+}
 // two values to T, 8 or 4 bytes
 template <typename T> __device__ __forceinline__ void store2(void* p, float a, float b) {
     if constexpr (sizeof(T) == 4) *reinterpret_cast<float2*>(p) = make_float2(a, b);

@@ -86,25 +86,27 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_latent_finish(SeqLatentFini
 // The same where the row is whole groups of four values, up to 1024 U of them: everything is requested at once (of C parts together), and the
 // row is read from LDS, where it took three or four round trips.  Gates are read only where they come in parts, and their sum goes back.
 // 8000 tokens of 6720 values and 4096 gates: 100 -> 71 us for 330 MB.  U = 4 where the row fits, since places behind its end are requested like others:
-// 150 tokens of 3648 in parts 6.4 us, with 8 groups 5.6, with 4 5.0; 100 of 1120 in parts 4.5, 5.6 and 4.7.
+// 150 tokens of 3648 in parts 6.4 us, with 8 groups 5.6, with 4 5.0; 100 of 1120 in parts 4.5, 5.6 and 4.7.  C = 0: a projection
+// that is larger than the 256 MB cache is read from its end, and past the caches: 8000 tokens of 10816 values, of which 6720 are read, 71 -> 57 us (2048
+// tokens 21.4 and 21.7, 4000 32 and 32; in rows of queries, keys and values 71 -> 67 for 8000 and 21.6 -> 22.4 for 2048, not done there).
 template <typename T, int U, int C>
 __global__ __launch_bounds__(kSeqThreads) void k_seq_latent_finish4(SeqLatentFinish a) {
     __shared__ float red[kSeqWaves];
     extern __shared__ __align__(16) char smem[];
     float* const row = reinterpret_cast<float*>(smem);   // [made], then the position's pairs
     float2* const pairs = reinterpret_cast<float2*>(row + a.made);
-    const int t = blockIdx.x, tid = threadIdx.x, n = a.D + a.R, n4 = a.n / 4, kv0 = a.H * n;
+    const int t = C == 0 ? (int)(gridDim.x - 1 - blockIdx.x) : (int)blockIdx.x, tid = threadIdx.x, n = a.D + a.R, n4 = a.n / 4, kv0 = a.H * n;
     float* const z = a.z + (size_t)t * a.ld;
     f32x4 x[U];
 #pragma unroll
-    for (int j = 0; j < U; ++j) x[j] = reinterpret_cast<const f32x4*>(z)[min(tid + j * kSeqThreads, n4 - 1)];
+    for (int j = 0; j < U; ++j) x[j] = load_row4<C == 0>(z, min(tid + j * kSeqThreads, n4 - 1));
     constexpr int kNorm = 2;                             // (a latent has 512 values at most)
     float w[kNorm];
 #pragma unroll
     for (int j = 0; j < kNorm; ++j) w[j] = a.own ? a.kv.w[min(tid + j * kSeqThreads, a.kv.rank - 1)] : 0.0f;
     float2 pair = make_float2(0.0f, 0.0f);
     if (tid < a.R / 2) pair = a.cs[(size_t)(a.pos0 + t) * (a.R / 2) + tid];
-    add_rows4<U, C>(x, z + a.part_stride, a.parts - 1, a.part_stride, n4);
+    add_rows4<U, (C > 0 ? C : 1)>(x, z + a.part_stride, a.parts - 1, a.part_stride, n4);
     float ss = 0.0f;
 #pragma unroll
     for (int j = 0; j < U; ++j) {
@@ -1036,16 +1038,12 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_streams4(SeqStreams a) {
     const int t = a.rows != nullptr ? a.rows[blockIdx.x] : (int)blockIdx.x, tid = threadIdx.x, n4 = a.width / 4;
     float* x = a.x + (size_t)t * a.streams * a.width;
     f32x4 o[S][U], w[U], y[U], z[M == kStreamsAgain ? U : 1];
-    auto load_stream = [](const float* p, int i) __attribute__((always_inline)) {
-        if constexpr (M != kStreamsKept) return __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p) + i);
-        else return reinterpret_cast<const f32x4*>(p)[i];
-    };
 #pragma unroll
     for (int j = 0; j < U; ++j) {
         const int i = min(tid + j * kSeqThreads, n4 - 1);
         if (a.tokens == nullptr) {
 #pragma unroll
-            for (int s = 0; s < S; ++s) o[s][j] = load_stream(x + (size_t)min(s, a.streams - 1) * a.width, i);
+            for (int s = 0; s < S; ++s) o[s][j] = load_row4<M != kStreamsKept>(x + (size_t)min(s, a.streams - 1) * a.width, i);
         } else {
             const T* e = reinterpret_cast<const T*>(a.embed + (size_t)a.tokens[t] * a.embed_pitch) + i * 4;
             const T* p = a.pos != nullptr ? reinterpret_cast<const T*>(a.pos + (size_t)(a.state != nullptr ? a.state[1] : a.pos0 + t) * a.embed_pitch) + i * 4 : nullptr;
@@ -1056,7 +1054,7 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_streams4(SeqStreams a) {
         }
         w[j] = a.w != nullptr ? reinterpret_cast<const f32x4*>(a.w)[i] : f32x4{0.f, 0.f, 0.f, 0.f};
         y[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if constexpr (M == kStreamsAgain) z[j] = reinterpret_cast<const f32x4*>(a.y0 + (size_t)t * a.width)[i];
+        if constexpr (M == kStreamsAgain) z[j] = load_row4<true>(a.y0 + (size_t)t * a.width, i);
     }
     if (a.ys != nullptr) {
         add_rows4<U, 2>(y, a.ys + (size_t)t * a.top * a.width, a.top, a.width, n4);
