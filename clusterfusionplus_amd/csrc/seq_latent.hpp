@@ -592,6 +592,10 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_latent_absorb(SeqLatentAbso
     }
 }
 
+// What weights and denominators are multiplied by, so that sums of a million latents stay within the range of the latents themselves: values made of latents
+// of any size may be small, and have sums that are in range.  A power of two, so outputs are the same bits without it wherever sums are in range.
+constexpr float kBlockWeight = 1.0f / (1 << 20);
+
 // Workgroup (split, block of 16 S columns).  As k_seq_latent_attn, but every wave takes its part of S sets of columns at a time, so that a tile is read from
 // LDS once for all of them: a tile is a chain of barrier, reads, products, exchange of scores and softmax, which takes 1.4 us for one set,
 // 1.65 for two and 2.3 for four.  What bounds it is that chain.  128 heads, 40 tokens at 3000, 5120 columns: a workgroup of four waves per token and 32
@@ -601,7 +605,7 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_latent_absorb(SeqLatentAbso
 struct SeqLatentBlock {
     const char* q;           // T [columns][crow bytes]
     const char* kc;          // cache row of position 0
-    float *acc, *ml;         // [ns][columns][rp], [ns][columns][2]
+    float *acc, *ml;         // [ns][columns][rp], [ns][columns][2]: sums and denominators times kBlockWeight
     float scale_log2;
     int n, H, pos0, crow, ns, rp;
 };
@@ -707,7 +711,7 @@ __global__ __launch_bounds__((kWave * BlockWaves<T, NR>::waves)) void k_seq_late
             for (int kt = 0; kt < KF; ++kt)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    x[kt][r] = fast_exp2(x[kt][r] - m);
+                    x[kt][r] = fast_exp2(x[kt][r] - m) * kBlockWeight;
                     sum += x[kt][r];
                 }
             l = l * c + rows_sum<16>(sum);
@@ -781,7 +785,8 @@ __global__ __launch_bounds__((kWave * BlockWaves<T, NR>::waves)) void k_seq_late
 }
 
 // Workgroup (head, up to 16 tokens, `rows` of the head's outputs): merges the splits of these columns, then its rows of W_uv, and the output gate.  The
-// latents lie in LDS as fp32 or as two bf16 parts, which keep 16 of their bits.  Bound by round trips and, with many columns, by the partial results, which
+// latents lie in LDS as fp32 or as two bf16 parts, which keep 16 of their bits (they are finite unless a cached latent is not, and then its scores are
+// no numbers either).  Bound by round trips and, with many columns, by the partial results, which
 // the workgroups of a head read once each (half of V): 16 heads, 8 tokens in 64 splits 9 us, 128 heads, 40 tokens in 3 splits 23 us.  A workgroup for
 // each token and 16 outputs, as for one token, took 22 and, with 128 heads, 149 us for 40 tokens.
 constexpr int kTurnSplits = 64;
@@ -836,7 +841,7 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_latent_turn_out(SeqLatentTu
         if (t >= nt) break;
         const float2 z = lane < a.ns ? ml[j] : make_float2(kNegBig, 0.0f);
         const float m = wave_max(fmaxf(z.x, snk)), e = fast_exp2(z.x - m);
-        const float l = wave_sum(z.y * e) + (a.sink != nullptr ? fast_exp2(snk - m) : 0.0f);
+        const float l = wave_sum(z.y * e) + (a.sink != nullptr ? fast_exp2(snk - m) * kBlockWeight : 0.0f);
         f[t][lane] = e / l;
     }
     __syncthreads();

@@ -65,3 +65,22 @@ def test_turns(name, dtype):
         got = m.forward(0, toks[pos:pos + n], pos, range(n))
         assert M.error(got, want[pos:pos + n]) < LIMIT[dtype]
         pos += n
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+def test_large_latents(dtype):
+    """A latent value near the end of the range, alike for all positions, which only small rows of W_uv read: weighted sums of it stay in range."""
+    cfg, pos, _ = TURNS["rank_of_100"]
+    w, toks, m = dict(M.weights(cfg, 5)), M.prompt(cfg, pos + 4, 6), "l0.mix."
+    for n in ("embed", "pos"):
+        w[n] = w[n].clone()
+        w[n][:, 1] = 3.0 if n == "embed" else 0.0
+    w[m + "dkv"][7] = 0
+    w[m + "dkv"][7, 1] = 1.0
+    w[m + "dkv.norm"][7], w[m + "uk"][:, 7] = 2.0 ** 124, 0
+    w[m + "uv"][:, 7] = torch.sign(w[m + "uv"][:, 7].float()).bfloat16() * 2.0 ** -124
+    assert P.turn(4, pos, cfg["layers"][0]["mixer"], dtype == torch.bfloat16, P.room(cfg["max_positions"], cfg["width"]))[0] > 0
+    c = build(cfg, w, dtype, capacity=cfg["max_positions"])
+    c.forward(0, toks[:pos], 0, [pos - 1])
+    assert M.error(c.forward(0, toks[pos:], pos, range(4)), M.oracle(cfg, w, toks)[pos:]) < LIMIT[dtype]
