@@ -84,3 +84,20 @@ def test_large_latents(dtype):
     c = build(cfg, w, dtype, capacity=cfg["max_positions"])
     c.forward(0, toks[:pos], 0, [pos - 1])
     assert M.error(c.forward(0, toks[pos:], pos, range(4)), M.oracle(cfg, w, toks)[pos:]) < LIMIT[dtype]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+def test_values_that_are_not_finite_stay_in_their_sequence(dtype):
+    """Heads whose keys end inside a unit of 16 bytes: what lies behind them in the keys' buffer meets zeros of the queries, and has to be finite."""
+    cfg = M.model(64, 51, [M.sunk(40, 66, 8, 100, 100)], positions=1700)
+    w, toks, pos = dict(M.weights(cfg, 5)), [t or 1 for t in M.prompt(cfg, 1500, 6)], 1500
+    w["embed"] = w["embed"].clone()
+    w["embed"][0] = float("inf")
+    assert P.turn(6, pos, cfg["layers"][0]["mixer"], dtype == torch.bfloat16, P.room(cfg["max_positions"], cfg["width"]))[0] > 0
+    m = build(cfg, w, dtype, capacity=cfg["max_positions"], slots=2)
+    want = m.forward(0, toks, 0, range(pos))
+    assert torch.isfinite(want).all()
+    m.forward(1, toks, 0)
+    assert not torch.isfinite(m.forward(1, [0] * 6, pos, range(6))).any()
+    assert torch.equal(m.forward(0, toks, 0, range(pos)), want)
