@@ -13,6 +13,7 @@
 #include <type_traits>
 
 #include "seq_device.hpp"
+#include "seq_plan.hpp"
 
 namespace cfpp {
 
@@ -784,19 +785,19 @@ __global__ __launch_bounds__((kWave * BlockWaves<T, NR>::waves)) void k_seq_late
     }
 }
 
-// Workgroup (head, up to 16 tokens, `rows` of the head's outputs): merges the splits of these columns, then its rows of W_uv, and the output gate.  The
+// Workgroup (head, up to 16 tokens, kTurnRows of the head's outputs, 16 of a wave): merges the splits of these columns, then its rows of W_uv, and the output gate.  The
 // latents lie in LDS as fp32 or as two bf16 parts, which keep 16 of their bits (they are finite unless a cached latent is not, and then its scores are
 // no numbers either).  Bound by round trips and, with many columns, by the partial results, which
 // the workgroups of a head read once each (half of V): 16 heads, 8 tokens in 64 splits 9 us, 128 heads, 40 tokens in 3 splits 23 us.  A workgroup for
 // each token and 16 outputs, as for one token, took 22 and, with 128 heads, 149 us for 40 tokens.
-constexpr int kTurnSplits = 64;
+static_assert(kTurnSplits <= kWave && kTurnRows == 16 * kSeqWaves, "a lane has a split, a wave 16 rows");
 struct SeqLatentTurnOut {
     const float *acc, *ml;
     const float* sink;       // nullable
     const float* gate;       // nullable: [tokens][ldg] before the sigmoid
     const char* w_uv;        // T [H * V][pitch bytes]
     char* out;               // T [tokens][ldo bytes]
-    int n, tokens, H, V, rows, pitch, ns, rp, ldg, ldo;      // tokens: of a workgroup
+    int n, tokens, H, V, pitch, ns, rp, ldg, ldo;            // tokens: of a workgroup
 };
 template <typename T>
 __global__ __launch_bounds__(kSeqThreads) void k_seq_latent_turn_out(SeqLatentTurnOut a) {
@@ -807,14 +808,13 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_latent_turn_out(SeqLatentTu
     const int t0 = blockIdx.y * a.tokens, nt = min(a.tokens, a.n - t0), lrow = a.pitch + 16, ncols = a.n * a.H;
     const float snk = a.sink != nullptr ? a.sink[h] * kLog2e : kNegBig;
     // the wave's first rows of W_uv are on their way beside the merge
-    const int steps = a.pitch / 64, v1 = min(a.V, ((int)blockIdx.z + 1) * a.rows);
+    const int steps = a.pitch / 64, v0 = (int)blockIdx.z * kTurnRows + wave * 16;
     u32x4 fw[kW];
-    auto rows_at = [&](int v0) { return a.w_uv + ((size_t)h * a.V + min(v0 + col, a.V - 1)) * a.pitch + g * 16; };
-    auto request = [&](const char* w, int k) __attribute__((always_inline)) {
+    const char* const w = a.w_uv + ((size_t)h * a.V + min(v0 + col, a.V - 1)) * a.pitch + g * 16;
+    auto request = [&](int k) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < kW; ++i) fw[i] = ld16(w + min(k + i, steps - 1) * 64);
     };
-    const int first = blockIdx.z * a.rows + wave * 16;
     const int r4 = a.rp / 4, c4 = a.pitch / (int)sizeof(T) / 4;      // groups of four latents, of four columns of a row of W_uv
     f32x4 y[kM];
     auto ask = [&](int i, int s0) __attribute__((always_inline)) {
@@ -833,7 +833,7 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_latent_turn_out(SeqLatentTu
     for (int j = 0; j < kT; ++j)
         ml[j] = *reinterpret_cast<const float2*>(a.ml + ((size_t)min(lane, a.ns - 1) * ncols + (size_t)(t0 + min(wave + j * kSeqWaves, nt - 1)) * a.H + h) * 2);
     ask(tid, 0);
-    request(rows_at(first), 0);
+    request(0);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < kT; ++j) {
@@ -873,27 +873,25 @@ __global__ __launch_bounds__(kSeqThreads) void k_seq_latent_turn_out(SeqLatentTu
         }
     }
     __syncthreads();
+    if (v0 >= a.V) return;
     const char* x = lat + min(col, nt - 1) * lrow + g * 16;
-    for (int v0 = first; v0 < v1; v0 += 16 * kSeqWaves) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        for (int k = 0; k < steps; k += kW) {
-            if (v0 != first || k > 0) request(rows_at(v0), k);
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int k = 0; k < steps; k += kW) {
+        if (k > 0) request(k);
 #pragma unroll
-            for (int i = 0; i < kW; ++i) {
-                if (k + i >= steps) break;
+        for (int i = 0; i < kW; ++i) {
+            if (k + i >= steps) break;
 #pragma unroll
-                for (int j = 0; j < kParts; ++j) acc = mma16<T>(fw[i], *reinterpret_cast<const u32x4*>(x + j * 16 * lrow + (k + i) * 64), acc);
-            }
+            for (int j = 0; j < kParts; ++j) acc = mma16<T>(fw[i], *reinterpret_cast<const u32x4*>(x + j * 16 * lrow + (k + i) * 64), acc);
         }
-        if (col < nt) {
-            T* o = reinterpret_cast<T*>(a.out + (size_t)(t0 + col) * a.ldo) + (size_t)h * a.V;
-            const float* gate = a.gate + (size_t)(t0 + col) * a.ldg + (size_t)h * a.V;
+    }
+    if (col >= nt) return;
+    T* o = reinterpret_cast<T*>(a.out + (size_t)(t0 + col) * a.ldo) + (size_t)h * a.V;
+    const float* gate = a.gate + (size_t)(t0 + col) * a.ldg + (size_t)h * a.V;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int v = v0 + g * 4 + r;
-                if (v < v1) o[v] = from_f32<T>(a.gate != nullptr ? acc[r] * sigmoid(gate[v]) : acc[r]);
-            }
-        }
+    for (int r = 0; r < 4; ++r) {
+        const int v = v0 + g * 4 + r;
+        if (v < a.V) o[v] = from_f32<T>(a.gate != nullptr ? acc[r] * sigmoid(gate[v]) : acc[r]);
     }
 }
 

@@ -187,8 +187,10 @@ struct LatentSizes {
     bool bf16;
     size_t room;             // floats for partial results
 };
-// splits 0: keys and values are made.  sets: of 16 columns in a block; tokens, rows: of a workgroup that merges and multiplies by W_uv.
-struct LatentTurn { int splits, sets, tokens, rows; };
+// splits 0: keys and values are made.  sets: of 16 columns in a block; tokens: of a workgroup that merges kTurnSplits splits at most and multiplies kTurnRows
+// rows of W_uv by them.
+struct LatentTurn { int splits, sets, tokens; };
+constexpr int kTurnSplits = 64, kTurnRows = 64;
 inline LatentTurn plan_latent_turn(const LatentSizes& z, int cus) {
     if (z.n > 256) return {};                            // (not measured, and never near the line)
     const int keys = z.bf16 ? 32 : 16, cols = z.n * z.heads, ctx = z.pos + z.n, tiles = ceil_div(ctx, keys), esize = z.bf16 ? 2 : 4;
@@ -199,7 +201,7 @@ inline LatentTurn plan_latent_turn(const LatentSizes& z, int cus) {
     const float least = z.bf16 ? 14.0f + 0.86f * gemm + 0.067f * mb + 1.3f * gflop : 1.0f + 0.7f * gemm + 0.26f * mb + 0.3f * gflop;
     LatentTurn best{};
     float cost = least - 4.0f;                           // (of what is chosen: a round of workgroups, its tiles, partial results, columns)
-    const int most = (int)std::min<size_t>({(size_t)64, z.room / ((size_t)cols * (z.rank + 2)), (size_t)ceil_div(tiles, 2)});
+    const int most = (int)std::min<size_t>({(size_t)kTurnSplits, z.room / ((size_t)cols * (z.rank + 2)), (size_t)ceil_div(tiles, 2)});
     for (int sets : {1, 2, 4}) {
         const float tile = sets == 1 ? 1.4f : sets == 2 ? 1.65f : 2.3f;
         for (int splits = 1; splits <= most; ++splits) {
@@ -208,11 +210,11 @@ inline LatentTurn plan_latent_turn(const LatentSizes& z, int cus) {
             const float t = z.bf16 ? 16.0f * rounds + 0.83f * walk + 0.44f * parts + 3.2e-3f * cols : 0.6f * rounds + 1.3f * walk + 0.6f * parts + 4e-3f * cols;
             if (t < cost) {
                 cost = t;
-                best = {splits, sets, 16, 64};
+                best = {splits, sets, 16};
             }
         }
     }
-    while (best.tokens > 2 && z.heads * ceil_div(z.vdim, best.rows) * ceil_div(z.n, best.tokens) < cus) best.tokens /= 2;
+    while (best.tokens > 2 && z.heads * ceil_div(z.vdim, kTurnRows) * ceil_div(z.n, best.tokens) < cus) best.tokens /= 2;
     return best;
 }
 

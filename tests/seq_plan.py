@@ -33,11 +33,10 @@ extern "C" int beside(int n, int top, int experts, int ff, int xbytes, int rows,
     const ExpertSizes e{n, top, experts, ff, xbytes};
     return plan_beside(e, plan_experts(e, bf16 != 0, cus), rows, kbytes, {shared_rows, n, shared_kbytes, ldy, (size_t)room}, bf16 != 0, cus);
 }
-extern "C" int turn(int n, int pos, int heads, int dim, int rot, int vdim, int kbytes, int rank, int bf16, long room, int cus, int* sets, int* tokens, int* rows) {
+extern "C" int turn(int n, int pos, int heads, int dim, int rot, int vdim, int kbytes, int rank, int bf16, long room, int cus, int* sets, int* tokens) {
     const LatentTurn t = plan_latent_turn({n, pos, heads, dim, rot, vdim, kbytes, rank, bf16 != 0, (size_t)room}, cus);
     *sets = t.sets;
     *tokens = t.tokens;
-    *rows = t.rows;
     return t.splits;
 }
 extern "C" int tile(int shape, int bf16) { return code(shape, 1, bf16 != 0); }
@@ -59,7 +58,7 @@ def lib():
     lib.product.argtypes = [i] * 4 + [l, i, i]
     lib.experts.argtypes = [i] * 7 + [p]
     lib.beside.argtypes = [i] * 10 + [l, i, i]
-    lib.turn.argtypes = [i] * 9 + [l, i, p, p, p]
+    lib.turn.argtypes = [i] * 9 + [l, i, p, p]
     lib.tile.argtypes = [i, i]
     lib.estimate.argtypes, lib.estimate.restype = [i] * 7, ctypes.c_float
     return lib
@@ -109,8 +108,8 @@ def experts(n, top, count, ff, width, bf16):
 
 
 def turn(n, pos, mixer, bf16, floats):
-    """Splits (0: keys and values are made), sets of columns in a block, and the merge's tokens and rows of a portion of n tokens at pos with latent attention."""
-    m, out = mixer, [ctypes.c_int() for _ in range(3)]
+    """Splits (0: keys and values are made), sets of columns in a block, and the merge's tokens of a portion of n tokens at pos with latent attention."""
+    m, out = mixer, [ctypes.c_int() for _ in range(2)]
     splits = lib().turn(n, pos, m["heads"], m["dim"], m["rot_dim"], m["vdim"], row_bytes(m["kv_rank"], bf16), (m["kv_rank"] + 15) // 16 * 16, bf16, floats, CUS,
                         *map(ctypes.byref, out))
     return (splits, *(x.value for x in out))
