@@ -106,13 +106,13 @@ def oracle(cfg, w, tokens, residuals=None, dtype=torch.float64):
     return O.forward(cfg, w, tokens, dtype, residuals)
 
 
-def far_key_model(heads, rank, length, at, rotated=False, seed=5):
+def far_key_model(heads, rank, length, at, rotated=False, seed=5, dims=(16, 8, 24), width=64):
     """One key that outweighs every other: position `at` holds token 0, which alone has feature 0; its plain key (or its
     rotated part, at angles that hardly move) points along a direction that every query has (feature 1, the same in all
     tokens), so whoever sees it, takes it."""
-    D, R, Dv = 16, 8, 24
-    cfg = model(64, 40, [sunk(heads, D, R, Dv, rank, scale=0.5, base=1e6, scaling=yarn(1e6, 1, 1e6, 1e5) if rotated else None)], positions=length, eps=1e-5)
-    w = weights(cfg, seed, peak=0.3, sink=0.3)
+    D, R, Dv = dims
+    cfg = model(width, 40, [sunk(heads, D, R, Dv, rank, scale=0.5, base=1e6, scaling=yarn(1e6, 1, 1e6, 1e5) if rotated else None)], positions=length, eps=1e-5)
+    w = weights(cfg, seed, peak=0.3 * (16 / D) ** 0.5, sink=0.3)
     g = torch.Generator().manual_seed(seed)
 
     def unit(n):
