@@ -347,13 +347,13 @@ def test_trace_program(checkpoint, tmp_path):
 
 # ---- other combinations of the library's mechanisms ----------------------------------------------------------------
 
-def grouped_layer_in_streams():
+def grouped_layer_in_streams(width=64, S=3, heads=4):
     """A Nibotar layer (chunked grouped attention; experts chosen by a table, and a shared one) inside three streams."""
     from clusterfusionplus_amd import nibotar
     from clusterfusionplus_amd.seq_model import Connections
-    cfg = NM.model(64, 51, [(NM.attn(4, 2, 24, 16, chunk=13), NM.moe(20, 6, 2, shared=44)), (NM.attn(2, 1, 16, 16), NM.dense(40))], softcap=None)
-    w, S = NM.weights(cfg, 7), 3
-    like = M.weights(M.model(64, 51, [M.gated(1, 8, 8, 8, 8, ff=8)] * 2, streams=S), 8)
+    cfg = NM.model(width, 51, [(NM.attn(heads, 2, 24, 16, chunk=13), NM.moe(20, 6, 2, shared=44)), (NM.attn(2, 1, 16, 16), NM.dense(40))], softcap=None)
+    w = NM.weights(cfg, 7)
+    like = M.weights(M.model(width, 51, [M.gated(1, 8, 8, 8, 8, ff=8)] * 2, streams=S), 8)
 
     def pack(dtype):
         p = nibotar.pack_weights(nibotar.parse_config(cfg), w, dtype, "cuda")
