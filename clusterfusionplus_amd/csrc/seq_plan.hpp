@@ -181,7 +181,14 @@ inline AttnPlan plan_attn(const AttnSizes& a, int cus, size_t room) {
 // 200, 1000, 3000 and 4000 (bf16: 128 differences, 6 us off on average; fp32: the uneven model alone).  In us per layer, made and read: 16 heads at 3000,
 // 2 tokens 108 / 91, 20 110 / 104, 40 113 / 112, 64 118 / 124; 128 heads at 3000, 2 tokens 411 / 282, 20 429 / 342, 64 480 / 469, 100 514 / 588; at 1000,
 // 20 333 / 319, 64 406 / 409; at 200, 10 300 / 302; 12 heads in fp32 at 3000, 2 tokens 111 / 85, 20 121 / 110, 64 139 / 164.  Not chosen within 4 us, which
-// is what the estimate misses small models by.  n tokens at pos and on; dim, rot, vdim: values of a head's key (plain, rotated) and value; bytes of a latent row, latents of it.
+// is what the estimate misses small models by.
+// Held against both ways over 11 models (12 to 128 heads of 64 to 192 dimensions, ranks of 64 to 512), 2 to 250 tokens at 150 to 64000, 1666 sizes in bf16 and
+// 1645 in fp32: layers take 25 and 35 % less on average where the latents are read (617 and 866 sizes); 8 and 6 of these are more than 0.6 % slower, 2.8 % at
+// most (fp32, 32 heads of rank 256, which takes the kernel for 512: 64 tokens at 6000 417 / 429).  Ranks of up to 128, whose kernel takes less than the estimate
+// says, are among them (353 sizes, 6 % faster and more); 382 sizes that would gain over 3 % are left to keys and values.  With more tokens the choice may come
+// back: the product that makes keys takes another row of tiles (64 heads at 2000: 48 tokens 173 / 178 us, 49 208 / 178; 32 heads at 1000: 24 159 / 165, 25
+// 164 / 164), or attention another block of columns.
+// n tokens at pos and on; dim, rot, vdim: values of a head's key (plain, rotated) and value; bytes of a latent row, latents of it.
 struct LatentSizes {
     int n, pos, heads, dim, rot, vdim, kbytes, rank;
     bool bf16;
@@ -192,7 +199,7 @@ struct LatentSizes {
 struct LatentTurn { int splits, sets, tokens; };
 constexpr int kTurnSplits = 64, kTurnRows = 64;
 inline LatentTurn plan_latent_turn(const LatentSizes& z, int cus) {
-    if (z.n > 256) return {};                            // (not measured, and never near the line)
+    if (z.n > 256) return {};                            // (not measured)
     const int keys = z.bf16 ? 32 : 16, cols = z.n * z.heads, ctx = z.pos + z.n, tiles = ceil_div(ctx, keys), esize = z.bf16 ? 2 : 4;
     const GemmSizes g{z.heads * (z.dim + z.vdim), ctx, z.kbytes, 0, 0};
     const GemmPlan made = plan_gemm(g, z.bf16, cus);
